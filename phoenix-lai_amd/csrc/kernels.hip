@@ -12,54 +12,36 @@ namespace phx {
 
 // ------------------------------------------------------------------------------ activation quantizers
 
-// The integers of Q8_K super-block b of row `row` (lane l holds elements 4l..4l+3 packed in pk) stored in
-// act's dot-product order (K4 / K6 / Q8K), with the sums of 16 (K4's s, and bh when set) and, with qh
-// set, the matrix cores' fp16 copies; the block's scale is the caller's.  qrow is the wave's 64-dword
-// LDS row through which the integers reach the packed orders.  Wave-level: all 64 lanes call it.
+// The integers of Q8_K super-block b of row `row` (lane l holds elements 4l..4l+3 packed in pk) stored as
+// act's rows, with the sums of 16 (bh when set) and, with qh set, the matrix cores' fp16 copies; the block's
+// scale is the caller's.  qrow is the wave's 64-dword LDS row through which the integers reach the fp16
+// copies' order.  Wave-level: all 64 lanes call it.
 __device__ __forceinline__ void store_q8k_block(const Act& act, int64_t row, int b, int lane, uint32_t pk,
                                                 uint32_t* qrow, float dval)
 {
-    int sm = (int)(int8_t)(pk & 0xFF) + (int)(int8_t)((pk >> 8) & 0xFF) + (int)(int8_t)((pk >> 16) & 0xFF) +
-             (int)(int8_t)(pk >> 24);
-    // block sums of 16: lanes 4j .. 4j + 3
-    sm += dpp_i<0xb1>(sm, sm);  // 4-lane sum: quad swaps
-    sm += dpp_i<0x4e>(sm, sm);
-    if ((lane & 3) == 0) {
-        if (act.fmt == ACT_K4 && act.s) act.s[row * act.sstride + b * 16 + (lane >> 2)] = sm;
-        if (act.bh) act.bh[row * act.bhstride + b * 16 + (lane >> 2)] = (uint16_t)f2h_bits((float)sm);  // exact
+    if (act.bh) {  // uniform; block sums of 16: lanes 4j .. 4j + 3
+        int sm = (int)(int8_t)(pk & 0xFF) + (int)(int8_t)((pk >> 8) & 0xFF) + (int)(int8_t)((pk >> 16) & 0xFF) +
+                 (int)(int8_t)(pk >> 24);
+        sm += dpp_i<0xb1>(sm, sm);  // 4-lane sum: quad swaps
+        sm += dpp_i<0x4e>(sm, sm);
+        if ((lane & 3) == 0)
+            act.bh[row * act.bhstride + b * 16 + (lane >> 2)] = (uint16_t)f2h_bits((float)sm);  // exact
     }
-    if (act.fmt == ACT_Q8K) {
-        if (act.q) ((uint32_t*)(act.q + row * act.qstride + (int64_t)b * 256))[lane] = pk;
-        if (!act.qh) return;  // uniform
-    }
+    if (act.q) ((uint32_t*)(act.q + row * act.qstride + (int64_t)b * 256))[lane] = pk;
+    if (!act.qh) return;  // uniform
     const uint8_t* qb = (const uint8_t*)qrow;
     qrow[lane] = pk;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     auto qv = [&](int e) { return (int)(int8_t)qb[e]; };
-    if (!act.q) {  // uniform: only the matrix cores' copy is wanted
-    } else if (act.fmt == ACT_K4) {  // dword (s, l) = x[32 s + l + 8 m], m = 0..3: lane = 8 s + l
-        const int s8 = lane >> 3, l = lane & 7, e = 32 * s8 + l;
-        ((uint32_t*)(act.q + row * act.qstride + (int64_t)b * 256))[lane] =
-            (uint32_t)qb[e] | ((uint32_t)qb[e + 8] << 8) | ((uint32_t)qb[e + 16] << 16) | ((uint32_t)qb[e + 24] << 24);
-    } else if (act.fmt == ACT_K6) {  // (P, l): lane = 8 P + l
-        const int P = lane >> 3, l = lane & 7, e = 32 * P + l;
-        uint32_t* dst = (uint32_t*)(act.q + row * act.qstride + (int64_t)b * 512);
-        int* c = act.s + row * act.sstride + b * 128;
-        dst[lane * 2 + 0] = (uint32_t)qb[e] | ((uint32_t)qb[e + 8] << 8);
-        dst[lane * 2 + 1] = ((uint32_t)qb[e + 16] << 16) | ((uint32_t)qb[e + 24] << 24);
-        c[(2 * P) * 8 + l] = -32 * (qv(e) + qv(e + 8));
-        c[(2 * P + 1) * 8 + l] = -32 * (qv(e + 16) + qv(e + 24));
-    }
-    if (act.qh) {  // the matrix cores' copy: exact fp16 integers (or, folded, fp16 of q * dval), halves
-                   // [l][s][mm']: lane = 8 l + s
-        const int l = lane >> 3, s8 = lane & 7, e = 32 * s8 + l;
-        uint32_t* hq = (uint32_t*)(act.qh + row * act.qhstride + (int64_t)b * 256) + l * 16 + s8 * 2;
-        const float f = act.fold ? dval : 1.0f;
-        hq[0] = f2h_bits((float)qv(e) * f) | (f2h_bits((float)qv(e + 16) * f) << 16);
-        hq[1] = f2h_bits((float)qv(e + 8) * f) | (f2h_bits((float)qv(e + 24) * f) << 16);
-    }
+    // the matrix cores' copy: exact fp16 integers (or, folded, fp16 of q * dval), halves [l][s][mm']:
+    // lane = 8 l + s
+    const int l = lane >> 3, s8 = lane & 7, e = 32 * s8 + l;
+    uint32_t* hq = (uint32_t*)(act.qh + row * act.qhstride + (int64_t)b * 256) + l * 16 + s8 * 2;
+    const float f = act.fold ? dval : 1.0f;
+    hq[0] = f2h_bits((float)qv(e) * f) | (f2h_bits((float)qv(e + 16) * f) << 16);
+    hq[1] = f2h_bits((float)qv(e + 8) * f) | (f2h_bits((float)qv(e + 24) * f) << 16);
     // the row is rewritten by the wave's next block only after every lane's reads above
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -68,8 +50,8 @@ __device__ __forceinline__ void store_q8k_block(const Act& act, int64_t row, int
 
 // Quantize one row (in LDS, `cols` floats) into format act, row index `row`.  Block-level (NT threads).
 //  Q8_0: CpuRef.QuantizeQ8_0 (src/CpuRef.cs:49-62), plus the block sum of q for the Q4_0 offset.
-//  K4/K6/Q8K: CpuRef.QuantizeQ8_K (src/CpuRefKQuants.cs:53-86), stored in the dot-product orders (and,
-//  with qh / bh set, the matrix cores' fp16 copies).
+//  Q8K: CpuRef.QuantizeQ8_K (src/CpuRefKQuants.cs:53-86) (and, with qh / bh set, the matrix cores' fp16
+//  copies).
 template <int NT>
 __device__ void quantize_row(const float* v, Act act, int64_t row)
 {
@@ -886,6 +868,9 @@ struct GroupArgs {
     float* out1;
     int split, out_stride;
     bool paired;
+    int nident = 0;    // > 0 (tiles null): one matrix, tile i the rows 4 i .. 4 i + 3 of nident, in order
+    int amax = 4;      // k_grouped_k: assignments a tile can hold in this call (its LDS), and the most tiles
+    int mt = 1;        // (workgroup b: tile b % mt, row group b / mt)
     const void* grid;  // IQ types: the expanded codebook (64-bit words for IQ2_XXS / IQ2_S, 32-bit for IQ3_S)
     Act req;                       // req.q set: the paired gate|up kernel also writes gelu(g) * u as Q8_0 rows
     const float* gelu_tab = nullptr;
@@ -1152,62 +1137,120 @@ __global__ __launch_bounds__(256) void k_grouped_q_ring(GroupArgs g)
         }
 }
 
-// K-quant rows: DotK (src/CpuRefKQuants.cs:177-212) per (row, assignment): per super-block the eight
-// integer lanes aux32[l] (element e contributes to lane e % 8), float lanes
+// K-quant rows of a few assignments: DotK (src/CpuRefKQuants.cs:177-212) per (row, assignment): per
+// super-block the eight integer lanes aux32[l] (element e contributes to lane e % 8), float lanes
 // sums[l] += (d * yd) * aux32[l], the Q4_K / Q5_K min term sumf -= (dmin * yd) * sumi, finally sumf += sums[l].
-template <int TYPE, int A>
-__global__ __launch_bounds__(256) void k_grouped_k(GroupArgs g)
+// A workgroup takes one row group (lane = row) of one tile of up to four assignments and a wave one
+// super-block at a time (a 1 KB run per 16-byte chunk), while the assignments' Q8_K integers are turned into
+// the weights' byte-lane order in LDS (dword (s, l): elements 32 s + l + 8 m, m = 0..3).  The float terms meet
+// in LDS, and the eight lanes' chains (and the min term's) run in super-block order, a wave per lane l.
+// Scales times dot products are 24-bit products (v_mad_i32_i24; a 32-bit multiply issues at a quarter of the
+// rate).
+constexpr int GK_W = 16;  // most waves, and super-blocks staged at a time
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int TYPE>
+__host__ __device__ constexpr int gk_terms() { return TYPE == PHX_Q6_K_DEV ? 8 : 9; }  // eight lanes and the min term
+// LDS: term buffers (two where a tile can hold more than one assignment), the chains' values, then per
+// assignment and super-block the integers (64 dwords), the sums of 32 (8) and the scale
+template <int TYPE>
+__host__ __device__ constexpr int gk_lds(int nw, int amax, int sg)
 {
-    const int tile = blockIdx.x;
-    if (tile >= *g.ntiles) return;
-    const Tile tl = g.tiles[tile];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int rgi = blockIdx.y * 4 + wave;
-    if (rgi >= g.rg) return;
+    return (amax > 1 ? 2 : 1) * nw * gk_terms<TYPE>() * 256 + amax * gk_terms<TYPE>() * 256 + amax * sg * (256 + 32 + 4);
+}
+template <int TYPE>
+__global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
+{
     constexpr bool Q4K = TYPE == PHX_Q4_K_DEV, Q5K = TYPE == PHX_Q5_K_DEV;
     constexpr bool AFF = Q4K || Q5K;  // scales and mins per 32 (the min term); else 16 signed scales per 16
-    constexpr int PAY = Q4K ? 144 : Q5K ? 176 : 208;
-    const uint8_t* wp = g.payload + tl.e * g.mat_pay + rgi * g.rg_pay + lane * PAY;
-    const uint8_t* wsb = g.scale + tl.e * g.mat_sc + ((int64_t)rgi * g.nb * 64 + lane) * (AFF ? 4 : 2);
-    int arow[A];
-    float sums[A][8], sumf[A];
-#pragma unroll
-    for (int i = 0; i < A; i++) {
-        arow[i] = i < tl.cnt ? g.perm[tl.start + i] / g.act_div : 0;
-        sumf[i] = 0.0f;
-#pragma unroll
-        for (int l = 0; l < 8; l++) sums[i][l] = 0.0f;
+    constexpr int PAY = Q4K ? 144 : Q5K ? 176 : 208, NT = gk_terms<TYPE>();
+    const int tile = blockIdx.x % g.mt;
+    Tile tl;
+    if (g.nident) {
+        tl = Tile{0, 4 * tile, min(4, g.nident - 4 * tile)};
+    } else {
+        if (tile >= *g.ntiles) return;  // uniform
+        tl = g.tiles[tile];
     }
-    for (int b = 0; b < g.nb; b++) {
-        uint32_t wv[PAY / 4];
-        {
-            const uint4* src = (const uint4*)(wp + (int64_t)b * 64 * PAY);
+    const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, nw = nt >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rgi = blockIdx.x / g.mt, nb = g.nb, cnt = min(tl.cnt, g.amax);
+    const int sg = min(nb, GK_W / nw * nw);  // super-blocks staged at a time: whole rounds of the waves
+    extern __shared__ __align__(16) unsigned char gk_smem[];
+    float* term = (float*)gk_smem;                                // [buffer][wave][NT][64]
+    float* chain = term + (g.amax > 1 ? 2 : 1) * nw * NT * 64;    // [assignment][NT][64]
+    uint32_t* xs = (uint32_t*)(chain + g.amax * NT * 64);         // [assignment][super-block][64]
+    int* xb = (int*)(xs + g.amax * sg * 64);                      // [assignment][super-block][8]
+    float* xd = (float*)(xb + g.amax * sg * 8);                   // [assignment][super-block]
+    const uint8_t* wp = g.payload + tl.e * g.mat_pay + rgi * g.rg_pay + lane * 16;
+    constexpr int SBY = AFF ? 4 : 2, BLK = 64 * (PAY + SBY);  // the rows' scales follow the block's chunks
+    auto arow = [&](int i) -> int64_t {
+        return g.nident ? tl.start + i : g.perm[tl.start + i] / g.act_div;
+    };
+    uint32_t wv[PAY / 4], dmw;
+    auto load = [&](int r0) {  // this wave's super-block of the round (past the end: the last one again)
+        const int b = min(r0 + wave, nb - 1);
+        const uint4* src = (const uint4*)(wp + (int64_t)b * BLK);
 #pragma unroll
-            for (int c = 0; c < PAY / 16; c++) {
-                uint4 t4 = src[c];
-                wv[4 * c] = t4.x; wv[4 * c + 1] = t4.y; wv[4 * c + 2] = t4.z; wv[4 * c + 3] = t4.w;
+        for (int c = 0; c < PAY / 16; c++) {
+            const uint4 t4 = src[c * 64];
+            wv[4 * c] = t4.x; wv[4 * c + 1] = t4.y; wv[4 * c + 2] = t4.z; wv[4 * c + 3] = t4.w;
+        }
+        const uint8_t* sp = wp + (int64_t)b * BLK + 64 * PAY - lane * (16 - SBY);
+        dmw = AFF ? *(const uint32_t*)sp : *(const uint16_t*)sp;
+    };
+    // integers of super-blocks s0 .. s0 + n - 1: a thread per 32-element sub-block and round loads eight dwords
+    // (elements 4 j .. 4 j + 3)
+    auto stage = [&](int s0, int n) {
+        for (int x = tid; x < cnt * n * 8; x += nt) {
+            const int xi = x / (n * 8), xr = x - xi * n * 8;
+            const u32x4_a4* src = (const u32x4_a4*)(g.act.q + arow(xi) * g.act.qstride + (int64_t)s0 * 256 + xr * 32);
+            const u32x4_a4 n0 = src[0], n1 = src[1];
+            if ((xr & 7) == 0) xd[xi * sg + (xr >> 3)] = g.act.d[arow(xi) * g.act.dstride + s0 + (xr >> 3)];
+            // 4 x 4 byte transposes: bytes l of dwords j, j + 2, j + 4, j + 6 (l = 4 j .. 4 j + 3)
+            uint32_t* dst = xs + (xi * sg + (xr >> 3)) * 64 + (xr & 7) * 8;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const uint32_t a0 = n0[j], a1 = n0[j + 2], a2 = n1[j], a3 = n1[j + 2];
+                const uint32_t p0 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), p1 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
+                const uint32_t p2 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), p3 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
+                *(uint4*)(dst + 4 * j) = make_uint4(__builtin_amdgcn_perm(p2, p0, 0x05040100u),
+                                                    __builtin_amdgcn_perm(p2, p0, 0x07060302u),
+                                                    __builtin_amdgcn_perm(p3, p1, 0x05040100u),
+                                                    __builtin_amdgcn_perm(p3, p1, 0x07060302u));
+            }
+            if (AFF) {
+                int sm = 0;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    sm = __builtin_amdgcn_sdot4((int)n0[j], 0x01010101, sm, false);
+                    sm = __builtin_amdgcn_sdot4((int)n1[j], 0x01010101, sm, false);
+                }
+                xb[(xi * sg + (xr >> 3)) * 8 + (xr & 7)] = sm;
             }
         }
-        float d, dmin = 0.0f;
-        if (AFF) {
-            uint32_t dm = *(const uint32_t*)(wsb + (int64_t)b * 64 * 4);
-            d = h2f(dm & 0xFFFF);
-            dmin = h2f(dm >> 16);
-        } else {
-            d = h2f(*(const uint16_t*)(wsb + (int64_t)b * 64 * 2));
+    };
+    int buf = 0;
+    for (int r0 = 0; r0 < nb; r0 += nw) {
+        const int nbr = min(nw, nb - r0);
+        load(r0);
+        if (r0 % sg == 0) {  // uniform; every read of the staged rows and terms before it is over
+            stage(r0, min(sg, nb - r0));
+            __syncthreads();
         }
-        // unpacked weight dwords
+        const int sl = r0 % sg + min(wave, nbr - 1);  // this wave's staged super-block
+        const float d = h2f(dmw & 0xFFFF), dmin = AFF ? h2f(dmw >> 16) : 0.0f;
+        // the row's values as byte dwords (Q6_K: value - 32, signed) and its scales
         uint32_t v[64];
         int sc[16], mn[8];
-        if (AFF) {
 #pragma unroll
-            for (int w = 0; w < 32; w++) {
-                v[2 * w] = wv[w] & 0x0F0F0F0Fu;
-                v[2 * w + 1] = (wv[w] >> 4) & 0x0F0F0F0Fu;
-            }
+        for (int w = 0; w < 32; w++) {
+            v[2 * w] = wv[w] & 0x0F0F0F0Fu;
+            v[2 * w + 1] = (wv[w] >> 4) & 0x0F0F0F0Fu;
+        }
+        if (AFF) {
             if (Q5K)  // the fifth bits: bit l of byte mm of dword s belongs to value dword 8 s + l, byte mm
 #pragma unroll
-                for (int x = 0; x < 64; x++) v[x] |= ((wv[36 + x / 8] >> (x % 8)) & 0x01010101u) << 4;
+                for (int x = 0; x < 64; x++) v[x] |= ((wv[PAY / 4 - 8 + x / 8] >> (x % 8)) & 0x01010101u) << 4;
 #pragma unroll
             for (int s = 0; s < 8; s++) {
                 sc[s] = (wv[32 + s / 4] >> (8 * (s % 4))) & 0xFF;
@@ -1215,69 +1258,87 @@ __global__ __launch_bounds__(256) void k_grouped_k(GroupArgs g)
             }
         } else {
 #pragma unroll
-            for (int w = 0; w < 32; w++) {
-                uint32_t lo0 = wv[w] & 0x0F0F0F0Fu, lo1 = (wv[w] >> 4) & 0x0F0F0F0Fu;
-                int k0 = 2 * w, k1 = 2 * w + 1;
-                uint32_t h0 = (wv[32 + k0 / 4] >> (2 * (k0 % 4))) & 0x03030303u;
-                uint32_t h1 = (wv[32 + k1 / 4] >> (2 * (k1 % 4))) & 0x03030303u;
-                v[k0] = lo0 | (h0 << 4);
-                v[k1] = lo1 | (h1 << 4);
+            for (int x = 0; x < 64; x++) {  // minus 32 per byte: 0x60 .. 0x9F after the add, no carry between bytes
+                v[x] |= ((wv[32 + x / 4] >> (2 * (x % 4))) & 0x03030303u) << 4;
+                v[x] = (v[x] + 0x60606060u) ^ 0x80808080u;
             }
 #pragma unroll
-            for (int s = 0; s < 16; s++) sc[s] = (int)(int8_t)((wv[48 + s / 4] >> (8 * (s % 4))) & 0xFF);
+            for (int s = 0; s < 16; s++) sc[s] = (int)(int8_t)((wv[PAY / 4 - 4 + s / 4] >> (8 * (s % 4))) & 0xFF);
         }
+        for (int i = 0; i < cnt; i++) {  // uniform
+            const uint4* x4 = (const uint4*)(xs + (i * sg + sl) * 64);
+            int aux[8];
 #pragma unroll
-        for (int i = 0; i < A; i++) {
-            if (i < tl.cnt) {
-                const int64_t r = arow[i];
-                int aux[8];
+            for (int l = 0; l < 8; l++) aux[l] = 0;
 #pragma unroll
-                for (int l = 0; l < 8; l++) aux[l] = 0;
-                if (AFF) {
-                    const uint32_t* xq = (const uint32_t*)(g.act.q + r * g.act.qstride + b * 256);
+            for (int s = 0; s < 8; s++) {
+                const uint4 xa = x4[2 * s], xc = x4[2 * s + 1];
+                const uint32_t x[8] = {xa.x, xa.y, xa.z, xa.w, xc.x, xc.y, xc.z, xc.w};
 #pragma unroll
-                    for (int s = 0; s < 8; s++)
-#pragma unroll
-                        for (int l = 0; l < 8; l++)
-                            aux[l] += sc[s] * __builtin_amdgcn_sdot4((int)v[s * 8 + l], (int)xq[s * 8 + l], 0, false);
-                } else {
-                    const uint32_t* xq = (const uint32_t*)(g.act.q + r * g.act.qstride + (int64_t)b * 512);
-                    const int* cterm = g.act.s + r * g.act.sstride + b * 128;
-#pragma unroll
-                    for (int P = 0; P < 8; P++)
-#pragma unroll
-                        for (int l = 0; l < 8; l++) {
-                            int pa = __builtin_amdgcn_sdot4((int)v[P * 8 + l], (int)xq[(P * 8 + l) * 2], cterm[(2 * P) * 8 + l], false);
-                            int pb = __builtin_amdgcn_sdot4((int)v[P * 8 + l], (int)xq[(P * 8 + l) * 2 + 1],
-                                                            cterm[(2 * P + 1) * 8 + l], false);
-                            aux[l] += sc[2 * P] * pa;
-                            aux[l] += sc[2 * P + 1] * pb;
-                        }
-                }
-                const float yd = g.act.d[r * g.act.dstride + b];
-                const float dd = d * yd;
-#pragma unroll
-                for (int l = 0; l < 8; l++) sums[i][l] += dd * (float)aux[l];
-                if (AFF) {
-                    const int* bs = g.act.s + r * g.act.sstride + b * 16;
-                    int sumi = 0;
-#pragma unroll
-                    for (int j = 0; j < 16; j++) sumi += bs[j] * mn[j / 2];
-                    const float dm = dmin * yd;
-                    sumf[i] -= dm * (float)sumi;
+                for (int l = 0; l < 8; l++) {
+                    const int p = __builtin_amdgcn_sdot4((int)v[8 * s + l], (int)x[l], 0, false);
+                    if (AFF) {
+                        aux[l] += __mul24(sc[s], p);
+                    } else {  // elements l, l + 8 carry scale 2 s, l + 16, l + 24 scale 2 s + 1
+                        const int pa = __builtin_amdgcn_sdot4((int)v[8 * s + l], (int)(x[l] & 0xFFFFu), 0, false);
+                        aux[l] += __mul24(sc[2 * s], pa);
+                        aux[l] += __mul24(sc[2 * s + 1], p - pa);
+                    }
                 }
             }
+            const float yd = xd[i * sg + sl], dd = d * yd;
+            float* t = term + (buf * nw + wave) * NT * 64 + lane;
+#pragma unroll
+            for (int l = 0; l < 8; l++) t[l * 64] = dd * (float)aux[l];
+            if (AFF) {
+                const int* bs = xb + (i * sg + sl) * 8;
+                int sumi = 0;
+#pragma unroll
+                for (int s = 0; s < 8; s++) sumi += __mul24(bs[s], mn[s]);
+                const float dm = dmin * yd;
+                t[8 * 64] = dm * (float)sumi;
+            }
+            __syncthreads();  // the terms are there; the other buffer's chains are done
+            for (int c = wave; c < NT; c += nw) {
+                float s = r0 ? chain[(i * NT + c) * 64 + lane] : 0.0f;
+                const float* tc = term + (buf * nw * NT + c) * 64 + lane;
+                if (c < 8)
+                    for (int j = 0; j < nbr; j++) s += tc[j * NT * 64];
+                else
+                    for (int j = 0; j < nbr; j++) s -= tc[j * NT * 64];
+                chain[(i * NT + c) * 64 + lane] = s;
+            }
+            if (g.amax > 1) buf ^= 1;
+            else if (r0 + nw < nb) __syncthreads();  // one buffer: the next round's terms wait for these chains
         }
     }
+    __syncthreads();
+    for (int i = wave; i < cnt; i += nw) {
+        const float* f = chain + i * NT * 64 + lane;
+        float s = AFF ? f[8 * 64] : 0.0f;
 #pragma unroll
-    for (int i = 0; i < A; i++) {
-        if (i < tl.cnt) {
-            float s = sumf[i];
-#pragma unroll
-            for (int l = 0; l < 8; l++) s += sums[i][l];
-            store_row(g, rgi, lane, g.perm[tl.start + i], s);
-        }
+        for (int l = 0; l < 8; l++) s += f[l * 64];
+        store_row(g, rgi, lane, g.nident ? tl.start + i : g.perm[tl.start + i], s);
     }
+}
+
+// A launch whose workgroups all find a compute unit of their own takes a wave per super-block (everything in
+// flight at once: a 4096-column Q4_K row group of four experts, 176 workgroups, 10.4 us against 37 for one
+// wave walking all 16 super-blocks; the Q6_K down 9.6 against 28).  A larger one takes rounds of about four
+// waves, several workgroups to a compute unit: their loads and chains run under each other's products, which
+// then bound it (about 700 VALU instructions per super-block and wave; 16 waves each 10-20% slower from 32
+// tokens on).
+template <int TYPE>
+static void launch_grouped_k(hipStream_t st, GroupArgs g, int max_tiles, int ncu)
+{
+    g.mt = max_tiles;
+    const bool wide = (int64_t)max_tiles * g.rg <= ncu;
+    const int rounds = wide ? (g.nb + GK_W - 1) / GK_W : (g.nb + 3) / 4, nw = (g.nb + rounds - 1) / rounds;
+    const int lds = gk_lds<TYPE>(nw, g.amax, std::min(g.nb, GK_W / nw * nw));
+    static_assert(gk_lds<TYPE>(GK_W, 4, GK_W) <= 160 * 1024, "the widest launch fits a compute unit's LDS");
+    (void)hipFuncSetAttribute((const void*)k_grouped_k<TYPE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              gk_lds<TYPE>(GK_W, 4, GK_W));
+    launch(k_grouped_k<TYPE>, dim3((unsigned)max_tiles * (unsigned)g.rg), dim3(64 * nw), (uint32_t)lds, st, g);
 }
 
 // Signs applied to four codebook bytes: bit j of nib set negates byte j.  The bit spread gives 0x01 in
@@ -1407,7 +1468,7 @@ static uint32_t grouped_q_lds(int type, int nb)
 
 void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles, int A,
                     const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
-                    const Act* req, const float* gelu_tab, int req_rows)
+                    const Act* req, const float* gelu_tab, int req_rows, int nident, int amax)
 {
     GroupArgs g;
     g.payload = w.payload;
@@ -1429,6 +1490,8 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
     g.out_stride = out_stride;
     g.paired = w.paired;
     g.grid = w.grid;
+    g.nident = nident;
+    g.amax = std::min(amax, 4);
     // the down input in the ring kernel's epilogue where it covers every block of the row (paired Q4_0 /
     // Q8_0 rows past QG_SHORT blocks into Q8_0 rows with no padding blocks); else k_requant after it
     const bool fuse = req && w.paired && w.nb > QG_SHORT && (w.type == PHX_Q4_0_DEV || w.type == PHX_Q8_0_DEV) &&
@@ -1448,9 +1511,9 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
         if (w.nb > QG_SHORT) launch((k_grouped_q_ring<PHX_Q8_0_DEV, 4>), grid, dim3(256), grouped_q_lds(w.type, w.nb), st, g);
         else launch((k_grouped_q<PHX_Q8_0_DEV, 4>), grid, dim3(256), 0, st, g);
         break;
-    case PHX_Q4_K_DEV: launch((k_grouped_k<PHX_Q4_K_DEV, 4>), grid, dim3(256), 0, st, g); break;
-    case PHX_Q5_K_DEV: launch((k_grouped_k<PHX_Q5_K_DEV, 4>), grid, dim3(256), 0, st, g); break;
-    case PHX_Q6_K_DEV: launch((k_grouped_k<PHX_Q6_K_DEV, 4>), grid, dim3(256), 0, st, g); break;
+    case PHX_Q4_K_DEV: launch_grouped_k<PHX_Q4_K_DEV>(st, g, max_tiles, 256); break;
+    case PHX_Q5_K_DEV: launch_grouped_k<PHX_Q5_K_DEV>(st, g, max_tiles, 256); break;
+    case PHX_Q6_K_DEV: launch_grouped_k<PHX_Q6_K_DEV>(st, g, max_tiles, 256); break;
     case PHX_IQ2_XXS_DEV: launch((k_grouped_iq<PHX_IQ2_XXS_DEV, 4>), grid, dim3(256), 0, st, g); break;
     case PHX_IQ2_S_DEV: launch((k_grouped_iq<PHX_IQ2_S_DEV, 4>), grid, dim3(256), 0, st, g); break;
     case PHX_IQ3_S_DEV: launch((k_grouped_iq<PHX_IQ3_S_DEV, 4>), grid, dim3(256), 0, st, g); break;
@@ -1915,8 +1978,8 @@ void launch_planar_act(hipStream_t st, int rows, int n, const int8_t* qs, const 
 }
 
 // Planar Q8_K rows (qs int8 [rows][n] in element order and the float scale [rows][n/256], the layout
-// phx_quant_q8_k writes) into the K-quant kernels' activation arrays (ACT_K4 / ACT_K6 orders, the sums
-// of 16, and with a.qh / a.bh set the matrix cores' fp16 copies).  One wave per 256-block.
+// phx_quant_q8_k writes) into the K-quant kernels' activation arrays (the scales, and with a.qh / a.bh set
+// the matrix cores' fp16 copies and sums of 16).  One wave per 256-block.
 __global__ __launch_bounds__(256) void k_planar_act_k(int64_t nblk, int nb, const int8_t* __restrict__ qs,
                                                       const float* __restrict__ d, Act a)
 {

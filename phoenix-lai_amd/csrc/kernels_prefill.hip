@@ -914,7 +914,7 @@ struct KmRing {
     static constexpr int ACT_N = 32 * KM_TOK * 16;          // [32 chunks][48 assignments][16 B]
     static constexpr int BSM_N = Q4K ? 4 * KM_TOK * 8 : 0;  // Q4_K: [4 quarters][48][4 fp16 bsums]
     static constexpr int YD_N = KM_TOK * 4;                 // [48] token scales
-    static constexpr int W_N = KM_NW * 16 * PAY;            // [8 waves][16 rows][PAY]
+    static constexpr int W_N = KM_NW * 16 * PAY;            // [8 waves][PAY / 16 chunks][16 rows][16 B]
     static constexpr int WS_N = KM_NW * 16 * 4;             // [8 waves][16 rows] 4-byte slots
     static constexpr int ACT = 0, BSM = ACT + KM_RING * ACT_N, YD = BSM + KM_RING * BSM_N;
     static constexpr int W = YD + KM_RING * YD_N, WS = W + KM_RING * W_N, BYTES = WS + KM_RING * WS_N;
@@ -975,39 +975,39 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
     }
     // (5) token scales of assignments 6 w + lane (lanes 0-5)
     const uint32_t vy = (uint32_t)(4 * arow(6 * wave + min(lane, 5)) * g.act.dstride);
-    // (6)-(8) the wave's 16 weight rows, 1 KB per load; (9) their scales (lanes 0-15)
+    // (6)-(8) the wave's 16 weight rows, four 16-byte chunks of the 16 per load (lane quarter q the load's
+    // chunk q); (9) their scales (lanes 0-15)
     const int gIc = min(gI, g.rg - 1);
     const __amdgpu_buffer_rsrc_t r_act = buf_rsrc(g.act.qh), r_yd = buf_rsrc(g.act.d);
     const __amdgpu_buffer_rsrc_t r_bh = buf_rsrc(Q4K ? (const void*)g.act.bh : (const void*)g.act.d);
     const __amdgpu_buffer_rsrc_t r_w = buf_rsrc(g.payload + tl.e * g.mat_pay + gIc * g.rg_pay);
-    const __amdgpu_buffer_rsrc_t r_s = buf_rsrc(g.scale + tl.e * g.mat_sc + (int64_t)gIc * nb * 64 * SBY);
-    const uint32_t vw = 16 * ws * PAY + 16 * lane, vs = (16 * ws + r16) * SBY;
+    const uint32_t vw = 1024 * q + 16 * (16 * ws + r16), vs = (16 * ws + r16) * SBY;
 
 #define KM_LOAD(rsrc, lds_off, size, voff, soff) \
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t)(ring + (lds_off)), size, voff, soff, 0, 0)
     auto issue = [&](auto SC, int b) {  // super-block b (clamped: past the end a harmless reload) into slot S
         constexpr int S = decltype(SC)::value;
         const uint32_t bc = (uint32_t)min(b, nb - 1);
-        const uint32_t sw = bc * 64 * PAY;
+        const uint32_t sw = bc * (64 * (PAY + SBY));  // the rows' scales follow the block's chunks
         const int wl = RG::W + S * RG::W_N + wave * 16 * PAY;
 #pragma unroll
         for (int i = 0; i < 3; i++) KM_LOAD(r_act, RG::ACT + S * RG::ACT_N + (3 * wave + i) * 1024, 16, vx[i], bc * 512);
         if (Q4K) {
             if (lane < 48) KM_LOAD(r_bh, RG::BSM + S * RG::BSM_N + 192 * wave, 4, vb, bc * 32);
         } else {
-            if (lane < 16) KM_LOAD(r_w, wl + 3072, 16, vw, sw + 3072);  // Q6_K rows: 3328 bytes
+            if (lane < 16) KM_LOAD(r_w, wl + 3072, 16, vw, sw + 12288);  // Q6_K: 13 chunks
         }
         if (lane < 6) KM_LOAD(r_yd, RG::YD + S * RG::YD_N + 24 * wave, 4, vy, bc * 4);
         KM_LOAD(r_w, wl, 16, vw, sw);
-        KM_LOAD(r_w, wl + 1024, 16, vw, sw + 1024);
+        KM_LOAD(r_w, wl + 1024, 16, vw, sw + 4096);
         if (Q4K) {
-            if (lane < 16) KM_LOAD(r_w, wl + 2048, 16, vw, sw + 2048);  // Q4_K rows: 2304 bytes
+            if (lane < 16) KM_LOAD(r_w, wl + 2048, 16, vw, sw + 8192);  // Q4_K: 9 chunks
         } else {
-            KM_LOAD(r_w, wl + 2048, 16, vw, sw + 2048);
+            KM_LOAD(r_w, wl + 2048, 16, vw, sw + 8192);
         }
         if (lane < 16) {
-            if (Q4K) KM_LOAD(r_s, RG::WS + S * RG::WS_N + 64 * wave, 4, vs, bc * 64 * SBY);
-            else KM_LOAD(r_s, RG::WS + S * RG::WS_N + 64 * wave, 2, vs, bc * 64 * SBY);
+            if (Q4K) KM_LOAD(r_w, RG::WS + S * RG::WS_N + 64 * wave, 4, vs, sw + 64 * PAY);
+            else KM_LOAD(r_w, RG::WS + S * RG::WS_N + 64 * wave, 2, vs, sw + 64 * PAY);
         }
     };
 #undef KM_LOAD
@@ -1038,12 +1038,15 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
     const uint32_t a_act = ring0 + RG::ACT + q * (KM_TOK * 16) + r16 * 16, a_act2 = a_act + 2 * RG::ACT_N;
     const uint32_t a_bs = ring0 + RG::BSM + q * (KM_TOK * 8) + r16 * 8;
     const uint32_t a_yd = ring0 + RG::YD + r16 * 4;
-    const uint32_t a_row = ring0 + RG::W + (wave * 16 + r16) * PAY + 32 * q;
-    const uint32_t a_sc = ring0 + RG::W + (wave * 16 + r16) * PAY + (Q4K ? 128 + 4 * (q >> 1) : 128 + 16 * q);
-    const uint32_t a_y = Q4K ? a_sc + 8 : ring0 + RG::W + (wave * 16 + r16) * PAY + 192 + 4 * q;
+    // the wave's weight rows sit chunk-major ([chunk][16 rows][16 B]): the 16 lanes of a read take 256
+    // consecutive bytes
+    const uint32_t a_w0 = ring0 + RG::W + wave * 16 * PAY + r16 * 16;
+    const uint32_t a_row = a_w0 + 2 * q * 256;
+    const uint32_t a_sc = a_w0 + (Q4K ? 8 * 256 + 4 * (q >> 1) : (8 + q) * 256);
+    const uint32_t a_y = Q4K ? a_sc + 8 : a_w0 + 12 * 256 + 4 * q;
     const uint32_t a_ws = ring0 + RG::WS + (wave * 16 + 4 * q) * 4;
     const uint32_t a_wr = ring0 + RG::WS + (wave * 16 + r16) * 4;  // FOLD: d (and dmin) of the A operand's row
-    static_assert((RING - 1) * RG::W_N + 192 + 16 * 3 + 16 < 65536, "weight slots within the LDS immediate");
+    static_assert((RING - 1) * RG::W_N + 256 + 16 < 65536, "weight slots within the LDS immediate");
     static_assert(RG::ACT_N + 8 * KM_TOK * 64 < 65536, "two activation slots within the LDS immediate");
     // activation chunk reads of slot S at inner offset O
     auto act_rd = [&](auto SC, auto OC) -> u32x4 {
@@ -1059,7 +1062,7 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
         // the super-block's weights, row scales, token scales, block sums and the first operands (a read's
         // result is used only after its wait, never first composed into another value)
         constexpr int OW = S * RG::W_N;
-        u32x4 D0 = ds_r128<OW>(a_row), D1 = ds_r128<OW + 16>(a_row);
+        u32x4 D0 = ds_r128<OW>(a_row), D1 = ds_r128<OW + 256>(a_row);
         // Q4_K: X0 the dword of sc[2 q], sc[2 q + 1], Y that of mins[2 q], mins[2 q + 1];
         // Q6_K: X the high-bit dwords (s = 2 q: lq 0, 1; s = 2 q + 1: lq 0, 1), Y sc[4 q .. 4 q + 3]
         u32x4 X;

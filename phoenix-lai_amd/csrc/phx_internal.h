@@ -74,7 +74,7 @@ inline void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, uint32_t lds
 constexpr int kRowGroup = 64;  // rows per interleaved row group: one wave64, lane = row
 
 // Activation formats produced for each weight type.
-enum ActFmt { ACT_Q8_0 = 0, ACT_K4 = 1, ACT_K6 = 2, ACT_Q8K = 3 };
+enum ActFmt { ACT_Q8_0 = 0, ACT_Q8K = 1 };
 
 // One stack of quantized matrices (experts, or one dense matrix), repacked at upload into row
 // groups of 64 rows: payload[m][rg][b][lane][pay] and scale[m][rg][b][lane][sbytes], so the 64
@@ -84,6 +84,10 @@ enum ActFmt { ACT_Q8_0 = 0, ACT_K4 = 1, ACT_K6 = 2, ACT_Q8K = 3 };
 // consecutive blocks: the decode kernels' layout), so a row group's weights and scales share pages.
 //   Q4_0: pay 16 (nibbles, low = element j, high = j+16), scale fp16 d
 //   Q8_0: pay 32 (int8), scale fp16 d
+// The K-quant blocks are stored chunk-major, payload[m][rg][b][pay / 16][lane][16]: chunk c (bytes 16 c ..
+// 16 c + 15) of the 64 rows is one contiguous 1 KB (a wave's 16-byte loads of one chunk touch 8 lines of
+// 128 B; with each row's 144-208 bytes together they touched 64), and the block's 64 row scales [lane][sbytes]
+// follow its chunks (blk_bytes per block, no scale array).
 //   Q4_K: pay 144 = 128 nibbles in (sub-block, l, m) order + sc[8] + m[8]; scale fp16 d | fp16 dmin << 16
 //   Q6_K: pay 208 = 128 low-nibble plane + 64 high-bit plane + int8 sc[16]; scale fp16 d
 //   IQ2_XXS / IQ2_S / IQ3_S: pay 64 / 80 / 112 = the block's bytes after d, unchanged (IQ3_S padded by 4);
@@ -98,6 +102,9 @@ struct QMat {
     uint8_t* payload = nullptr;
     uint8_t* scale = nullptr;
     const void* grid = nullptr;         // IQ types: the context's expanded codebook of this type
+    // K-quants: a block's row scales follow its payload in the row group's span
+    bool sc_inside() const { return type == PHX_Q4_K_DEV || type == PHX_Q5_K_DEV || type == PHX_Q6_K_DEV; }
+    int64_t blk_bytes() const { return (int64_t)kRowGroup * (pay + (sc_inside() ? sbytes : 0)); }
     bool has_sc8() const { return type == PHX_Q4_0_DEV || type == PHX_Q8_0_DEV; }
     int64_t sc8_off() const { return (int64_t)nb * kRowGroup * pay; }  // scale groups within a row group
     int64_t mat_pay_stride() const { return (int64_t)rg * rg_pay; }
@@ -106,11 +113,7 @@ struct QMat {
 
 // Quantized activation rows for one weight type.
 //   ACT_Q8_0: q int8 [cols], d f32 [cols/32] (value of the fp16 scale), s int32 [cols/32] block sums
-//   ACT_K4:   q int8 [cols] permuted per 32-sub-block as dwords (l, m) = x[32s + l + 8m],
-//             d f32 [cols/256], s int32 [cols/16] (the Q8_K bsums)
-//   ACT_K6:   q int32 [cols/256][8 P][8 l][2] masked pair dwords, d f32 [cols/256],
-//             s int32 [cols/256][16 sub][8 l] offset terms -32*(x_l + x_{l+8})
-//   ACT_Q8K:  q int8 [cols] in element order, d f32 [cols/256] (the IQ types' Q8_K input)
+//   ACT_Q8K:  q int8 [cols] in element order, d f32 [cols/256] (the Q8_K input of the K and IQ types)
 struct Act {
     int fmt = ACT_Q8_0;
     int cols = 0;
@@ -121,12 +124,12 @@ struct Act {
     int* s = nullptr;
     int sstride = 0;      // ints per row
     uint16_t* qh = nullptr;  // optional: the same integers as fp16 bits [row][cols] (for MFMA); ACT_Q8_0 in
-                             // element order, the K formats per super-block in the order [l][s][mm']:
+                             // element order, ACT_Q8K per super-block in the order [l][s][mm']:
                              // x(32 s + l + 8 {0, 2, 1, 3}[mm'])
     int64_t qhstride = 0;    // halves per row
     bool fold = false;       // ACT_Q8_0 with qh: qh holds fp16(q * d), the block scale folded in (the
                              // tolerance mode's operands), instead of the integers
-    uint16_t* bh = nullptr;  // optional, K formats: the Q8_K block sums as fp16 [row][cols / 16]
+    uint16_t* bh = nullptr;  // optional, ACT_Q8K: the block sums of 16 as fp16 [row][cols / 16]
     int64_t bhstride = 0;    // halves per row
 };
 
@@ -160,10 +163,12 @@ void launch_topk(hipStream_t st, int T, int E, int k, int rule, const float* log
 void launch_dispatch(hipStream_t st, int n_assign, int E, int A, const int* ids, int* offsets, int* perm,
                      Tile* tiles, int* ntiles);
 // req: the paired gate|up product's down input (gelu(g) * u as Q8_0 rows, req_rows of them), formed in
-// the product's epilogue where it can be, else by k_requant after it
+// the product's epilogue where it can be, else by k_requant after it.  nident > 0 (K-quant types, tiles and
+// perm unused): one matrix over nident rows in order.  amax: no tile of the call holds more assignments
 void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
                     int A, const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
-                    const Act* req = nullptr, const float* gelu_tab = nullptr, int req_rows = 0);
+                    const Act* req = nullptr, const float* gelu_tab = nullptr, int req_rows = 0, int nident = 0,
+                    int amax = 4);
 void launch_requant(hipStream_t st, int rows, int nf, const float* g, const float* u, const float* gelu_tab, Act act);
 // standalone Q8_0 (fmt_k 0) / Q8_K (fmt_k 1) quantizer of rows x n inputs; mode as PHX_QUANT_*; -1 on a bad mode
 int launch_quant(hipStream_t st, int fmt_k, int mode, int rows, int n, float eps, const float* x, const float* aux,
@@ -256,7 +261,7 @@ void launch_copy_small(hipStream_t st, void* dst, const void* src, int64_t bytes
 void launch_copy_done(hipStream_t st, void* d0, const void* s0, void* d1, const void* s1, int64_t bytes, uint32_t* ctr,
                       uint32_t* done);
 void launch_planar_act(hipStream_t st, int rows, int n, const int8_t* qs, const uint16_t* d, Act a);
-// planar Q8_K rows (qs [rows][n], d [rows][n/256]) into a's K-quant orders (ACT_K4 / ACT_K6, qh / bh when set)
+// planar Q8_K rows (qs [rows][n], d [rows][n/256]) into a's matrix-core copies (d, qh, and bh when set)
 void launch_planar_act_k(hipStream_t st, int rows, int n, const int8_t* qs, const float* d, Act a);
 void launch_selftest(hipStream_t st, int op, int n, const float* a, const float* b, float* out, const float* gelu_tab);
 void launch_selftest_seq(hipStream_t st, int m, int rows, const float* a, float* out);

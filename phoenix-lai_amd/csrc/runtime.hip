@@ -115,8 +115,7 @@ int block_elems(int t) { return (t == PHX_Q4_0 || t == PHX_Q8_0) ? 32 : 256; }
 int dev_type(int t) { return t == PHX_Q3_K ? PHX_Q6_K : t; }
 int act_fmt(int t)
 {
-    t = dev_type(t);
-    return (t == PHX_Q4_K || t == PHX_Q5_K) ? ACT_K4 : t == PHX_Q6_K ? ACT_K6 : iq_type(t) ? ACT_Q8K : ACT_Q8_0;
+    return (t == PHX_Q4_0 || t == PHX_Q8_0) ? ACT_Q8_0 : ACT_Q8K;
 }
 int iq_pay(int t) { return t == PHX_IQ2_XXS ? 64 : t == PHX_IQ2_S ? 80 : 112; }
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
@@ -307,15 +306,19 @@ void repack(int type, const uint8_t* src, int n_mat, int rows, int cols, QMat& q
     q.sbytes = (type == PHX_Q4_K || type == PHX_Q5_K) ? 4 : 2;
     const int64_t rb = row_bytes(type, cols), bb = rb / q.nb;
     const int nb8 = (q.nb + 7) / 8;
-    q.rg_pay = (int64_t)q.nb * kRowGroup * q.pay + (q.has_sc8() ? (int64_t)nb8 * kRowGroup * 16 : 0);
+    q.rg_pay = q.blk_bytes() * q.nb + (q.has_sc8() ? (int64_t)nb8 * kRowGroup * 16 : 0);
     h.payload.assign((size_t)q.mat_pay_stride() * n_mat, 0);
-    h.scale.assign((size_t)q.mat_sc_stride() * n_mat, 0);
+    h.scale.assign(q.sc_inside() ? 16 : (size_t)q.mat_sc_stride() * n_mat, 0);
     const int64_t total_rows = (int64_t)n_mat * rows;
     unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
     std::vector<std::thread> th;
     for (unsigned w = 0; w < nt; w++) {
         th.emplace_back([&, w]() {
-            for (int64_t gr = w; gr < total_rows; gr += nt) {
+            // runs of 64 rows: a thread's 16-byte chunks fill whole cache lines
+            for (int64_t i = 0; i < total_rows; i++) {
+                const int64_t gr = 64 * (int64_t)w + i / 64 * 64 * nt + i % 64;
+                if (gr - gr % 64 >= total_rows) break;
+                if (gr >= total_rows) continue;
                 int m = (int)(gr / rows), r = (int)(gr % rows);
                 int rg = r / kRowGroup, lane = r % kRowGroup;
                 if (paired) {
@@ -325,10 +328,18 @@ void repack(int type, const uint8_t* src, int n_mat, int rows, int cols, QMat& q
                 }
                 const uint8_t* row = src + gr * rb;
                 uint8_t* rgp = h.payload.data() + ((int64_t)m * q.rg + rg) * q.rg_pay;
+                uint8_t blk[256];  // a block's payload before its 16-byte chunks are spread (K-quants)
                 for (int b = 0; b < q.nb; b++) {
                     int64_t idx = (((int64_t)m * q.rg + rg) * q.nb + b) * kRowGroup + lane;
-                    repack_block(type, row + b * bb, rgp + ((int64_t)b * kRowGroup + lane) * q.pay,
-                                 h.scale.data() + idx * q.sbytes);
+                    if (!q.sc_inside()) {
+                        repack_block(type, row + b * bb, rgp + ((int64_t)b * kRowGroup + lane) * q.pay,
+                                     h.scale.data() + idx * q.sbytes);
+                        continue;
+                    }
+                    uint8_t* base = rgp + b * q.blk_bytes();
+                    repack_block(type, row + b * bb, blk, base + kRowGroup * q.pay + lane * q.sbytes);
+                    uint8_t* dst = base + 16 * lane;
+                    for (int c = 0; c < q.pay / 16; c++) memcpy(dst + (int64_t)c * 16 * kRowGroup, blk + 16 * c, 16);
                 }
             }
         });
@@ -511,7 +522,7 @@ enum WsId {
     W_X, W_SHARED, W_OUT, W_RIN, W_XSCALE, W_AGU_Q, W_AGU_D, W_AGU_S, W_ASH_Q, W_ASH_D, W_ASH_S, W_LOGITS, W_IDS, W_W,
     W_OFF, W_PERM, W_TILES, W_NTILES, W_G, W_U, W_ADN_Q, W_ADN_D, W_ADN_S, W_YD, W_SHG, W_SHU, W_ASD_Q, W_ASD_D,
     W_ASD_S, W_SHOUT, W_ZERO, W_STILES, W_SNTILES, W_SOFF, W_SPERM, W_LB, W_BB, W_ADEC, W_SDEC, W_AGUP, W_ASHP, W_AGU_H, W_ADN_H, W_ASH_H, W_ASD_H, W_X2,
-    W_MM_IDS, W_MM_OFF, W_MM_PERM, W_MM_TILES, W_MM_NT, W_MM_D, W_MM_S, W_MM_H, W_AGU_BH, W_ADN_BH, W_MK_Q, W_MK_BH, W_KB,
+    W_MM_IDS, W_MM_OFF, W_MM_PERM, W_MM_TILES, W_MM_NT, W_MM_D, W_MM_S, W_MM_H, W_AGU_BH, W_ADN_BH, W_MK_BH, W_KB,
     W_CBAD, W_RSCALE, W_COUNT
 };
 
@@ -545,9 +556,7 @@ template <class T> T* wp(phx_moe_ctx* c, int id) { return (T*)c->ws[id].p; }
 void act_sizes(int fmt, int64_t rows, int cols, size_t& qb, size_t& db, size_t& sb)
 {
     if (fmt == ACT_Q8_0) { qb = rows * cols; db = rows * (cols / 32) * 4; sb = rows * (cols / 32) * 4; }
-    else if (fmt == ACT_K4) { qb = rows * cols; db = rows * (cols / 256) * 4; sb = rows * (cols / 16) * 4; }
-    else if (fmt == ACT_Q8K) { qb = rows * cols; db = rows * (cols / 256) * 4; sb = 4; }
-    else { qb = rows * (cols / 256) * 512; db = rows * (cols / 256) * 4; sb = rows * (cols / 256) * 128 * 4; }
+    else { qb = rows * cols; db = rows * (cols / 256) * 4; sb = 4; }
 }
 
 Act make_act(phx_moe_ctx* c, int fmt, int cols, int qid, int did, int sid)
@@ -559,9 +568,7 @@ Act make_act(phx_moe_ctx* c, int fmt, int cols, int qid, int did, int sid)
     a.d = wp<float>(c, did);
     a.s = wp<int>(c, sid);
     if (fmt == ACT_Q8_0) { a.qstride = cols; a.dstride = cols / 32; a.sstride = cols / 32; }
-    else if (fmt == ACT_K4) { a.qstride = cols; a.dstride = cols / 256; a.sstride = cols / 16; }
-    else if (fmt == ACT_Q8K) { a.qstride = cols; a.dstride = cols / 256; a.sstride = 0; }
-    else { a.qstride = (int64_t)(cols / 256) * 512; a.dstride = cols / 256; a.sstride = (cols / 256) * 128; }
+    else { a.qstride = cols; a.dstride = cols / 256; a.sstride = 0; }
     return a;
 }
 
@@ -995,7 +1002,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
                                 wp<float>(c, W_G), wp<float>(c, W_U), nf, nf);
         else  // the down input from the product's epilogue (or k_requant right after it)
             launch_grouped(st, L.gu, agu, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, tileA, wp<int>(c, W_PERM),
-                           k, wp<float>(c, W_G), wp<float>(c, W_U), nf, nf, &adn, c->gelu_tab, n);
+                           k, wp<float>(c, W_G), wp<float>(c, W_U), nf, nf, &adn, c->gelu_tab, n, 0, T);
     }
     if (kmma) {
         ProfScope p(c, PHX_K_REQUANT);
@@ -1011,7 +1018,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
                                 wp<float>(c, W_YD), wp<float>(c, W_YD), d, d);
         else
             launch_grouped(st, L.dn, adn, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, tileA, wp<int>(c, W_PERM),
-                           1, wp<float>(c, W_YD), wp<float>(c, W_YD), d, d);
+                           1, wp<float>(c, W_YD), wp<float>(c, W_YD), d, d, nullptr, nullptr, 0, 0, T);
     }
     const float* sh = shared;
     if (shared_ffn) {
@@ -1033,13 +1040,13 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
                                 nullptr, nullptr, nff, nff, 0, &asd, T, c->gelu_tab);  // (no reader of g, u)
         else
             launch_grouped(st, L.sgu, ash, wp<Tile>(c, W_STILES), wp<int>(c, W_SNTILES), smax, kTileA, wp<int>(c, W_SPERM),
-                           1, wp<float>(c, W_SHG), wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T);
+                           1, wp<float>(c, W_SHG), wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T, 0, T);
         if (smma)
             launch_grouped_mfma(st, L.sdn, asd, wp<Tile>(c, W_STILES), wp<int>(c, W_SNTILES), smax, wp<int>(c, W_SPERM), 1,
                                 wp<float>(c, W_SHOUT), wp<float>(c, W_SHOUT), d, d, T);
         else
             launch_grouped(st, L.sdn, asd, wp<Tile>(c, W_STILES), wp<int>(c, W_SNTILES), smax, kTileA, wp<int>(c, W_SPERM),
-                           1, wp<float>(c, W_SHOUT), wp<float>(c, W_SHOUT), d, d);
+                           1, wp<float>(c, W_SHOUT), wp<float>(c, W_SHOUT), d, d, nullptr, nullptr, 0, 0, T);
         sh = wp<float>(c, W_SHOUT);
     }
     {
@@ -2049,15 +2056,28 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
     if ((uintptr_t)xq % 4 || (uintptr_t)xd % 4 || (uintptr_t)y % 4)
         return set_err(c, PHX_ERR_ARG, "matmul_k: xq, xd and y need 4-byte alignment");
     ENTER(c);
-    const int fmt = act_fmt(w->type), cols = w->cols;
+    const int cols = w->cols;
     // the general path's rule with one matrix (at least 8 rows per matrix): the matrix cores, else the
     // VALU row walk
     const bool kmma = T >= 8 && kmma_type(w->type);
     const int A = kmma ? kKmmaTile : kTileA;
     const int max_tiles = (T + A - 1) / A;
-    size_t qb, db, sb;
-    act_sizes(fmt, T, cols, qb, db, sb);
+    hipStream_t st = c->stream;
     int rc;
+    if (!kmma) {
+        // the VALU rows read the caller's planar rows and take them in order: one launch, no workspace
+        Act a;
+        a.fmt = ACT_Q8K;
+        a.cols = cols;
+        a.q = (int8_t*)xq;
+        a.qstride = cols;
+        a.d = (float*)xd;
+        a.dstride = cols / 256;
+        launch_grouped(st, w->q, a, nullptr, nullptr, max_tiles, A, nullptr, 1, y, y, w->rows, w->rows, nullptr, nullptr, 0,
+                       T, T);
+        HIPCHK(c, launch_status(c));
+        return PHX_OK;
+    }
 #define ENS(id, bytes) \
     if ((rc = ensure(c, id, (size_t)(bytes)))) return rc
     ENS(W_MM_IDS, (size_t)T * 4);
@@ -2065,32 +2085,27 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
     ENS(W_MM_PERM, (size_t)T * 4);
     ENS(W_MM_TILES, (size_t)max_tiles * sizeof(Tile));
     ENS(W_MM_NT, 4);
-    ENS(W_MK_Q, qb);
-    ENS(W_MM_D, db);
-    ENS(W_MM_S, sb);
-    if (kmma) ENS(W_MM_H, (size_t)T * cols * 2);
-    if (kmma && fmt == ACT_K4) ENS(W_MK_BH, (size_t)T * (cols / 16) * 2);
+    ENS(W_MM_D, (size_t)T * (cols / 256) * 4);
+    ENS(W_MM_H, (size_t)T * cols * 2);
+    if (w->type == PHX_Q4_K) ENS(W_MK_BH, (size_t)T * (cols / 16) * 2);
 #undef ENS
-    hipStream_t st = c->stream;
-    Act a = make_act(c, fmt, cols, W_MK_Q, W_MM_D, W_MM_S);
-    if (kmma) {
-        a.qh = wp<uint16_t>(c, W_MM_H);
-        a.qhstride = cols;
-        if (fmt == ACT_K4) {
-            a.bh = wp<uint16_t>(c, W_MK_BH);
-            a.bhstride = cols / 16;
-        }
+    Act a;
+    a.fmt = ACT_Q8K;
+    a.cols = cols;
+    a.d = wp<float>(c, W_MM_D);
+    a.dstride = cols / 256;
+    a.qh = wp<uint16_t>(c, W_MM_H);
+    a.qhstride = cols;
+    if (w->type == PHX_Q4_K) {
+        a.bh = wp<uint16_t>(c, W_MK_BH);
+        a.bhstride = cols / 16;
     }
     launch_planar_act_k(st, T, cols, xq, xd, a);
     launch_fill_u32(st, (uint32_t*)wp<int>(c, W_MM_IDS), T, 0u);
     launch_dispatch(st, T, 1, A, wp<int>(c, W_MM_IDS), wp<int>(c, W_MM_OFF), wp<int>(c, W_MM_PERM),
                     wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT));
-    if (kmma)
-        launch_grouped_kmma(st, w->q, a, wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT), max_tiles, wp<int>(c, W_MM_PERM), 1,
-                            y, y, w->rows, w->rows);
-    else
-        launch_grouped(st, w->q, a, wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT), max_tiles, A, wp<int>(c, W_MM_PERM), 1,
-                       y, y, w->rows, w->rows);
+    launch_grouped_kmma(st, w->q, a, wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT), max_tiles, wp<int>(c, W_MM_PERM), 1, y,
+                        y, w->rows, w->rows);
     HIPCHK(c, launch_status(c));
     return PHX_OK;
 }
