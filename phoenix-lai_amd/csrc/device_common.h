@@ -644,4 +644,85 @@ __device__ __forceinline__ void tie(u32x4& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void tie(u32x2& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void tie(uint32_t& v) { asm volatile("" : "+v"(v)); }
 
+// Q8_K of one 256-element super-block held as four consecutive values per lane of a wave
+// (CpuRef.QuantizeQ8_K, src/CpuRefKQuants.cs:53-86): the lane's four integers as bytes; *dval the scale.
+__device__ __forceinline__ uint32_t q8_k_wave(float4 v4, float* dval)
+{
+    const int lane = threadIdx.x & 63;
+    const float x[4] = {v4.x, v4.y, v4.z, v4.w};
+    // the reference's scan: the first element of largest |x| (strict '>', from 0)
+    float amax = 0.0f, vmax = 0.0f;
+    int imax = 1 << 30;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (fabsf(x[j]) > amax) {
+            amax = fabsf(x[j]);
+            vmax = x[j];
+            imax = 4 * lane + j;
+        }
+    // the wave's first largest |x| by DPP steps (lanes outside a step's rows keep their own triple),
+    // lane 63 ending with the result
+    auto step = [&](auto C, auto RM) {
+        constexpr int CTRL = decltype(C)::value, ROWMASK = decltype(RM)::value;
+        const float oa = dpp_f<CTRL, ROWMASK>(amax, amax), ov = dpp_f<CTRL, ROWMASK>(vmax, vmax);
+        const int oi = dpp_i<CTRL, ROWMASK>(imax, imax);
+        if (oa > amax || (oa == amax && oi < imax)) {
+            amax = oa;
+            vmax = ov;
+            imax = oi;
+        }
+    };
+    step(ic<0xb1>{}, ic<0xf>{});
+    step(ic<0x4e>{}, ic<0xf>{});
+    step(ic<0x141>{}, ic<0xf>{});
+    step(ic<0x140>{}, ic<0xf>{});
+    step(ic<0x142>{}, ic<0xa>{});
+    step(ic<0x143>{}, ic<0xc>{});
+    amax = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(amax), 63));
+    vmax = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(vmax), 63));
+    const float iscale = amax == 0.0f ? 0.0f : -127.0f / vmax;
+    int q[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) q[j] = amax == 0.0f ? 0 : min(nearest_int(iscale * x[j]), 127);
+    *dval = amax == 0.0f ? 0.0f : 1.0f / iscale;
+    return (uint32_t)(q[0] & 0xFF) | ((uint32_t)(q[1] & 0xFF) << 8) | ((uint32_t)(q[2] & 0xFF) << 16) |
+           ((uint32_t)q[3] << 24);
+}
+
+// The integers of Q8_K super-block b of row `row` (lane l holds elements 4l..4l+3 packed in pk) stored as
+// act's rows, with the sums of 16 (bh when set) and, with qh set, the matrix cores' fp16 copies; the block's
+// scale is the caller's.  qrow is the wave's 64-dword LDS row through which the integers reach the fp16
+// copies' order.  Wave-level: all 64 lanes call it.
+__device__ __forceinline__ void store_q8k_block(const Act& act, int64_t row, int b, int lane, uint32_t pk,
+                                                uint32_t* qrow, float dval)
+{
+    if (act.bh) {  // uniform; block sums of 16: lanes 4j .. 4j + 3
+        int sm = (int)(int8_t)(pk & 0xFF) + (int)(int8_t)((pk >> 8) & 0xFF) + (int)(int8_t)((pk >> 16) & 0xFF) +
+                 (int)(int8_t)(pk >> 24);
+        sm += dpp_i<0xb1>(sm, sm);  // 4-lane sum: quad swaps
+        sm += dpp_i<0x4e>(sm, sm);
+        if ((lane & 3) == 0)
+            act.bh[row * act.bhstride + b * 16 + (lane >> 2)] = (uint16_t)f2h_bits((float)sm);  // exact
+    }
+    if (act.q) ((uint32_t*)(act.q + row * act.qstride + (int64_t)b * 256))[lane] = pk;
+    if (!act.qh) return;  // uniform
+    const uint8_t* qb = (const uint8_t*)qrow;
+    qrow[lane] = pk;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    auto qv = [&](int e) { return (int)(int8_t)qb[e]; };
+    // the matrix cores' copy: exact fp16 integers (or, folded, fp16 of q * dval), halves [l][s][mm']:
+    // lane = 8 l + s
+    const int l = lane >> 3, s8 = lane & 7, e = 32 * s8 + l;
+    uint32_t* hq = (uint32_t*)(act.qh + row * act.qhstride + (int64_t)b * 256) + l * 16 + s8 * 2;
+    const float f = act.fold ? dval : 1.0f;
+    hq[0] = f2h_bits((float)qv(e) * f) | (f2h_bits((float)qv(e + 16) * f) << 16);
+    hq[1] = f2h_bits((float)qv(e + 8) * f) | (f2h_bits((float)qv(e + 24) * f) << 16);
+    // the row is rewritten by the wave's next block only after every lane's reads above
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace phx

@@ -99,6 +99,8 @@ struct DecArgs {
     const float* xin;     // with xres: the residual's source rows when not xres itself (or null)
     const float* gelu_tab;
     int* flags;           // [0] norm fallbacks, [1] router fallbacks
+    Tile* gtiles;         // one token: the general path's tile list and count, written by the selection (or null)
+    int* ngtiles;
 };
 
 // ------------------------------------------------------------------------------ helpers
@@ -585,7 +587,27 @@ __device__ __forceinline__ void store_qh(const Act& act, int t, int b, int l8, i
     *(uint2*)(act.qh + (int64_t)t * act.qhstride + 32 * b + 4 * l8) = act.fold ? fold_q4(qw, dval) : int_q4(qw);
 }
 
-template <int PER, bool FUSED>
+// The token's Q8_K input rows (K-quant and IQ weights; either input may still be Q8_0): super-block i of the
+// waves `first`, `first` + stride, ... (one per wave, whole waves), through the wave's LDS row qrow.
+__device__ __forceinline__ void route_q8k(const DecArgs& a, int t, int first, int stride, const float* sx, float rinv,
+                                          uint32_t* qrow)
+{
+    const int lane = threadIdx.x & 63;
+    auto one = [&](const Act& act, const float* norm, int i) {
+        const float4 xv = *(const float4*)(sx + 256 * i + 4 * lane), nv = ((const float4*)norm)[64 * i + lane];
+        float dval;
+        const uint32_t pk = q8_k_wave(
+            make_float4((xv.x * rinv) * nv.x, (xv.y * rinv) * nv.y, (xv.z * rinv) * nv.z, (xv.w * rinv) * nv.w), &dval);
+        if (lane == 0) act.d[(int64_t)t * act.dstride + i] = dval;
+        store_q8k_block(act, t, i, lane, pk, qrow, dval);
+    };
+    for (int i = first; i < a.d / 256; i += stride) {  // wave-uniform
+        if (a.agu.fmt == ACT_Q8K) one(a.agu, a.pre2, i);
+        if (a.ash.q && a.ash.fmt == ACT_Q8K) one(a.ash, a.fnorm, i);
+    }
+}
+
+template <int PER, bool FUSED, bool KQ>
 __device__ __forceinline__ void route_wg(const DecArgs& a, int t, int e, float* sx, float* sg, float* sw,
                                          const CombArgs& prev, float* scb)
 {
@@ -707,16 +729,18 @@ __device__ __forceinline__ void route_wg(const DecArgs& a, int t, int e, float* 
         const float4 xq = *(const float4*)(sx + 32 * b + 4 * l8);
         float dval;
         int sum;
-        const int qw = q8_0_oct(make_float4((xq.x * rinv) * nv.x, (xq.y * rinv) * nv.y, (xq.z * rinv) * nv.z,
-                                            (xq.w * rinv) * nv.w),
-                                &dval, &sum);
-        ((int*)(a.agu.q + (int64_t)t * a.agu.qstride))[8 * b + l8] = qw;
-        if (a.agu.qh) store_qh(a.agu, t, b, l8, qw, dval);
-        if (l8 == 0) {
-            a.agu.d[(int64_t)t * a.agu.dstride + b] = dval;
-            a.agu.s[(int64_t)t * a.agu.sstride + b] = sum;
+        if (!KQ || a.agu.fmt == ACT_Q8_0) {
+            const int qw = q8_0_oct(make_float4((xq.x * rinv) * nv.x, (xq.y * rinv) * nv.y, (xq.z * rinv) * nv.z,
+                                                (xq.w * rinv) * nv.w),
+                                    &dval, &sum);
+            ((int*)(a.agu.q + (int64_t)t * a.agu.qstride))[8 * b + l8] = qw;
+            if (a.agu.qh) store_qh(a.agu, t, b, l8, qw, dval);
+            if (l8 == 0) {
+                a.agu.d[(int64_t)t * a.agu.dstride + b] = dval;
+                a.agu.s[(int64_t)t * a.agu.sstride + b] = sum;
+            }
         }
-        if (a.ash.q) {
+        if (a.ash.q && (!KQ || a.ash.fmt == ACT_Q8_0)) {
             const int qs = q8_0_oct(make_float4((xq.x * rinv) * fv.x, (xq.y * rinv) * fv.y, (xq.z * rinv) * fv.z,
                                                 (xq.w * rinv) * fv.w),
                                     &dval, &sum);
@@ -728,6 +752,10 @@ __device__ __forceinline__ void route_wg(const DecArgs& a, int t, int e, float* 
             }
         }
     }
+    if constexpr (KQ) {  // from the last wave on, as the 32-blocks
+        __shared__ uint32_t qsm[RT_MAXW][64];
+        route_q8k(a, t, e + (nw - 1 - wave) * a.E, nw * a.E, sx, rinv, qsm[wave]);
+    }
     TL_STAMP(a.seq, 0, 3);
 }
 
@@ -735,7 +763,7 @@ __device__ __forceinline__ void route_wg(const DecArgs& a, int t, int e, float* 
 // staging's clamped last loads land in the padding)
 __host__ __device__ inline int route_row_floats(int d, int nt) { return (d / 4 + nt - 1) / nt * nt * 4; }
 
-template <int PER, bool FUSED>
+template <int PER, bool FUSED, bool KQ = false>
 __device__ __forceinline__ void route_at(const DecArgs& a, const CombArgs& prev, float* rsm)
 {
     const int t = blockIdx.x / a.E, e = blockIdx.x % a.E, dp = route_row_floats(a.d, blockDim.x);
@@ -743,14 +771,15 @@ __device__ __forceinline__ void route_at(const DecArgs& a, const CombArgs& prev,
     float* sg = sx + dp;
     float* sw = sg + dp;
     float* scb = sw + dp;  // fused: the combine's two rows
-    route_wg<PER, FUSED>(a, t, e, sx, sg, sw, prev, scb);
+    route_wg<PER, FUSED, KQ>(a, t, e, sx, sg, sw, prev, scb);
 }
 
-template <int PER>
+// KQ: at least one of the layer's inputs is Q8_K
+template <int PER, bool KQ>
 __global__ __launch_bounds__(64 * RT_MAXW) void k_dec_route(DecArgs a)
 {
     extern __shared__ __align__(16) float rsm[];  // x, router scale, W row: route_row_floats(d, NT) each
-    route_at<PER, false>(a, CombArgs{}, rsm);
+    route_at<PER, false, KQ>(a, CombArgs{}, rsm);
 }
 
 // A layer of a stack whose previous layer's combine is folded in: every (token, expert) workgroup forms
@@ -770,7 +799,7 @@ __global__ __launch_bounds__(64 * RT_MAXW) void k_dec_route_fused(CombArgs prev,
 // per token, g this one's index) are quantized here, as route_wg quantizes b = e + E j.  (Two experts
 // per workgroup measured no faster at C5: 15.6 against 15.4 us.)
 constexpr int RT_RX = 4;
-template <int PER>
+template <int PER, bool KQ>
 __global__ __launch_bounds__(256) void k_dec_route_mx(DecArgs a)
 {
     extern __shared__ __align__(16) float rsm[];  // x, router scale, RT_RX W rows: route_row_floats(d, NT) each
@@ -883,16 +912,18 @@ __global__ __launch_bounds__(256) void k_dec_route_mx(DecArgs a)
         const float4 xq = *(const float4*)(sx + 32 * b + 4 * l8);
         float dval;
         int sum;
-        const int qw = q8_0_oct(make_float4((xq.x * rinv) * nv.x, (xq.y * rinv) * nv.y, (xq.z * rinv) * nv.z,
-                                            (xq.w * rinv) * nv.w),
-                                &dval, &sum);
-        ((int*)(a.agu.q + (int64_t)t * a.agu.qstride))[8 * b + l8] = qw;
-        if (a.agu.qh) store_qh(a.agu, t, b, l8, qw, dval);
-        if (l8 == 0) {
-            a.agu.d[(int64_t)t * a.agu.dstride + b] = dval;
-            a.agu.s[(int64_t)t * a.agu.sstride + b] = sum;
+        if (!KQ || a.agu.fmt == ACT_Q8_0) {
+            const int qw = q8_0_oct(make_float4((xq.x * rinv) * nv.x, (xq.y * rinv) * nv.y, (xq.z * rinv) * nv.z,
+                                                (xq.w * rinv) * nv.w),
+                                    &dval, &sum);
+            ((int*)(a.agu.q + (int64_t)t * a.agu.qstride))[8 * b + l8] = qw;
+            if (a.agu.qh) store_qh(a.agu, t, b, l8, qw, dval);
+            if (l8 == 0) {
+                a.agu.d[(int64_t)t * a.agu.dstride + b] = dval;
+                a.agu.s[(int64_t)t * a.agu.sstride + b] = sum;
+            }
         }
-        if (a.ash.q) {
+        if (a.ash.q && (!KQ || a.ash.fmt == ACT_Q8_0)) {
             const int qs = q8_0_oct(make_float4((xq.x * rinv) * fv.x, (xq.y * rinv) * fv.y, (xq.z * rinv) * fv.z,
                                                 (xq.w * rinv) * fv.w),
                                     &dval, &sum);
@@ -904,13 +935,17 @@ __global__ __launch_bounds__(256) void k_dec_route_mx(DecArgs a)
             }
         }
     }
+    if constexpr (KQ) {
+        __shared__ uint32_t qsm[RT_MAXW][64];
+        route_q8k(a, t, eg + (nw - 1 - wave) * G, nw * G, sx, rinv, qsm[wave]);
+    }
 }
-template <int P> struct KRouteMx { static constexpr auto fn = k_dec_route_mx<P>; };
+template <int P, bool KQ> struct KRouteMx { static constexpr auto fn = k_dec_route_mx<P, KQ>; };
 
 // Elements per thread: 4 (d / 4 threads) for a stack's few tokens, where the router's chain of
 // reductions is the layer's latency; d / 256 (256 threads) for many tokens, where more workgroups per CU
 // hide each other's barriers.  Each width is its own instantiation (its own register budget).
-template <int P> struct KRoute { static constexpr auto fn = k_dec_route<P>; };
+template <int P> struct KRoute { static constexpr auto fn = k_dec_route<P, false>; };
 static int route_per(int T, int E, int d) { return (int64_t)T * E > 1024 ? d / 256 : 4; }
 static auto route_kernel(int per)
 {
@@ -1595,6 +1630,27 @@ __global__ __launch_bounds__(CF_NT) void k_cert_select_one(DecArgs a)
     const bool exact = s_bad != 0;  // uniform
     if (exact) select_exact<true>(b, csm, s_ids, &s_bad, red, true);
     if (wave == 0) token_routing_out(a, t, exact ? (const double*)csm : b.Lb, s_ids);
+    // one token: its lists here, as k_dispatch would write them (an assignment per expert, in expert order)
+    if (!a.gtiles) return;  // uniform
+    __syncthreads();        // the exact selection's ids
+    if (wave == 1) {
+        const int id = clamp_id(s_ids[min(lane, a.k - 1)], a.E);
+        int pos = 0;
+        for (int j = 0; j < a.k; j++) {
+            const int o = __builtin_amdgcn_readlane(id, j);
+            pos += o < id || (o == id && j < lane);
+        }
+        if (lane < a.k) {
+            a.perm[pos] = lane;
+            a.gtiles[pos] = Tile{id, pos, 1};
+        }
+        if (lane == 0) *a.ngtiles = a.k;
+        for (int e = lane; e <= a.E; e += 64) {
+            int c = 0;
+            for (int j = 0; j < a.k; j++) c += __builtin_amdgcn_readlane(id, j) < e;
+            a.offsets[e] = c;
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------ k_router_mm
@@ -2188,6 +2244,8 @@ static DecArgs dec_args(const DecLayerH& h)
     a.xin = h.xin;
     a.gelu_tab = h.gelu_tab;
     a.flags = h.flags;
+    a.gtiles = h.gtiles;
+    a.ngtiles = h.ngtiles;
     return a;
 }
 
@@ -2236,41 +2294,55 @@ template <int T> struct KGu { static constexpr auto fn = k_dec_gu<T, 768>; };
 template <int T> struct KGuW { static constexpr auto fn = k_dec_gu<T, 1024>; };
 template <int T> struct KDown { static constexpr auto fn = k_dec_down<T>; };
 
+template <bool KQ>
 static auto route_mx_kernel(int per)
 {
     switch (per) {
-    case 1: return KRouteMx<1>::fn;
-    case 2: return KRouteMx<2>::fn;
-    case 3: return KRouteMx<3>::fn;
-    case 4: return KRouteMx<4>::fn;
-    case 5: return KRouteMx<5>::fn;
-    case 6: return KRouteMx<6>::fn;
-    case 7: return KRouteMx<7>::fn;
-    case 8: return KRouteMx<8>::fn;
-    case 9: return KRouteMx<9>::fn;
-    case 10: return KRouteMx<10>::fn;
-    case 11: return KRouteMx<11>::fn;
-    case 12: return KRouteMx<12>::fn;
-    case 13: return KRouteMx<13>::fn;
-    case 14: return KRouteMx<14>::fn;
-    case 15: return KRouteMx<15>::fn;
-    default: return KRouteMx<16>::fn;
+    case 1: return KRouteMx<1, KQ>::fn;
+    case 2: return KRouteMx<2, KQ>::fn;
+    case 3: return KRouteMx<3, KQ>::fn;
+    case 4: return KRouteMx<4, KQ>::fn;
+    case 5: return KRouteMx<5, KQ>::fn;
+    case 6: return KRouteMx<6, KQ>::fn;
+    case 7: return KRouteMx<7, KQ>::fn;
+    case 8: return KRouteMx<8, KQ>::fn;
+    case 9: return KRouteMx<9, KQ>::fn;
+    case 10: return KRouteMx<10, KQ>::fn;
+    case 11: return KRouteMx<11, KQ>::fn;
+    case 12: return KRouteMx<12, KQ>::fn;
+    case 13: return KRouteMx<13, KQ>::fn;
+    case 14: return KRouteMx<14, KQ>::fn;
+    case 15: return KRouteMx<15, KQ>::fn;
+    default: return KRouteMx<16, KQ>::fn;
     }
 }
+
+// whether launch_dec_route takes the layer's Q8_K inputs: whole super-blocks, and its workgroups' waves cover them
+// (d / 4 threads and every expert always do)
+static bool route_mx(const DecLayerH& h)
+{
+    const int nt = h.d / route_per(h.T, h.E, h.d);
+    return (int64_t)h.T * h.E > 1024 && h.E % RT_RX == 0 && h.d / 32 <= nt / 8 * (h.E / RT_RX);
+}
+bool dec_route_q8k(const DecLayerH& h) { return (int64_t)h.T * h.E <= 1024 || route_mx(h); }
 
 void launch_dec_route(hipStream_t st, const DecLayerH& h)
 {
     const int per = route_per(h.T, h.E, h.d), nt = h.d / per;
+    const bool kq = h.agu.fmt == ACT_Q8K || (h.sgu && h.ash.q && h.ash.fmt == ACT_Q8K);  // dec_route_q8k(h) holds
     // a workgroup per token and RT_RX experts, where its 8-lane groups cover the token's input blocks
-    if ((int64_t)h.T * h.E > 1024 && h.E % RT_RX == 0 && h.d / 32 <= nt / 8 * (h.E / RT_RX)) {
+    if (route_mx(h)) {
         const size_t lds = (size_t)(2 + RT_RX) * route_row_floats(h.d, nt) * 4;
-        const auto kr = route_mx_kernel(per);
-        raise_lds(kr, lds);
-        launch(kr, dim3(h.T * (h.E / RT_RX)), dim3(nt), (uint32_t)lds, st, dec_args(h));
+        auto go = [&](auto kr) {
+            raise_lds(kr, lds);
+            launch(kr, dim3(h.T * (h.E / RT_RX)), dim3(nt), (uint32_t)lds, st, dec_args(h));
+        };
+        if (kq) go(route_mx_kernel<true>(per));
+        else go(route_mx_kernel<false>(per));
         return;
     }
     const size_t lds = (size_t)3 * route_row_floats(h.d, nt) * 4;
-    const auto kr = route_kernel(per);
+    const auto kr = kq ? k_dec_route<4, true> : route_kernel(per);
     raise_lds(kr, lds);
     launch(kr, dim3(h.T * h.E), dim3(nt), (uint32_t)lds, st, dec_args(h));
 }

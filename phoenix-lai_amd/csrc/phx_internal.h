@@ -219,11 +219,15 @@ struct DecLayerH {
     float *w, *logits, *g, *u, *yd, *shg, *shu, *shout, *out, *xres;
     const float* xin = nullptr;  // the residual's source rows when not xres itself
     DecTile* tiles;
+    Tile* gtiles = nullptr;  // launch_cert_select, one token: also write the general path's lists here
+    int* ngtiles = nullptr;
     Act agu, ash, adn, asd;  // packed Q8_0 rows: expert and shared inputs [T], down inputs [T*k], [T]
     const float* gelu_tab;
 };
 bool dec_supported(const DecLayerH& h);
 void launch_dec_route(hipStream_t st, const DecLayerH& h);
+// whether launch_dec_route can write Q8_K input rows (agu or ash ACT_Q8K) for this call
+bool dec_route_q8k(const DecLayerH& h);
 // the general path's selection from k_dec_route's certified sums: ids, weights and logits per token
 void launch_cert_select(hipStream_t st, const DecLayerH& h);
 // whether launch_cert_select runs as one launch (a workgroup per token in at most two rounds over the

@@ -836,7 +836,8 @@ int run_layer_decode(phx_moe_ctx* c, const Layer& L, int T, const float* x, cons
 // The general path routes through the certified router (k_dec_route's double sums and bounds, then
 // k_cert_select: the decode path's selection, exact chains for a token it cannot certify) where the
 // router launch has few enough workgroups (T * E of them, each reading a router row) and the expert
-// input is Q8_0 (k_dec_route writes it, with the matrix cores' fp16 copy where the rows carry one);
+// input is quantized there (Q8_0 by 8-lane groups, Q8_K by whole waves, with the matrix cores' fp16 copy
+// where the rows carry one);
 // otherwise, and always under PHX_FLAG_EXACT_ROUTER, through the exact float chains.
 // The router workgroups also quantize the expert (and shared) input: workgroup (t, e) takes blocks
 // e + g E for each of its eight-thread groups g, so the groups of a token's E workgroups must cover its
@@ -847,8 +848,12 @@ bool cert_route(const Layer& L, int T, bool shared_ffn)
     const phx_moe_layer_desc& D = L.desc;
     if ((int64_t)T * D.n_expert > CERT_MAX_TE || D.d > 4096 || D.d % 256 != 0 || D.n_expert > 256) return false;
     if (D.d / 32 > 32 * D.n_expert) return false;
-    if (!dec_type(D.gate_up_type) || (shared_ffn && !dec_type(D.shared_type))) return false;
-    return true;
+    if (dec_type(D.gate_up_type) && (!shared_ffn || dec_type(D.shared_type))) return true;
+    DecLayerH h{};  // Q8_K inputs (K-quant and IQ weights): whole super-blocks by the router's waves
+    h.T = T;
+    h.d = D.d;
+    h.E = D.n_expert;
+    return dec_route_q8k(h);
 }
 
 // prefill-sized expert work (several assignments per expert on average) runs on the matrix cores, whose
@@ -913,6 +918,10 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
         }
         {
             ProfScope p(c, PHX_K_TOPK);
+            if (T == 1) {  // the selection writes the one token's lists too
+                h.gtiles = wp<Tile>(c, W_TILES);
+                h.ngtiles = wp<int>(c, W_NTILES);
+            }
             launch_cert_select(st, h);
         }
     } else {
@@ -975,7 +984,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
     // walk is VALU-bound: larger tiles cost occupancy and measured slower)
     const int tileA = mma ? kMmaTile : kmma ? kKmmaTile : kTileA;
     const int max_tiles = std::min(n, (n + tileA - 1) / tileA + E);
-    {
+    if (!(cert && T == 1)) {
         ProfScope p(c, PHX_K_DISPATCH);
         launch_dispatch(st, n, E, tileA, wp<int>(c, W_IDS), wp<int>(c, W_OFF), wp<int>(c, W_PERM), wp<Tile>(c, W_TILES),
                         wp<int>(c, W_NTILES));
