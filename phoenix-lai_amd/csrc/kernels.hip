@@ -782,6 +782,9 @@ void launch_dispatch(hipStream_t st, int n, int E, int A, const int* ids, int* o
 // reference row dot: sum += (float)isum * (d_w * d_x) (src/CpuRefGemma.cs:27-36, src/CpuRef.cs:106-115).
 // Weights are read once per tile for all its assignments; activations are wave-uniform.
 
+// a 16-byte load of rows that are only 4-byte aligned
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
 struct GroupArgs {
     const uint8_t* payload;
     const uint8_t* scale;
@@ -796,13 +799,28 @@ struct GroupArgs {
     float* out1;
     int split, out_stride;
     bool paired;
+    const uint16_t* d16 = nullptr;  // k_grouped_q_wide: the scales as planar fp16 bits (act.d unused)
     int nident = 0;    // > 0 (tiles null): one matrix, tile i the rows 4 i .. 4 i + 3 of nident, in order
-    int amax = 4;      // k_grouped_k: assignments a tile can hold in this call (its LDS), and the most tiles
+    int amax = 4;      // k_grouped_k, k_grouped_q_wide: assignments a tile can hold in this call (its LDS), and the most tiles
     int mt = 1;        // (workgroup b: tile b % mt, row group b / mt)
     const void* grid;  // IQ types: the expanded codebook (64-bit words for IQ2_XXS / IQ2_S, 32-bit for IQ3_S)
     Act req;                       // req.q set: the paired gate|up kernel also writes gelu(g) * u as Q8_0 rows
     const float* gelu_tab = nullptr;
 };
+
+// the workgroup's tile (four list positions at most), false past the last one (uniform), and the assignment at
+// list position p
+__device__ __forceinline__ bool group_tile(const GroupArgs& g, int tile, Tile* tl)
+{
+    if (g.nident) {
+        *tl = Tile{0, 4 * tile, min(4, g.nident - 4 * tile)};
+        return true;
+    }
+    if (tile >= *g.ntiles) return false;
+    *tl = g.tiles[tile];
+    return true;
+}
+__device__ __forceinline__ int group_perm(const GroupArgs& g, int p) { return g.nident ? p : g.perm[p]; }
 
 // Output of lane `lane` of row group rgi for assignment row a: natural row order, or for a paired
 // gate|up matrix lanes 0-31 = gate output 32 rgi + lane, lanes 32-63 = the matching up output.
@@ -847,8 +865,8 @@ template <int TYPE, int A>
 __global__ __launch_bounds__(256) void k_grouped_q(GroupArgs g)
 {
     const int tile = blockIdx.x;
-    if (tile >= *g.ntiles) return;
-    const Tile tl = g.tiles[tile];
+    Tile tl;
+    if (!group_tile(g, tile, &tl)) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int rgi = blockIdx.y * 4 + wave;
     if (rgi >= g.rg) return;
@@ -859,7 +877,7 @@ __global__ __launch_bounds__(256) void k_grouped_q(GroupArgs g)
     float acc[A];
 #pragma unroll
     for (int i = 0; i < A; i++) {
-        arow[i] = i < tl.cnt ? g.perm[tl.start + i] / g.act_div : 0;
+        arow[i] = i < tl.cnt ? group_perm(g, tl.start + i) / g.act_div : 0;
         acc[i] = 0.0f;
     }
     for (int b = 0; b < g.nb; b++) {
@@ -897,7 +915,7 @@ __global__ __launch_bounds__(256) void k_grouped_q(GroupArgs g)
     }
 #pragma unroll
     for (int i = 0; i < A; i++)
-        if (i < tl.cnt) store_row(g, rgi, lane, g.perm[tl.start + i], acc[i]);
+        if (i < tl.cnt) store_row(g, rgi, lane, group_perm(g, tl.start + i), acc[i]);
 }
 
 // Q4_0 / Q8_0 rows of more than QG_SHORT blocks.  The tile's activation rows (integers, scales and, for
@@ -913,8 +931,8 @@ template <int TYPE, int A>
 __global__ __launch_bounds__(256) void k_grouped_q_ring(GroupArgs g)
 {
     const int tile = blockIdx.x;
-    if (tile >= *g.ntiles) return;  // uniform over the workgroup
-    const Tile tl = g.tiles[tile];
+    Tile tl;
+    if (!group_tile(g, tile, &tl)) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int rgi = blockIdx.y * 4 + wave;
     const bool live = rgi < g.rg;  // a wave past the last row group streams a clamped one, stores nothing
@@ -936,7 +954,7 @@ __global__ __launch_bounds__(256) void k_grouped_q_ring(GroupArgs g)
     float acc[A];
 #pragma unroll
     for (int i = 0; i < A; i++) {
-        arow[i] = g.perm[tl.start + min(i, cnt - 1)] / g.act_div;
+        arow[i] = group_perm(g, tl.start + min(i, cnt - 1)) / g.act_div;
         acc[i] = 0.0f;
     }
     unsigned char* myring = ringb + wave * (QG_R * SLOT);
@@ -1059,10 +1077,122 @@ __global__ __launch_bounds__(256) void k_grouped_q_ring(GroupArgs g)
 #pragma unroll
     for (int i = 0; i < A; i++)
         if (i < cnt) {  // uniform
-            const int64_t a = g.perm[tl.start + i];
+            const int64_t a = group_perm(g, tl.start + i);
             store_row(g, rgi, lane, a, acc[i]);
             if (g.req.q) requant_block(g, rgi, a, acc[i]);
         }
+}
+
+// Q4_0 / Q8_0 rows, the whole row at once: a workgroup takes one row group (lane = row) of one tile of up to
+// four assignments and wave w the eight blocks 8 w .. 8 w + 7 of a round (one scale group), every load of the
+// workgroup's weights in flight together while the assignments' integers are staged in LDS (read back as
+// wave-wide broadcasts).  The terms (float)isum * (d_w * d_x) meet in LDS, and wave i adds assignment i's in
+// block order: the reference's chain.  The walk of one wave over a row group's blocks that this replaces where
+// it is faster (launch_grouped) leaves a wave's latency per block and few waves.
+constexpr int GQ_W = 16;  // most waves (128 blocks per round)
+template <int TYPE>
+__global__ __launch_bounds__(64 * GQ_W) void k_grouped_q_wide(GroupArgs g)
+{
+    constexpr bool Q4 = TYPE == PHX_Q4_0_DEV;
+    constexpr int PAY = Q4 ? 16 : 32, NC = PAY / 16;
+    Tile tl;
+    if (!group_tile(g, blockIdx.x % g.mt, &tl)) return;  // uniform
+    const int rgi = blockIdx.x / g.mt, nb = g.nb, cnt = min(tl.cnt, g.amax);
+    const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, nw = nt >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ch = min(nb, 8 * nw);  // blocks per round
+    extern __shared__ __align__(16) unsigned char gq_smem[];
+    float* term = (float*)gq_smem;                          // [assignment][ch][64]
+    uint4* xs = (uint4*)(term + g.amax * ch * 64);          // [assignment][ch][2]
+    float2* xd = (float2*)(xs + g.amax * ch * 2);           // [assignment][ch]: scale, sum (bits of an int)
+    const uint8_t* rgp = g.payload + tl.e * g.mat_pay + rgi * g.rg_pay;
+    const uint8_t* wp = rgp + lane * PAY;
+    const uint8_t* sp = rgp + (int64_t)nb * 64 * PAY + lane * 16;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // wave w: assignments w, w + nw, ...
+    for (int r0 = 0; r0 < nb; r0 += ch) {
+        const int nbr = min(ch, nb - r0), b0 = r0 + 8 * wave;
+        uint4 w[8][NC];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {  // (past the row's end: its last block again)
+            const uint4* src = (const uint4*)(wp + (int64_t)min(b0 + j, nb - 1) * 64 * PAY);
+#pragma unroll
+            for (int c = 0; c < NC; c++) w[j][c] = src[c];
+        }
+        const uint4 sg = *(const uint4*)(sp + (int64_t)(min(b0, nb - 1) / 8) * 64 * 16);
+        if (r0) __syncthreads();  // the previous round's chains
+        for (int x = tid; x < cnt * nbr; x += nt) {
+            const int i = x / nbr, b = x - i * nbr;
+            const int64_t row = group_perm(g, tl.start + i) / g.act_div;
+            const u32x4_a4* src = (const u32x4_a4*)(g.act.q + row * g.act.qstride + (int64_t)(r0 + b) * 32);
+            const u32x4_a4 n0 = src[0], n1 = src[1];
+            const float d = g.d16 ? h2f(g.d16[row * nb + r0 + b]) : g.act.d[row * g.act.dstride + r0 + b];
+            xs[(i * ch + b) * 2] = make_uint4(n0.x, n0.y, n0.z, n0.w);
+            xs[(i * ch + b) * 2 + 1] = make_uint4(n1.x, n1.y, n1.z, n1.w);
+            int sm = 0;
+            if (Q4)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    sm = __builtin_amdgcn_sdot4((int)n0[k], 0x01010101, sm, false);
+                    sm = __builtin_amdgcn_sdot4((int)n1[k], 0x01010101, sm, false);
+                }
+            xd[i * ch + b] = make_float2(d, __int_as_float(8 * sm));
+        }
+        __syncthreads();
+        const uint32_t sgw[4] = {sg.x, sg.y, sg.z, sg.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (8 * wave + j >= nbr) break;  // uniform
+            const float dw = h2f((sgw[j / 2] >> (16 * (j & 1))) & 0xFFFFu);
+            uint32_t v[8];
+            if (Q4) {
+                const uint32_t p[4] = {w[j][0].x, w[j][0].y, w[j][0].z, w[j][0].w};
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    v[k] = p[k] & 0x0F0F0F0Fu;
+                    v[4 + k] = (p[k] >> 4) & 0x0F0F0F0Fu;
+                }
+            } else {
+                const uint4 a = w[j][0], b = w[j][NC - 1];
+                v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+                v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+            }
+            for (int i = 0; i < cnt; i++) {  // uniform
+                const int o = i * ch + 8 * wave + j;
+                const uint4 xa = xs[2 * o], xb = xs[2 * o + 1];
+                const float2 ds = xd[o];
+                const uint32_t x[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+                int s0 = 0, s1 = 0;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    s0 = __builtin_amdgcn_sdot4((int)v[k], (int)x[k], s0, false);
+                    s1 = __builtin_amdgcn_sdot4((int)v[4 + k], (int)x[4 + k], s1, false);
+                }
+                int isum = s0 + s1;
+                if (Q4) isum -= __float_as_int(ds.y);
+                const float dd = dw * ds.x;
+                term[o * 64 + lane] = (float)isum * dd;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int i = wave + q * nw;
+            if (i < cnt) {
+                const float* t = term + (int64_t)i * ch * 64 + lane;
+#pragma unroll 8
+                for (int b = 0; b < nbr; b++) acc[q] += t[b * 64];
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int i = wave + q * nw;
+        if (i < cnt) {  // uniform
+            const int64_t a = group_perm(g, tl.start + i);
+            store_row(g, rgi, lane, a, acc[q]);
+            if (g.req.q) requant_block(g, rgi, a, acc[q]);
+        }
+    }
 }
 
 // K-quant rows of a few assignments: DotK (src/CpuRefKQuants.cs:177-212) per (row, assignment): per
@@ -1075,7 +1205,6 @@ __global__ __launch_bounds__(256) void k_grouped_q_ring(GroupArgs g)
 // Scales times dot products are 24-bit products (v_mad_i32_i24; a 32-bit multiply issues at a quarter of the
 // rate).
 constexpr int GK_W = 16;  // most waves, and super-blocks staged at a time
-typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int TYPE>
 __host__ __device__ constexpr int gk_terms() { return TYPE == PHX_Q6_K_DEV ? 8 : 9; }  // eight lanes and the min term
 // LDS: term buffers (two where a tile can hold more than one assignment), the chains' values, then per
@@ -1093,12 +1222,7 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
     constexpr int PAY = Q4K ? 144 : Q5K ? 176 : 208, NT = gk_terms<TYPE>();
     const int tile = blockIdx.x % g.mt;
     Tile tl;
-    if (g.nident) {
-        tl = Tile{0, 4 * tile, min(4, g.nident - 4 * tile)};
-    } else {
-        if (tile >= *g.ntiles) return;  // uniform
-        tl = g.tiles[tile];
-    }
+    if (!group_tile(g, tile, &tl)) return;
     const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, nw = nt >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rgi = blockIdx.x / g.mt, nb = g.nb, cnt = min(tl.cnt, g.amax);
@@ -1112,7 +1236,7 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
     const uint8_t* wp = g.payload + tl.e * g.mat_pay + rgi * g.rg_pay + lane * 16;
     constexpr int SBY = AFF ? 4 : 2, BLK = 64 * (PAY + SBY);  // the rows' scales follow the block's chunks
     auto arow = [&](int i) -> int64_t {
-        return g.nident ? tl.start + i : g.perm[tl.start + i] / g.act_div;
+        return group_perm(g, tl.start + i) / g.act_div;
     };
     uint32_t wv[PAY / 4], dmw;
     auto load = [&](int r0) {  // this wave's super-block of the round (past the end: the last one again)
@@ -1246,7 +1370,7 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
         float s = AFF ? f[8 * 64] : 0.0f;
 #pragma unroll
         for (int l = 0; l < 8; l++) s += f[l * 64];
-        store_row(g, rgi, lane, g.nident ? tl.start + i : g.perm[tl.start + i], s);
+        store_row(g, rgi, lane, group_perm(g, tl.start + i), s);
     }
 }
 
@@ -1296,8 +1420,8 @@ __global__ __launch_bounds__(256) void k_grouped_iq(GroupArgs g)
     for (int i = threadIdx.x; i < NW; i += 256) cb[i] = ((const uint32_t*)g.grid)[i];
     __syncthreads();
     const int tile = blockIdx.x;
-    if (tile >= *g.ntiles) return;
-    const Tile tl = g.tiles[tile];
+    Tile tl;
+    if (!group_tile(g, tile, &tl)) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int rgi = blockIdx.y * 4 + wave;
     if (rgi >= g.rg) return;
@@ -1307,7 +1431,7 @@ __global__ __launch_bounds__(256) void k_grouped_iq(GroupArgs g)
     float sumf[A];
 #pragma unroll
     for (int i = 0; i < A; i++) {
-        arow[i] = i < tl.cnt ? g.perm[tl.start + i] / g.act_div : 0;
+        arow[i] = i < tl.cnt ? group_perm(g, tl.start + i) / g.act_div : 0;
         sumf[i] = 0.0f;
     }
     for (int b = 0; b < g.nb; b++) {
@@ -1382,7 +1506,7 @@ __global__ __launch_bounds__(256) void k_grouped_iq(GroupArgs g)
     }
 #pragma unroll
     for (int i = 0; i < A; i++)
-        if (i < tl.cnt) store_row(g, rgi, lane, g.perm[tl.start + i], IQ3 ? sumf[i] : 0.125f * sumf[i]);
+        if (i < tl.cnt) store_row(g, rgi, lane, group_perm(g, tl.start + i), IQ3 ? sumf[i] : 0.125f * sumf[i]);
 }
 
 // dynamic LDS of k_grouped_q_ring<type, 4>: the rings and one activation chunk, at least QG_LDS_MIN
@@ -1394,9 +1518,21 @@ static uint32_t grouped_q_lds(int type, int nb)
     return (uint32_t)std::max(need, QG_LDS_MIN);
 }
 
+template <int TYPE>
+static void launch_grouped_q_wide(hipStream_t st, GroupArgs g, int max_tiles)
+{
+    g.mt = max_tiles;
+    const int rounds = (g.nb + 8 * GQ_W - 1) / (8 * GQ_W), nw = ((g.nb + 7) / 8 + rounds - 1) / rounds;
+    const int ch = std::min(g.nb, 8 * nw), most = 4 * 8 * GQ_W * (256 + 40);
+    static_assert(4 * 8 * GQ_W * (256 + 40) <= 160 * 1024, "the widest launch fits a compute unit's LDS");
+    (void)hipFuncSetAttribute((const void*)k_grouped_q_wide<TYPE>, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    launch(k_grouped_q_wide<TYPE>, dim3((unsigned)max_tiles * (unsigned)g.rg), dim3(64 * nw),
+           (uint32_t)(g.amax * ch * (256 + 40)), st, g);
+}
+
 void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles, int A,
                     const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
-                    const Act* req, const float* gelu_tab, int req_rows, int nident, int amax)
+                    const Act* req, const float* gelu_tab, int req_rows, int nident, int amax, const uint16_t* d16)
 {
     GroupArgs g;
     g.payload = w.payload;
@@ -1420,9 +1556,14 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
     g.grid = w.grid;
     g.nident = nident;
     g.amax = std::min(amax, 4);
+    g.d16 = d16;
+    // Q4_0 / Q8_0: the whole-row kernel while a launch has few workgroups (a layer of 32 experts, d = 1024, T = 24:
+    // 60 us against 168 for the walks below; of 128 experts, d = 2816, about 3000 workgroups: 133 either way,
+    // and from 4000 the walks' several workgroups per compute unit are faster, 136 against 160)
+    const bool wide = w.has_sc8() && (d16 || (int64_t)max_tiles * w.rg <= 2048);
     // the down input in the ring kernel's epilogue where it covers every block of the row (paired Q4_0 /
     // Q8_0 rows past QG_SHORT blocks into Q8_0 rows with no padding blocks); else k_requant after it
-    const bool fuse = req && w.paired && w.nb > QG_SHORT && (w.type == PHX_Q4_0_DEV || w.type == PHX_Q8_0_DEV) &&
+    const bool fuse = req && w.paired && (wide || w.nb > QG_SHORT) && (w.type == PHX_Q4_0_DEV || w.type == PHX_Q8_0_DEV) &&
                       req->fmt == ACT_Q8_0 && req->cols == 32 * w.rg && split == 32 * w.rg && !req->qh;
     if (fuse) {
         g.req = *req;
@@ -1432,11 +1573,13 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
     (void)A;  // the tile size the dispatch used: 4, the one instantiation
     switch (w.type) {
     case PHX_Q4_0_DEV:
-        if (w.nb > QG_SHORT) launch((k_grouped_q_ring<PHX_Q4_0_DEV, 4>), grid, dim3(256), grouped_q_lds(w.type, w.nb), st, g);
+        if (wide) launch_grouped_q_wide<PHX_Q4_0_DEV>(st, g, max_tiles);
+        else if (w.nb > QG_SHORT) launch((k_grouped_q_ring<PHX_Q4_0_DEV, 4>), grid, dim3(256), grouped_q_lds(w.type, w.nb), st, g);
         else launch((k_grouped_q<PHX_Q4_0_DEV, 4>), grid, dim3(256), 0, st, g);
         break;
     case PHX_Q8_0_DEV:
-        if (w.nb > QG_SHORT) launch((k_grouped_q_ring<PHX_Q8_0_DEV, 4>), grid, dim3(256), grouped_q_lds(w.type, w.nb), st, g);
+        if (wide) launch_grouped_q_wide<PHX_Q8_0_DEV>(st, g, max_tiles);
+        else if (w.nb > QG_SHORT) launch((k_grouped_q_ring<PHX_Q8_0_DEV, 4>), grid, dim3(256), grouped_q_lds(w.type, w.nb), st, g);
         else launch((k_grouped_q<PHX_Q8_0_DEV, 4>), grid, dim3(256), 0, st, g);
         break;
     case PHX_Q4_K_DEV: launch_grouped_k<PHX_Q4_K_DEV>(st, g, max_tiles, 256); break;
@@ -1865,38 +2008,20 @@ void launch_stream_copy(hipStream_t st, void* dst, const void* src, int64_t byte
     launch(k_stream_copy, dim3(256 * 8), dim3(256), 0, st, (uint4*)dst, (const uint4*)src, bytes / 16);
 }
 
-// Planar Q8_0 rows (qs int8 [rows][n] and fp16 scale bits [rows][n/32], the layout phx_quant_q8_0
-// writes) into the grouped kernels' activation arrays: each block's scale as a float, the sum of its
-// integers (the Q4_0 offset term of the VALU kernels) and, when a.qh is set, the integers as exact
-// fp16 (the matrix-core operands).  An 8-lane group per block, four integers per lane.
+// Planar Q8_0 rows (qs int8 [rows][n] and fp16 scale bits [rows][n/32], the layout phx_quant_q8_0 writes) into
+// the matrix-core kernels' activation arrays: each block's scale as a float and the integers as exact fp16.
+// An 8-lane group per block, four integers per lane.
 __global__ __launch_bounds__(256) void k_planar_act(int64_t nblk, int nb, const int8_t* __restrict__ qs,
                                                     const uint16_t* __restrict__ d, Act a)
 {
     const int64_t g = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 3;
     const int l8 = threadIdx.x & 7;
-    const bool ok = g < nblk;
-    const int64_t gc = ok ? g : nblk - 1;  // every lane takes part in the group's shuffles
-    const uint32_t w = ((const uint32_t*)qs)[gc * 8 + l8];
-    const int q0 = (int8_t)(w & 0xFF), q1 = (int8_t)((w >> 8) & 0xFF), q2 = (int8_t)((w >> 16) & 0xFF),
-              q3 = (int8_t)(w >> 24);
-    int sm = q0 + q1 + q2 + q3;
-    sm += dpp_i<0xb1>(sm, sm);  // 8-lane sum: quad swaps, then the other quad (half-row mirror)
-    sm += dpp_i<0x4e>(sm, sm);
-    sm += dpp_i<0x141>(sm, sm);
-    if (!ok) return;
+    if (g >= nblk) return;
+    const uint32_t w = ((const uint32_t*)qs)[g * 8 + l8];
     const int64_t t = g / nb;
     const int b = (int)(g - t * nb);
-    if (l8 == 0) {
-        a.d[t * a.dstride + b] = h2f(d[g]);
-        a.s[t * a.sstride + b] = sm;
-    }
-    if (a.qh) {
-        const uint32_t h01 = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)q0) |
-                             ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)q1) << 16);
-        const uint32_t h23 = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)q2) |
-                             ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)q3) << 16);
-        *(uint2*)(a.qh + t * a.qhstride + b * 32 + 4 * l8) = make_uint2(h01, h23);
-    }
+    if (l8 == 0) a.d[t * a.dstride + b] = h2f(d[g]);
+    *(uint2*)(a.qh + t * a.qhstride + b * 32 + 4 * l8) = int_q4((int)w);
 }
 
 void launch_planar_act(hipStream_t st, int rows, int n, const int8_t* qs, const uint16_t* d, Act a)

@@ -46,6 +46,9 @@ struct MmaArgs {
     const int* ntiles;
     const int* perm;
     int act_div;
+    // ident > 0 (tiles, ntiles and perm unused): one matrix over the rows 0 .. ident - 1 in order, in tiles of
+    // identA
+    int ident, identA;
     float* out0;
     float* out1;
     int split, out_stride;
@@ -62,6 +65,20 @@ struct MmaArgs {
     int64_t qnpos;
     const float* gelu_tab;
 };
+
+// the workgroup's tile, false past the last one (uniform), and the assignment at list position p
+__device__ __forceinline__ bool mma_tile_of(const MmaArgs& g, int tile, Tile* tl)
+{
+    if (g.ident) {
+        const int t0 = tile * g.identA;
+        *tl = Tile{0, t0, min(g.identA, g.ident - t0)};
+        return t0 < g.ident;
+    }
+    if (tile >= *g.ntiles) return false;
+    *tl = g.tiles[tile];
+    return true;
+}
+__device__ __forceinline__ int mma_perm(const MmaArgs& g, int p) { return g.ident ? p : g.perm[p]; }
 
 constexpr int MMA_NT = 4;                 // 32-token column tiles per workgroup
 constexpr int MMA_TOK = 32 * MMA_NT;      // tile capacity (kMmaTile)
@@ -128,12 +145,12 @@ __device__ __forceinline__ void mma_tile(const MmaArgs& g, const Tile& tl, int c
     for (int i = 0; i < 2; i++) {
         const int t = min(32 * wave + 16 * i + (lane >> 2), cnt - 1);  // past cnt: a valid row, never stored
         const int q = (lane & 3) ^ ((lane >> 4) & 3);
-        const int64_t row = lst ? (int64_t)(tl.start + t) * 32 : (int64_t)(g.perm[tl.start + t] / g.act_div) * g.act.qhstride;
+        const int64_t row = lst ? (int64_t)(tl.start + t) * 32 : (int64_t)(mma_perm(g, tl.start + t) / g.act_div) * g.act.qhstride;
         vx[i] = (uint32_t)(2 * (row + 8 * q));
     }
     // (3) token scales of tokens 32 w + lane (lanes 0-31)
     const int td = min(32 * wave + r32, cnt - 1);
-    const uint32_t vds = (uint32_t)(4 * (lst ? (int64_t)tl.start + td : (int64_t)(g.perm[tl.start + td] / g.act_div) * g.act.dstride));
+    const uint32_t vds = (uint32_t)(4 * (lst ? (int64_t)tl.start + td : (int64_t)(mma_perm(g, tl.start + td) / g.act_div) * g.act.dstride));
     // (4) weight payload: Q4_0 rows 32 half + lane (lanes 0-31), Q8_0 row 32 half + lane / 2, half lane % 2;
     // (5) weight scales of rows 32 half + lane (lanes 0-31): fp16 at (b / 8, row) * 16 + (b % 8) * 2
     const int gIc = min(gI, g.rg - 1);
@@ -366,7 +383,7 @@ __device__ __forceinline__ void mma_tile(const MmaArgs& g, const Tile& tl, int c
     // hold the next index's load back)
     int pa[NJ];
 #pragma unroll
-    for (int j = 0; j < NJ; j++) pa[j] = g.perm[tl.start + min(32 * j + r32, cnt - 1)];
+    for (int j = 0; j < NJ; j++) pa[j] = mma_perm(g, tl.start + min(32 * j + r32, cnt - 1));
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int sidx = 32 * j + r32;
@@ -424,8 +441,8 @@ __global__ __launch_bounds__(256, 3) void k_grouped_mfma(MmaArgs g)
     __shared__ __align__(16) unsigned char ring[MmaSlot<TYPE>::LDS];
     int bx;
     const int tile = xcd_tile(&bx);
-    if (tile >= *g.ntiles) return;  // uniform over the workgroup
-    const Tile tl = g.tiles[tile];
+    Tile tl;
+    if (!mma_tile_of(g, tile, &tl)) return;  // uniform over the workgroup
     const int cnt = min(tl.cnt, MMA_TOK);
 #ifdef PHX_TIMELINE
     // start and end of each workgroup: entries 2 f, 2 f + 1 of f = tile * gridDim.x + row-group pair (down
@@ -498,7 +515,7 @@ __device__ __forceinline__ void coop_tile(const MmaArgs& g, const Tile& tl, int 
     for (int i = 0; i < 2; i++) {
         const int t = min(32 * wave + 16 * i + (lane >> 2), cnt - 1);  // past cnt: a valid row, never stored
         const int q = (lane & 3) ^ ((lane >> 4) & 3);
-        const int64_t row = lst ? (int64_t)(tl.start + t) * 32 : (int64_t)(g.perm[tl.start + t] / g.act_div) * g.act.qhstride;
+        const int64_t row = lst ? (int64_t)(tl.start + t) * 32 : (int64_t)(mma_perm(g, tl.start + t) / g.act_div) * g.act.qhstride;
         vx[i] = (uint32_t)(2 * (row + 8 * q));
     }
     const int gIc = min(gI, g.rg - 1);
@@ -726,7 +743,7 @@ __device__ __forceinline__ void coop_tile(const MmaArgs& g, const Tile& tl, int 
         // store, a store round takes its own by a lane shuffle (a load per round would wait behind the
         // previous round's stores)
         static_assert(NJ <= 4, "two indices per lane cover the tile");
-        const int pa0 = g.perm[tl.start + min(lane, cnt - 1)], pa1 = g.perm[tl.start + min(64 + lane, cnt - 1)];
+        const int pa0 = mma_perm(g, tl.start + min(lane, cnt - 1)), pa1 = mma_perm(g, tl.start + min(64 + lane, cnt - 1));
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
 #pragma unroll
@@ -768,7 +785,7 @@ __device__ __forceinline__ void coop_tile(const MmaArgs& g, const Tile& tl, int 
     }
     int pa[NJ];  // every index load before the first store
 #pragma unroll
-    for (int j = 0; j < NJ; j++) pa[j] = g.perm[tl.start + min(32 * j + r32, cnt - 1)];
+    for (int j = 0; j < NJ; j++) pa[j] = mma_perm(g, tl.start + min(32 * j + r32, cnt - 1));
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int sidx = 32 * j + r32;
@@ -812,8 +829,8 @@ __global__ __launch_bounds__(256, 2) void k_grouped_coop(MmaArgs g)
     __shared__ __align__(16) unsigned char ring[CoopSlot<TYPE>::LDS];
     int bx;
     const int tile = xcd_tile(&bx);
-    if (tile >= *g.ntiles) return;  // uniform over the workgroup
-    const Tile tl = g.tiles[tile];
+    Tile tl;
+    if (!mma_tile_of(g, tile, &tl)) return;  // uniform over the workgroup
     const int cnt = min(tl.cnt, MMA_TOK);
 #ifdef PHX_TIMELINE
     const int wgf = tile * gridDim.x + bx, tbase = g.paired ? 0 : 16384;  // as in k_grouped_mfma
@@ -832,7 +849,7 @@ __global__ __launch_bounds__(256, 2) void k_grouped_coop(MmaArgs g)
 
 void launch_grouped_mfma(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
                          const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
-                         int64_t npos, const Act* qout, int64_t qnpos, const float* gelu_tab)
+                         int64_t npos, const Act* qout, int64_t qnpos, const float* gelu_tab, int ident, int identA)
 {
     MmaArgs g;
     g.payload = w.payload;
@@ -849,6 +866,8 @@ void launch_grouped_mfma(hipStream_t st, const QMat& w, Act act, const Tile* til
     g.ntiles = ntiles;
     g.perm = perm;
     g.act_div = act_div;
+    g.ident = ident;
+    g.identA = identA;
     g.out0 = out0;
     g.out1 = out1;
     g.split = split;
@@ -958,7 +977,7 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
     // the direct loads' lane sources (assignments past cnt: a valid row, never stored), as buffer -> LDS
     // loads: each lane's byte offset (a VGPR, the same for every super-block) and the super-block's
     // uniform offset (an SGPR)
-    auto arow = [&](int t) -> int64_t { return g.perm[tl.start + min(t, cnt - 1)] / g.act_div; };
+    auto arow = [&](int t) -> int64_t { return mma_perm(g, tl.start + min(t, cnt - 1)) / g.act_div; };
     // (1)-(3) activation chunks: load i of wave w fills positions 64 (3 w + i) + lane of the
     // [chunk][assignment] array: chunk p / 48 of assignment p % 48
     uint32_t vx[3];
@@ -1275,7 +1294,7 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
     // before the first store
     int pa[NJ];
 #pragma unroll
-    for (int c = 0; c < NJ; c++) pa[c] = g.perm[tl.start + min(16 * c + r16, cnt - 1)];
+    for (int c = 0; c < NJ; c++) pa[c] = mma_perm(g, tl.start + min(16 * c + r16, cnt - 1));
 #pragma unroll
     for (int c = 0; c < NJ; c++) {
         const int t = 16 * c + r16;
@@ -1322,8 +1341,8 @@ __global__ __launch_bounds__(KM_NW * 64, 1) void k_grouped_kmma(MmaArgs g)
     // grid order (the XCD-aware order of the Q4_0 / Q8_0 kernel measured slower here: C4 gate|up
     // 227 -> 233 us, down 171 -> 175 us)
     const int bx = blockIdx.x, tile = blockIdx.y;
-    if (tile >= *g.ntiles) return;  // uniform over the workgroup
-    const Tile tl = g.tiles[tile];
+    Tile tl;
+    if (!mma_tile_of(g, tile, &tl)) return;  // uniform over the workgroup
     const int cnt = min(tl.cnt, KM_TOK);
     if (cnt > 32) kmma_tile<TYPE, 3, FOLD>(g, tl, cnt, kring, bx);
     else if (cnt > 16) kmma_tile<TYPE, 2, FOLD>(g, tl, cnt, kring, bx);
@@ -1331,7 +1350,8 @@ __global__ __launch_bounds__(KM_NW * 64, 1) void k_grouped_kmma(MmaArgs g)
 }
 
 void launch_grouped_kmma(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
-                         const int* perm, int act_div, float* out0, float* out1, int split, int out_stride)
+                         const int* perm, int act_div, float* out0, float* out1, int split, int out_stride, int ident,
+                         int identA)
 {
     MmaArgs g{};
     g.payload = w.payload;
@@ -1347,6 +1367,8 @@ void launch_grouped_kmma(hipStream_t st, const QMat& w, Act act, const Tile* til
     g.ntiles = ntiles;
     g.perm = perm;
     g.act_div = act_div;
+    g.ident = ident;
+    g.identA = identA;
     g.out0 = out0;
     g.out1 = out1;
     g.split = split;

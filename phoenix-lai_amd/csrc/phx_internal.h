@@ -163,12 +163,13 @@ void launch_topk(hipStream_t st, int T, int E, int k, int rule, const float* log
 void launch_dispatch(hipStream_t st, int n_assign, int E, int A, const int* ids, int* offsets, int* perm,
                      Tile* tiles, int* ntiles);
 // req: the paired gate|up product's down input (gelu(g) * u as Q8_0 rows, req_rows of them), formed in
-// the product's epilogue where it can be, else by k_requant after it.  nident > 0 (K-quant types, tiles and
-// perm unused): one matrix over nident rows in order.  amax: no tile of the call holds more assignments
+// the product's epilogue where it can be, else by k_requant after it.  nident > 0 (tiles and perm
+// unused): one matrix over nident rows in order.  amax: no tile of the call holds more assignments;
+// d16 (Q4_0 / Q8_0): the scales as planar fp16 bits [row][cols / 32] in place of act.d
 void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
                     int A, const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
                     const Act* req = nullptr, const float* gelu_tab = nullptr, int req_rows = 0, int nident = 0,
-                    int amax = 4);
+                    int amax = 4, const uint16_t* d16 = nullptr);
 void launch_requant(hipStream_t st, int rows, int nf, const float* g, const float* u, const float* gelu_tab, Act act);
 // standalone Q8_0 (fmt_k 0) / Q8_K (fmt_k 1) quantizer of rows x n inputs; mode as PHX_QUANT_*; -1 on a bad mode
 int launch_quant(hipStream_t st, int fmt_k, int mode, int rows, int n, float eps, const float* x, const float* aux,
@@ -186,17 +187,20 @@ void launch_matvec(hipStream_t st, int type, int rows, int nb, int T, const uint
 // scales at d[b * npos + p]).  For a paired gate|up matrix with qout set, the kernel also does the
 // GELU-gated requant into qout in that layout over qnpos positions (its qh and d only).  fold: the
 // tolerance mode (scales folded into fp16 operands, the row accumulated on the matrix cores).
+// ident > 0: one matrix over ident rows in order, in tiles of identA (<= kMmaTile; tiles, ntiles and perm
+// unused, max_tiles = ceil(ident / identA)); launch_grouped_kmma the same.
 constexpr int kMmaTile = 128;
 void launch_grouped_mfma(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
                          const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
                          int64_t npos = 0, const Act* qout = nullptr, int64_t qnpos = 0,
-                         const float* gelu_tab = nullptr);
+                         const float* gelu_tab = nullptr, int ident = 0, int identA = 0);
 // K-quant prefill path (kernels_prefill.hip): Q4_K / Q6_K grouped products on MFMA, tiles of up to
 // kKmmaTile assignments, activations' fp16 copies (qh; Q4_K also bh) in row order; arguments and outputs
 // as launch_grouped
 constexpr int kKmmaTile = 48;
 void launch_grouped_kmma(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
-                         const int* perm, int act_div, float* out0, float* out1, int split, int out_stride);
+                         const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
+                         int ident = 0, int identA = 0);
 void launch_combine(hipStream_t st, int T, int d, int k, float eps, const float* yd, const float* w,
                     const float* shared, const float* post1, const float* post2, float* out, float* x_resid,
                     const float* post_ffw, int* flags);

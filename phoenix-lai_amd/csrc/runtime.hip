@@ -521,8 +521,8 @@ struct CtxScope {
 enum WsId {
     W_X, W_SHARED, W_OUT, W_RIN, W_XSCALE, W_AGU_Q, W_AGU_D, W_AGU_S, W_ASH_Q, W_ASH_D, W_ASH_S, W_LOGITS, W_IDS, W_W,
     W_OFF, W_PERM, W_TILES, W_NTILES, W_G, W_U, W_ADN_Q, W_ADN_D, W_ADN_S, W_YD, W_SHG, W_SHU, W_ASD_Q, W_ASD_D,
-    W_ASD_S, W_SHOUT, W_ZERO, W_STILES, W_SNTILES, W_SOFF, W_SPERM, W_LB, W_BB, W_ADEC, W_SDEC, W_AGUP, W_ASHP, W_AGU_H, W_ADN_H, W_ASH_H, W_ASD_H, W_X2,
-    W_MM_IDS, W_MM_OFF, W_MM_PERM, W_MM_TILES, W_MM_NT, W_MM_D, W_MM_S, W_MM_H, W_AGU_BH, W_ADN_BH, W_MK_BH, W_KB,
+    W_ASD_S, W_SHOUT, W_LB, W_BB, W_ADEC, W_SDEC, W_AGUP, W_ASHP, W_AGU_H, W_ADN_H, W_ASH_H, W_ASD_H, W_X2,
+    W_MM_D, W_MM_H, W_AGU_BH, W_ADN_BH, W_MK_BH, W_KB,
     W_CBAD, W_RSCALE, W_COUNT
 };
 
@@ -546,7 +546,6 @@ int ensure(phx_moe_ctx* c, int id, size_t bytes)
     size_t n = std::max<size_t>(bytes, 256);
     HIPCHK(c, dev_malloc(c, &b.p, n));
     b.bytes = n;
-    if (id == W_ZERO) HIPCHK(c, hipMemset(b.p, 0, n));
     return PHX_OK;
 }
 
@@ -655,11 +654,6 @@ int ensure_workspace(phx_moe_ctx* c, const Layer& L, int T)
         ENS(W_SHG, (size_t)T * D.n_ff_shared * 4);
         ENS(W_SHU, (size_t)T * D.n_ff_shared * 4);
         ENS(W_SHOUT, (size_t)T * D.d * 4);
-        ENS(W_ZERO, (size_t)T * 4);
-        ENS(W_STILES, (size_t)((T + kTileA - 1) / kTileA + 1) * sizeof(Tile));
-        ENS(W_SNTILES, 4);
-        ENS(W_SOFF, 8);
-        ENS(W_SPERM, (size_t)T * 4);
     }
     ENS(W_TILES, (size_t)((n + 1) / 2 + D.n_expert) * sizeof(DecTile));
     ENS(W_ADEC, (size_t)n * (D.down_cols / 32) * 40);
@@ -870,6 +864,24 @@ bool keeps_gu(phx_moe_ctx* c, const Layer& L, int T, unsigned flags)
     return (flags & PHX_FLAG_KEEP_INTERMEDIATES) || use_decode(c, L, T, flags) || !mma_path(L.desc, T);
 }
 
+// Tiles of a single matrix's matrix-core product over T rows in order (row-group pairs x tiles workgroups).
+// Q4_0 / Q8_0: up to three workgroups share a compute unit, so tiles shrink while the launch has under two per
+// unit (2112 x 2816: T = 256 69 -> 37 us, T = 2048 92 -> 78 us with 64-row tiles; 32-row ones there 83).
+int ident_tile(int T, int pairs, int ncu)
+{
+    int A = kMmaTile;
+    while (A > 32 && (int64_t)((T + A - 1) / A) * pairs < 2 * ncu) A /= 2;
+    return A;
+}
+// K-quants: one workgroup fills a compute unit's LDS, so the smallest tile that keeps to one round (2816 x 2304
+// Q6_K, T = 300: 46 -> 39 us with 32-row tiles, 55 with 16-row ones in two rounds).
+int ident_tile_k(int T, int pairs, int ncu)
+{
+    int A = 16;
+    while (A < kKmmaTile && (int64_t)((T + A - 1) / A) * pairs > ncu) A += 16;
+    return A;
+}
+
 int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, const float* shared, float* out, float* xres,
                       bool exact, bool fast, bool keep)
 {
@@ -1033,10 +1045,9 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
     if (shared_ffn) {
         ProfScope p(c, PHX_K_SHARED);
         const int nff = D.n_ff_shared;
-        const int sA = smma ? kMmaTile : kTileA;
-        const int smax = (T + sA - 1) / sA + 1;
-        launch_dispatch(st, T, 1, sA, wp<int>(c, W_ZERO), wp<int>(c, W_SOFF), wp<int>(c, W_SPERM), wp<Tile>(c, W_STILES),
-                        wp<int>(c, W_SNTILES));
+        // one matrix over the tokens in order: tiles straight from the token numbers, no lists
+        const int sA = smma ? ident_tile(T, (L.sgu.rg + 1) / 2, c->ncu) : kTileA, smax = (T + sA - 1) / sA;
+        const int sB = smma ? ident_tile(T, (L.sdn.rg + 1) / 2, c->ncu) : kTileA, smaxb = (T + sB - 1) / sB;
         Act asd = make_act(c, act_fmt(D.shared_type), round_up(nff, block_elems(D.shared_type)), W_ASD_Q, W_ASD_D,
                            W_ASD_S);
         if (smma) {
@@ -1045,17 +1056,17 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             asd.fold = fast;
         }
         if (smma)
-            launch_grouped_mfma(st, L.sgu, ash, wp<Tile>(c, W_STILES), wp<int>(c, W_SNTILES), smax, wp<int>(c, W_SPERM), 1,
-                                nullptr, nullptr, nff, nff, 0, &asd, T, c->gelu_tab);  // (no reader of g, u)
+            launch_grouped_mfma(st, L.sgu, ash, nullptr, nullptr, smax, nullptr, 1, nullptr, nullptr, nff, nff, 0, &asd, T,
+                                c->gelu_tab, T, sA);  // (no reader of g, u)
         else
-            launch_grouped(st, L.sgu, ash, wp<Tile>(c, W_STILES), wp<int>(c, W_SNTILES), smax, kTileA, wp<int>(c, W_SPERM),
-                           1, wp<float>(c, W_SHG), wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T, 0, T);
+            launch_grouped(st, L.sgu, ash, nullptr, nullptr, smax, kTileA, nullptr, 1, wp<float>(c, W_SHG),
+                           wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T, T, T);
         if (smma)
-            launch_grouped_mfma(st, L.sdn, asd, wp<Tile>(c, W_STILES), wp<int>(c, W_SNTILES), smax, wp<int>(c, W_SPERM), 1,
-                                wp<float>(c, W_SHOUT), wp<float>(c, W_SHOUT), d, d, T);
+            launch_grouped_mfma(st, L.sdn, asd, nullptr, nullptr, smaxb, nullptr, 1, wp<float>(c, W_SHOUT),
+                                wp<float>(c, W_SHOUT), d, d, T, nullptr, 0, nullptr, T, sB);
         else
-            launch_grouped(st, L.sdn, asd, wp<Tile>(c, W_STILES), wp<int>(c, W_SNTILES), smax, kTileA, wp<int>(c, W_SPERM),
-                           1, wp<float>(c, W_SHOUT), wp<float>(c, W_SHOUT), d, d, nullptr, nullptr, 0, 0, T);
+            launch_grouped(st, L.sdn, asd, nullptr, nullptr, smaxb, kTileA, nullptr, 1, wp<float>(c, W_SHOUT),
+                           wp<float>(c, W_SHOUT), d, d, nullptr, nullptr, 0, T, T);
         sh = wp<float>(c, W_SHOUT);
     }
     {
@@ -1569,8 +1580,6 @@ int phx_moe_ffn_noalloc(phx_moe_ctx* c, int layer, int T, float* x, const float*
     const bool prof = c->profiling;  // the timers would create events
     c->profiling = false;
     if (rc == PHX_OK) {
-        // the shared FFN's one-expert ids must read zero; the array keeps the previous call's bytes
-        if (c->ws[W_ZERO].p) launch_fill_u32(c->stream, (uint32_t*)c->ws[W_ZERO].p, (int64_t)T, 0u);
         rc = run_layer(c, L, T, x, shared, out, (flags & PHX_FLAG_RESIDUAL) ? x : nullptr, flags);
     }
     c->profiling = prof;
@@ -2010,21 +2019,20 @@ int phx_matmul(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, con
         return set_err(c, PHX_ERR_ARG, "matmul: xq needs 4-byte, xd 2-byte, y 4-byte alignment");
     ENTER(c);
     const int nb = w->cols / 32;
-    // many tokens: the matrix cores on the integers as exact fp16; a few: the VALU row walk
-    const bool mma = T >= 32;
-    const int A = mma ? kMmaTile : kTileA;
+    // few rows, or few enough workgroups of four rows to run in about two per compute unit: the whole-row
+    // kernel on the caller's planar rows, one launch; else the matrix cores on the integers as exact fp16
+    // (2112 x 2816 Q4_0: T = 64 32 against 36 us, T = 96 41 against 36; 4224 x 4096: T = 31 44 against 51,
+    // T = 48 54 against 50)
+    const bool mma = T > 16 && (int64_t)((T + kTileA - 1) / kTileA) * w->q.rg > 9 * c->ncu / 4;
+    const int A = mma ? ident_tile(T, (w->q.rg + 1) / 2, c->ncu) : kTileA;
     const int max_tiles = (T + A - 1) / A;
     int rc;
 #define ENS(id, bytes) \
     if ((rc = ensure(c, id, (size_t)(bytes)))) return rc
-    ENS(W_MM_IDS, (size_t)T * 4);
-    ENS(W_MM_OFF, 8);
-    ENS(W_MM_PERM, (size_t)T * 4);
-    ENS(W_MM_TILES, (size_t)max_tiles * sizeof(Tile));
-    ENS(W_MM_NT, 4);
-    ENS(W_MM_D, (size_t)T * nb * 4);
-    ENS(W_MM_S, (size_t)T * nb * 4);
-    if (mma) ENS(W_MM_H, (size_t)T * w->cols * 2);
+    if (mma) {
+        ENS(W_MM_D, (size_t)T * nb * 4);
+        ENS(W_MM_H, (size_t)T * w->cols * 2);
+    }
 #undef ENS
     hipStream_t st = c->stream;
     Act a;
@@ -2032,25 +2040,20 @@ int phx_matmul(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, con
     a.cols = w->cols;
     a.q = (int8_t*)xq;
     a.qstride = w->cols;
-    a.d = wp<float>(c, W_MM_D);
-    a.dstride = nb;
-    a.s = wp<int>(c, W_MM_S);
-    a.sstride = nb;
     if (mma) {
+        a.d = wp<float>(c, W_MM_D);
+        a.dstride = nb;
         a.qh = wp<uint16_t>(c, W_MM_H);
         a.qhstride = w->cols;
     }
-    launch_planar_act(st, T, w->cols, xq, xd, a);
-    // every token is an assignment of the one matrix: the stable dispatch gives the identity list
-    launch_fill_u32(st, (uint32_t*)wp<int>(c, W_MM_IDS), T, 0u);
-    launch_dispatch(st, T, 1, A, wp<int>(c, W_MM_IDS), wp<int>(c, W_MM_OFF), wp<int>(c, W_MM_PERM),
-                    wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT));
+    if (mma) launch_planar_act(st, T, w->cols, xq, xd, a);
+    // one matrix over the tokens in order: tiles straight from the token numbers, no lists
     if (mma)
-        launch_grouped_mfma(st, w->q, a, wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT), max_tiles, wp<int>(c, W_MM_PERM), 1,
-                            y, y, w->rows, w->rows, 0, nullptr, 0, nullptr);
+        launch_grouped_mfma(st, w->q, a, nullptr, nullptr, max_tiles, nullptr, 1, y, y, w->rows, w->rows, 0, nullptr, 0,
+                            nullptr, T, A);
     else
-        launch_grouped(st, w->q, a, wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT), max_tiles, A, wp<int>(c, W_MM_PERM), 1,
-                       y, y, w->rows, w->rows);
+        launch_grouped(st, w->q, a, nullptr, nullptr, max_tiles, A, nullptr, 1, y, y, w->rows, w->rows, nullptr, nullptr, 0,
+                       T, T, xd);
     HIPCHK(c, launch_status(c));
     return PHX_OK;
 }
@@ -2069,7 +2072,7 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
     // the general path's rule with one matrix (at least 8 rows per matrix): the matrix cores, else the
     // VALU row walk
     const bool kmma = T >= 8 && kmma_type(w->type);
-    const int A = kmma ? kKmmaTile : kTileA;
+    const int A = kmma ? ident_tile_k(T, (w->q.rg + 1) / 2, c->ncu) : kTileA;
     const int max_tiles = (T + A - 1) / A;
     hipStream_t st = c->stream;
     int rc;
@@ -2089,11 +2092,6 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
     }
 #define ENS(id, bytes) \
     if ((rc = ensure(c, id, (size_t)(bytes)))) return rc
-    ENS(W_MM_IDS, (size_t)T * 4);
-    ENS(W_MM_OFF, 8);
-    ENS(W_MM_PERM, (size_t)T * 4);
-    ENS(W_MM_TILES, (size_t)max_tiles * sizeof(Tile));
-    ENS(W_MM_NT, 4);
     ENS(W_MM_D, (size_t)T * (cols / 256) * 4);
     ENS(W_MM_H, (size_t)T * cols * 2);
     if (w->type == PHX_Q4_K) ENS(W_MK_BH, (size_t)T * (cols / 16) * 2);
@@ -2110,11 +2108,7 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
         a.bhstride = cols / 16;
     }
     launch_planar_act_k(st, T, cols, xq, xd, a);
-    launch_fill_u32(st, (uint32_t*)wp<int>(c, W_MM_IDS), T, 0u);
-    launch_dispatch(st, T, 1, A, wp<int>(c, W_MM_IDS), wp<int>(c, W_MM_OFF), wp<int>(c, W_MM_PERM),
-                    wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT));
-    launch_grouped_kmma(st, w->q, a, wp<Tile>(c, W_MM_TILES), wp<int>(c, W_MM_NT), max_tiles, wp<int>(c, W_MM_PERM), 1, y,
-                        y, w->rows, w->rows);
+    launch_grouped_kmma(st, w->q, a, nullptr, nullptr, max_tiles, nullptr, 1, y, y, w->rows, w->rows, T, A);
     HIPCHK(c, launch_status(c));
     return PHX_OK;
 }
