@@ -380,7 +380,7 @@ struct phx_moe_ctx {
     hipStream_t stream = nullptr;
     // the general path's prologue runs on side beside the matrix-core router (fork and join events)
     hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_shared = nullptr;
     std::string err;
     float* gelu_tab = nullptr;
     std::vector<Layer> layers;
@@ -913,6 +913,46 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
         ash.qhstride = d;
         ash.fold = fast;
     }
+    // the shared FFN needs only its quantized input: it runs on the side stream beside the selection and the
+    // experts' products, which leave it compute units (77 tokens: 110 us of its own launches on 34 to 132
+    // workgroups), joined before the combine
+    auto shared_branch = [&]() {
+        hipStream_t st = c->side;
+        ProfScope p(c, PHX_K_SHARED);
+        const int nff = D.n_ff_shared;
+        // one matrix over the tokens in order: tiles straight from the token numbers, no lists
+        const int sA = smma ? ident_tile(T, (L.sgu.rg + 1) / 2, c->ncu) : kTileA, smax = (T + sA - 1) / sA;
+        const int sB = smma ? ident_tile(T, (L.sdn.rg + 1) / 2, c->ncu) : kTileA, smaxb = (T + sB - 1) / sB;
+        Act asd = make_act(c, act_fmt(D.shared_type), round_up(nff, block_elems(D.shared_type)), W_ASD_Q, W_ASD_D,
+                           W_ASD_S);
+        if (smma) {
+            asd.qh = wp<uint16_t>(c, W_ASD_H);
+            asd.qhstride = asd.cols;
+            asd.fold = fast;
+        }
+        if (smma)
+            launch_grouped_mfma(st, L.sgu, ash, nullptr, nullptr, smax, nullptr, 1, nullptr, nullptr, nff, nff, 0, &asd, T,
+                                c->gelu_tab, T, sA);  // (no reader of g, u)
+        else
+            launch_grouped(st, L.sgu, ash, nullptr, nullptr, smax, kTileA, nullptr, 1, wp<float>(c, W_SHG),
+                           wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T, T, T);
+        if (smma)
+            launch_grouped_mfma(st, L.sdn, asd, nullptr, nullptr, smaxb, nullptr, 1, wp<float>(c, W_SHOUT),
+                                wp<float>(c, W_SHOUT), d, d, T, nullptr, 0, nullptr, T, sB);
+        else
+            launch_grouped(st, L.sdn, asd, nullptr, nullptr, smaxb, kTileA, nullptr, 1, wp<float>(c, W_SHOUT),
+                           wp<float>(c, W_SHOUT), d, d, nullptr, nullptr, 0, T, T);
+    };
+    auto start_shared = [&](bool on_side) -> int {  // on_side: its input was written on the side stream
+        if (!shared_ffn) return PHX_OK;
+        if (!on_side) {
+            HIPCHK(c, hipEventRecord(c->ev_fork, st));
+            HIPCHK(c, hipStreamWaitEvent(c->side, c->ev_fork, 0));
+        }
+        shared_branch();
+        HIPCHK(c, hipEventRecord(c->ev_shared, c->side));
+        return PHX_OK;
+    };
     // the certified routers (decode-style workgroups per pair up to CERT_MAX_TE pairs, the matrix-core
     // one beyond), else the exact chains
     const bool cert = !exact && cert_route(L, T, shared_ffn);
@@ -928,6 +968,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             ProfScope p(c, PHX_K_ROUTER);
             launch_dec_route(st, h);
         }
+        if (int rc = start_shared(false)) return rc;
         {
             ProfScope p(c, PHX_K_TOPK);
             if (T == 1) {  // the selection writes the one token's lists too
@@ -955,7 +996,10 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             launch_prologue(sp, T, d, D.eps, x, L.gis, L.pre2, shared_ffn ? L.ffn_norm : nullptr,
                             rx ? nullptr : wp<float>(c, W_RIN), wp<float>(c, W_XSCALE), pgu, psh, c->flags);
         };
-        if (!mmr) prologue(st);
+        if (!mmr) {
+            prologue(st);
+            if (int rc = start_shared(false)) return rc;
+        }
         // up to 64 experts the router's waves hold all of a token's logits and take its top-k themselves
         const bool fused_topk = E <= 64;
         if (mmr) {
@@ -975,6 +1019,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             prologue(c->side);
             HIPCHK(c, hipEventRecord(c->ev_join, c->side));
             joined = true;
+            if (int rc = start_shared(true)) return rc;
             ProfScope p(c, PHX_K_TOPK);
             launch_cert_select(st, h);
         } else {
@@ -1041,34 +1086,8 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             launch_grouped(st, L.dn, adn, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, tileA, wp<int>(c, W_PERM),
                            1, wp<float>(c, W_YD), wp<float>(c, W_YD), d, d, nullptr, nullptr, 0, 0, T);
     }
-    const float* sh = shared;
-    if (shared_ffn) {
-        ProfScope p(c, PHX_K_SHARED);
-        const int nff = D.n_ff_shared;
-        // one matrix over the tokens in order: tiles straight from the token numbers, no lists
-        const int sA = smma ? ident_tile(T, (L.sgu.rg + 1) / 2, c->ncu) : kTileA, smax = (T + sA - 1) / sA;
-        const int sB = smma ? ident_tile(T, (L.sdn.rg + 1) / 2, c->ncu) : kTileA, smaxb = (T + sB - 1) / sB;
-        Act asd = make_act(c, act_fmt(D.shared_type), round_up(nff, block_elems(D.shared_type)), W_ASD_Q, W_ASD_D,
-                           W_ASD_S);
-        if (smma) {
-            asd.qh = wp<uint16_t>(c, W_ASD_H);
-            asd.qhstride = asd.cols;
-            asd.fold = fast;
-        }
-        if (smma)
-            launch_grouped_mfma(st, L.sgu, ash, nullptr, nullptr, smax, nullptr, 1, nullptr, nullptr, nff, nff, 0, &asd, T,
-                                c->gelu_tab, T, sA);  // (no reader of g, u)
-        else
-            launch_grouped(st, L.sgu, ash, nullptr, nullptr, smax, kTileA, nullptr, 1, wp<float>(c, W_SHG),
-                           wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T, T, T);
-        if (smma)
-            launch_grouped_mfma(st, L.sdn, asd, nullptr, nullptr, smaxb, nullptr, 1, wp<float>(c, W_SHOUT),
-                                wp<float>(c, W_SHOUT), d, d, T, nullptr, 0, nullptr, T, sB);
-        else
-            launch_grouped(st, L.sdn, asd, nullptr, nullptr, smaxb, kTileA, nullptr, 1, wp<float>(c, W_SHOUT),
-                           wp<float>(c, W_SHOUT), d, d, nullptr, nullptr, 0, T, T);
-        sh = wp<float>(c, W_SHOUT);
-    }
+    if (shared_ffn) HIPCHK(c, hipStreamWaitEvent(st, c->ev_shared, 0));  // the shared branch, before the combine
+    const float* sh = shared_ffn ? wp<float>(c, W_SHOUT) : shared;
     {
         ProfScope p(c, PHX_K_COMBINE);
         launch_combine(st, T, d, k, D.eps, wp<float>(c, W_YD), wp<float>(c, W_W), sh, L.post1, L.post2, out, xres,
@@ -1283,7 +1302,8 @@ int phx_moe_create(int hip_device, phx_moe_ctx** out)
         if ((h = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess ||
             (h = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking)) != hipSuccess ||
             (h = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming)) != hipSuccess ||
-            (h = hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming)) != hipSuccess) {
+            (h = hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming)) != hipSuccess ||
+            (h = hipEventCreateWithFlags(&c->ev_shared, hipEventDisableTiming)) != hipSuccess) {
             rc = set_err(c, hip_code(h), "hipStreamCreate failed");
             break;
         }
@@ -1331,6 +1351,7 @@ void phx_moe_destroy(phx_moe_ctx* c)
     if (c->iq_grid) (void)hipFree(c->iq_grid);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
+    if (c->ev_shared) (void)hipEventDestroy(c->ev_shared);
     if (c->side) (void)hipStreamDestroy(c->side);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
