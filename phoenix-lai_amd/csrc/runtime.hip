@@ -851,10 +851,21 @@ bool cert_route(const Layer& L, int T, bool shared_ffn)
 }
 
 // prefill-sized expert work (several assignments per expert on average) runs on the matrix cores, whose
-// kernels read the activations' fp16 copies
+// kernels read the activations' fp16 copies: from three per expert (128 experts of d = 2816, Q4_0: T = 32 145 us
+// on the VALU rows against 177, T = 48 192 against 188, T = 77 238 against 205, T = 127 317 against 207)
 static bool mma_path(const phx_moe_layer_desc& D, int T)
 {
-    return mfma_type(D.gate_up_type) && mfma_type(D.down_type) && T * D.n_used >= 8 * D.n_expert;
+    return mfma_type(D.gate_up_type) && mfma_type(D.down_type) && T * D.n_used >= 3 * D.n_expert;
+}
+
+// K-quants: from one per expert, unless the VALU rows' workgroups (a row group and a tile each) stay few
+// (64 experts of d = 4096: T = 4 82 us on the VALU rows against 101, T = 8 157 against 153, T = 16 257 against
+// 200, T = 64 442 against 325, T = 127 680 against 360)
+static bool kmma_path(const phx_moe_layer_desc& D, int T, int ncu)
+{
+    if (!kmma_type(D.gate_up_type) || !kmma_type(D.down_type)) return false;
+    const int n = T * D.n_used;
+    return n >= 8 * D.n_expert || (n >= D.n_expert && (int64_t)n * ((D.n_ff + 31) / 32) > 4 * ncu);
 }
 
 // whether a call stores the gate and up products for phx_moe_get_intermediates: the matrix-core Q4_0 /
@@ -891,7 +902,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
     const int n = T * k;
     const bool shared_ffn = shared == nullptr && D.n_ff_shared > 0;
     const bool mma = mma_path(D, T);
-    const bool kmma = kmma_type(D.gate_up_type) && kmma_type(D.down_type) && n >= 8 * E;
+    const bool kmma = kmma_path(D, T, c->ncu);
     const bool smma = shared_ffn && mfma_type(D.shared_type) && T >= 32;
     Act agu = make_act(c, act_fmt(D.gate_up_type), d, W_AGU_Q, W_AGU_D, W_AGU_S);
     if (mma || kmma) {

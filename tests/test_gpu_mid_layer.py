@@ -1,0 +1,74 @@
+"""Layers of a few assignments per expert, on both sides of the matrix cores' thresholds, and the shared FFN
+beside the experts (it runs on the context's second stream, joined before the combine).
+
+Q4_0 / Q8_0 products move to the matrix cores at three assignments per expert, K-quant ones at one where the
+row walk would take more than a few workgroups per compute unit; both are the reference's chains, so every
+stage equals the oracle bit for bit.  The stream test queues calls without waits, over two layers, several
+token counts and both routers, and replays a captured stack: every result equals the same call made alone."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import check_layer
+
+pytestmark = pytest.mark.gpu
+
+
+def say(s):
+    print(s, flush=True)
+
+
+CASES = {
+    "q4_0_below": (dict(idx=91, T=11, d=1024, E=8, k=2, nf=256, gu=2, dn=2, nff=288, sh=2), 11),
+    "q4_0_at": (dict(idx=92, T=12, d=1024, E=8, k=2, nf=256, gu=2, dn=2, nff=288, sh=2), 12),
+    "q8_0_at_shared_mfma": (dict(idx=93, T=36, d=512, E=24, k=2, nf=256, gu=8, dn=8, nff=256, sh=8), 36),
+    "q4k_q6k_few_workgroups": (dict(idx=94, T=8, d=512, E=8, k=2, nf=512, gu=12, dn=14), 8),
+    "q4k_q6k_matrix_cores": (dict(idx=95, T=20, d=512, E=8, k=2, nf=1024, gu=12, dn=14), 20),
+    "q6k_q4k_shared_q5k": (dict(idx=96, T=24, d=512, E=8, k=2, nf=1024, gu=14, dn=12, nff=512, sh=13), 24),
+}
+
+
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("case", list(CASES))
+def test_mid_sized_layers_match_oracle(ctx, pkg, orc, case, exact):
+    cfg, T = CASES[case]
+    say(f"mid layer {case} exact={exact}")
+    L = pkg.synth.make_layer(cfg, norms="random")
+    ctx.upload(0, L)
+    check_layer(ctx, orc, L, pkg.synth.make_input(cfg, T=T), tag=f"mid {case}", exact=exact)
+
+
+def test_shared_branch_stream_order(pkg):
+    say("shared FFN beside the experts: queued calls and a captured stack")
+    cfg = dict(idx=97, T=40, d=512, E=16, k=2, nf=256, gu=2, dn=2, nff=512, sh=2)
+    layers = pkg.synth.make_stack(cfg, 2)
+    P = pkg.PHX
+    with pkg.MoeContext(0) as c:
+        for i, L in enumerate(layers):
+            c.upload(i, L)
+        rng = np.random.default_rng(3)
+        Ts = [40, 700, 19, 130, 40, 513, 33]
+        xs = [rng.standard_normal((T, 512)).astype(np.float32) for T in Ts]
+        alone = [[c.ffn(i % 2, x, exact_router=e) for e in (False, True)] for i, x in enumerate(xs)]
+        xb, ob = [], []
+        for x in xs:
+            xb.append(c.alloc(x.nbytes))
+            xb[-1].upload(x)
+            ob.append([c.alloc(x.nbytes), c.alloc(x.nbytes)])
+        for _ in range(3):
+            for i, T in enumerate(Ts):
+                for e, flag in enumerate((0, P.FLAG_EXACT_ROUTER)):
+                    c.ffn_device(i % 2, T, xb[i].ptr, None, ob[i][e].ptr, flag | P.FLAG_ASYNC)
+        c.sync()
+        for i, x in enumerate(xs):
+            for e in range(2):
+                np.testing.assert_array_equal(ob[i][e].download(x.shape), alone[i][e], err_msg=f"call {i} exact={e}")
+        c.stack_capture(0, 2, 40)
+        first = c.stack_run(xs[0])
+        y = xs[0].copy()
+        for i in range(2):
+            _, y = c.ffn(i, y, residual=True)
+        np.testing.assert_array_equal(first, y)
+        for _ in range(3):
+            np.testing.assert_array_equal(c.stack_run(xs[0]), first)
+        for b in xb + [o for p in ob for o in p]:
+            b.free()
