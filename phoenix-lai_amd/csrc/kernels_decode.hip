@@ -2375,8 +2375,10 @@ void launch_router_mm(hipStream_t st, int T, int d, int E, float eps, const floa
                       float* xscale, double* Lb, double* Bb, uint32_t* kb, int* cbad, int* flags)
 {
     const RmArgs a{T, d, E, eps, x, Ws, Wn, xscale, Lb, Bb, (uint4*)kb, cbad, flags};
-    // 32 x 32 tiles where they still give a workgroup per compute unit, 16 x 16 below
-    if ((int64_t)((T + 31) / 32) * ((E + 31) / 32) >= 256) {
+    // 16 x 16 tiles while they run in two rounds over the compute units (a workgroup each), 32 x 32 above: one
+    // round of those takes what two rounds of the small ones do (128 experts, d = 2816: T = 1500, 188 large tiles
+    // or three rounds of small ones)
+    if ((int64_t)((T + 15) / 16) * ((E + 15) / 16) > 512) {
         using RG = RmLds<2, 2>;
         raise_lds(KRm<2, 2>::fn, RG::BYTES);
         launch(KRm<2, 2>::fn, dim3((T + 31) / 32, (E + 31) / 32), dim3(RM_NW * 64), (uint32_t)RG::BYTES, st, a);
