@@ -2276,6 +2276,8 @@ bool dec_supported(const DecLayerH& h)
     if (h.d > 4096 || h.d % 256 || h.gu->nb > DMAXNB || h.gu->nb > 32 * h.E || h.dn->nb > DMAXNB || h.E > 256 || h.T * h.k > 256) return false;
     if (h.sgu && (h.sgu->nb > DMAXNB || h.sdn->nb > DMAXNB)) return false;
     if (nt_gu(h) < std::max(h.E, h.T * h.k)) return false;  // build_tiles: a thread per expert and assignment
+    // a tile of two assignments needs a wave per chain: two waves per down row group (n_ff past 256)
+    if (h.T > 1 && waves_for(h.dn->nb) < DROWS) return false;
     return gu_lds(h) <= 160 * 1024 && down_lds(h) <= 160 * 1024;
 }
 
