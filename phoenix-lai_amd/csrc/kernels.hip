@@ -799,6 +799,9 @@ struct GroupArgs {
     float* out1;
     int split, out_stride;
     bool paired;
+    const float* gsrc = nullptr;    // k_grouped_k: set, its rows are the Q8_K of gelu(gsrc) * usrc ([row][snf], zeros
+    const float* usrc = nullptr;    // past snf), formed here, and act is unused
+    int snf = 0;
     const uint16_t* d16 = nullptr;  // k_grouped_q_wide: the scales as planar fp16 bits (act.d unused)
     int nident = 0;    // > 0 (tiles null): one matrix, tile i the rows 4 i .. 4 i + 3 of nident, in order
     int amax = 4;      // k_grouped_k, k_grouped_q_wide: assignments a tile can hold in this call (its LDS), and the most tiles
@@ -1208,11 +1211,13 @@ constexpr int GK_W = 16;  // most waves, and super-blocks staged at a time
 template <int TYPE>
 __host__ __device__ constexpr int gk_terms() { return TYPE == PHX_Q6_K_DEV ? 8 : 9; }  // eight lanes and the min term
 // LDS: term buffers (two where a tile can hold more than one assignment), the chains' values, then per
-// assignment and super-block the integers (64 dwords), the sums of 32 (8) and the scale
+// assignment and super-block the integers (64 dwords), the sums of 32 (8) and the scale, and where the rows are
+// formed here their integers in element order
 template <int TYPE>
-__host__ __device__ constexpr int gk_lds(int nw, int amax, int sg)
+__host__ __device__ constexpr int gk_lds(int nw, int amax, int sg, bool form)
 {
-    return (amax > 1 ? 2 : 1) * nw * gk_terms<TYPE>() * 256 + amax * gk_terms<TYPE>() * 256 + amax * sg * (256 + 32 + 4);
+    return (amax > 1 ? 2 : 1) * nw * gk_terms<TYPE>() * 256 + amax * gk_terms<TYPE>() * 256 +
+           amax * sg * (256 + 32 + 4 + (form ? 256 : 0));
 }
 template <int TYPE>
 __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
@@ -1233,6 +1238,7 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
     uint32_t* xs = (uint32_t*)(chain + g.amax * NT * 64);         // [assignment][super-block][64]
     int* xb = (int*)(xs + g.amax * sg * 64);                      // [assignment][super-block][8]
     float* xd = (float*)(xb + g.amax * sg * 8);                   // [assignment][super-block]
+    uint32_t* xn = (uint32_t*)(xd + g.amax * sg);                 // [assignment][super-block][64], rows formed here
     const uint8_t* wp = g.payload + tl.e * g.mat_pay + rgi * g.rg_pay + lane * 16;
     constexpr int SBY = AFF ? 4 : 2, BLK = 64 * (PAY + SBY);  // the rows' scales follow the block's chunks
     auto arow = [&](int i) -> int64_t {
@@ -1253,11 +1259,35 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
     // integers of super-blocks s0 .. s0 + n - 1: a thread per 32-element sub-block and round loads eight dwords
     // (elements 4 j .. 4 j + 3)
     auto stage = [&](int s0, int n) {
+        if (g.gsrc) {  // uniform; a wave per super-block (the values of k_requant)
+            for (int x = wave; x < cnt * n; x += nw) {
+                const int xi = x / n, sb = x - xi * n, col = (s0 + sb) * 256 + 4 * lane;
+                float4 e = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (col < g.snf) {
+                    const int64_t o = arow(xi) * g.snf + col;
+                    const float4 gv = *(const float4*)(g.gsrc + o), uv = *(const float4*)(g.usrc + o);
+                    e = make_float4(gelu_ref(gv.x, g.gelu_tab) * uv.x, gelu_ref(gv.y, g.gelu_tab) * uv.y,
+                                    gelu_ref(gv.z, g.gelu_tab) * uv.z, gelu_ref(gv.w, g.gelu_tab) * uv.w);
+                }
+                float dval;
+                xn[(xi * sg + sb) * 64 + lane] = q8_k_wave(e, &dval);
+                if (lane == 0) xd[xi * sg + sb] = dval;
+            }
+            __syncthreads();
+        }
         for (int x = tid; x < cnt * n * 8; x += nt) {
             const int xi = x / (n * 8), xr = x - xi * n * 8;
-            const u32x4_a4* src = (const u32x4_a4*)(g.act.q + arow(xi) * g.act.qstride + (int64_t)s0 * 256 + xr * 32);
-            const u32x4_a4 n0 = src[0], n1 = src[1];
-            if ((xr & 7) == 0) xd[xi * sg + (xr >> 3)] = g.act.d[arow(xi) * g.act.dstride + s0 + (xr >> 3)];
+            u32x4_a4 n0, n1;
+            if (g.gsrc) {
+                const u32x4_a4* src = (const u32x4_a4*)(xn + (xi * sg + (xr >> 3)) * 64 + (xr & 7) * 8);
+                n0 = src[0];
+                n1 = src[1];
+            } else {
+                const u32x4_a4* src = (const u32x4_a4*)(g.act.q + arow(xi) * g.act.qstride + (int64_t)s0 * 256 + xr * 32);
+                n0 = src[0];
+                n1 = src[1];
+            }
+            if (!g.gsrc && (xr & 7) == 0) xd[xi * sg + (xr >> 3)] = g.act.d[arow(xi) * g.act.dstride + s0 + (xr >> 3)];
             // 4 x 4 byte transposes: bytes l of dwords j, j + 2, j + 4, j + 6 (l = 4 j .. 4 j + 3)
             uint32_t* dst = xs + (xi * sg + (xr >> 3)) * 64 + (xr & 7) * 8;
 #pragma unroll
@@ -1386,10 +1416,10 @@ static void launch_grouped_k(hipStream_t st, GroupArgs g, int max_tiles, int ncu
     g.mt = max_tiles;
     const bool wide = (int64_t)max_tiles * g.rg <= ncu;
     const int rounds = wide ? (g.nb + GK_W - 1) / GK_W : (g.nb + 3) / 4, nw = (g.nb + rounds - 1) / rounds;
-    const int lds = gk_lds<TYPE>(nw, g.amax, std::min(g.nb, GK_W / nw * nw));
-    static_assert(gk_lds<TYPE>(GK_W, 4, GK_W) <= 160 * 1024, "the widest launch fits a compute unit's LDS");
+    const int lds = gk_lds<TYPE>(nw, g.amax, std::min(g.nb, GK_W / nw * nw), g.gsrc != nullptr);
+    static_assert(gk_lds<TYPE>(GK_W, 4, GK_W, true) <= 160 * 1024, "the widest launch fits a compute unit's LDS");
     (void)hipFuncSetAttribute((const void*)k_grouped_k<TYPE>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              gk_lds<TYPE>(GK_W, 4, GK_W));
+                              gk_lds<TYPE>(GK_W, 4, GK_W, true));
     launch(k_grouped_k<TYPE>, dim3((unsigned)max_tiles * (unsigned)g.rg), dim3(64 * nw), (uint32_t)lds, st, g);
 }
 
@@ -1532,7 +1562,7 @@ static void launch_grouped_q_wide(hipStream_t st, GroupArgs g, int max_tiles)
 
 void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles, int A,
                     const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
-                    const Act* req, const float* gelu_tab, int req_rows, int nident, int amax, const uint16_t* d16)
+                    const Act* req, const float* gelu_tab, int req_rows, int nident, int amax, const uint16_t* d16, const GeluRows* form)
 {
     GroupArgs g;
     g.payload = w.payload;
@@ -1557,6 +1587,12 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
     g.nident = nident;
     g.amax = std::min(amax, 4);
     g.d16 = d16;
+    if (form) {
+        g.gsrc = form->g;
+        g.usrc = form->u;
+        g.snf = form->nf;
+        g.gelu_tab = gelu_tab;
+    }
     // Q4_0 / Q8_0: the whole-row kernel while a launch has few workgroups (a layer of 32 experts, d = 1024, T = 24:
     // 60 us against 168 for the walks below; of 128 experts, d = 2816, about 3000 workgroups: 133 either way,
     // and from 4000 the walks' several workgroups per compute unit are faster, 136 against 160)
