@@ -914,8 +914,11 @@ void launch_grouped_mfma(hipStream_t st, const QMat& w, Act act, const Tile* til
 // Work layout: a workgroup of eight waves covers two row groups (wave w: rows 16 (w % 4) .. + 15 of
 // row group 2 x + w / 4) and one tile of up to 48 assignments (three 16-assignment column tiles).  Per
 // super-block its operands reach LDS by direct loads into a ring slot, RING - 1 super-blocks ahead: the
-// activation chunks chunk-major ([chunk][assignment][16 B]: the 16 lanes of an operand read one
-// 256-byte run), Q4_K block sums and token scales, each wave's 16 weight rows and their scales.  Each
+// activations assignment-major (a load's 64 lanes take two 512-byte runs of memory; chunk-major they took 64
+// runs of 16 bytes, whose cache lines held the kernel back: 64 experts, d = 4096, T = 512, the layer 471 ->
+// 436 us) with each assignment's 32 chunks XOR-swizzled by the assignment (the 16 lanes of an operand, 16
+// assignments' same chunk, hit 16 distinct bank groups), Q4_K block sums and token scales, each wave's 16 weight
+// rows and their scales.  Each
 // wave issues the same KM_DMA loads per super-block (some with lanes masked off), so its own count of
 // outstanding loads tells when a super-block has landed.
 constexpr int KM_TOK = 48;  // assignments per tile (kKmmaTile)
@@ -930,7 +933,7 @@ template <int TYPE>
 struct KmRing {
     static constexpr bool Q4K = TYPE == PHX_Q4_K_DEV;
     static constexpr int PAY = Q4K ? 144 : 208;
-    static constexpr int ACT_N = 32 * KM_TOK * 16;          // [32 chunks][48 assignments][16 B]
+    static constexpr int ACT_N = KM_TOK * 32 * 16;          // [48 assignments][32 chunks][16 B]
     static constexpr int BSM_N = Q4K ? 4 * KM_TOK * 8 : 0;  // Q4_K: [4 quarters][48][4 fp16 bsums]
     static constexpr int YD_N = KM_TOK * 4;                 // [48] token scales
     static constexpr int W_N = KM_NW * 16 * PAY;            // [8 waves][PAY / 16 chunks][16 rows][16 B]
@@ -978,13 +981,13 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
     // loads: each lane's byte offset (a VGPR, the same for every super-block) and the super-block's
     // uniform offset (an SGPR)
     auto arow = [&](int t) -> int64_t { return mma_perm(g, tl.start + min(t, cnt - 1)) / g.act_div; };
-    // (1)-(3) activation chunks: load i of wave w fills positions 64 (3 w + i) + lane of the
-    // [chunk][assignment] array: chunk p / 48 of assignment p % 48
+    // (1)-(3) activations: load i of wave w brings the 32 chunks of assignments 2 (3 w + i) and the next, 512
+    // consecutive bytes each, position p of assignment t holding chunk p ^ (t % 16)
     uint32_t vx[3];
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const int p = 64 * (3 * wave + i) + lane;
-        vx[i] = (uint32_t)(2 * (arow(p % KM_TOK) * g.act.qhstride + 8 * (p / KM_TOK)));
+        const int t = 2 * (3 * wave + i) + (lane >> 5);
+        vx[i] = (uint32_t)(2 * (arow(t) * g.act.qhstride + 8 * ((lane & 31) ^ (t & 15))));
     }
     // (4) Q4_K: dword 48 w + lane (lanes 0-47) of the block sums' [quarter][assignment][2 dwords]
     uint32_t vb = 0;
@@ -1054,7 +1057,9 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
     for (int c = 0; c < NJ; c++) acc[c] = zero4;
     // the lane's LDS read addresses in slot 0 of each region (slot S: + S * region slot bytes in the
     // immediate; the third activation slot from a second address, past the immediate's 64 KB)
-    const uint32_t a_act = ring0 + RG::ACT + q * (KM_TOK * 16) + r16 * 16, a_act2 = a_act + 2 * RG::ACT_N;
+    // (chunk 4 l + q of assignment 16 c + r16: position (4 l + q) ^ r16, so l's low bits flip address bits 6 and 7)
+    static_assert(RG::ACT == 0 && RG::ACT_N % 256 == 0, "the activation slots keep the swizzle's address bits");
+    const uint32_t p_act = RG::ACT + r16 * 512 + ((q ^ r16) & 15) * 16;
     const uint32_t a_bs = ring0 + RG::BSM + q * (KM_TOK * 8) + r16 * 8;
     const uint32_t a_yd = ring0 + RG::YD + r16 * 4;
     // the wave's weight rows sit chunk-major ([chunk][16 rows][16 B]): the 16 lanes of a read take 256
@@ -1066,12 +1071,15 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
     const uint32_t a_ws = ring0 + RG::WS + (wave * 16 + 4 * q) * 4;
     const uint32_t a_wr = ring0 + RG::WS + (wave * 16 + r16) * 4;  // FOLD: d (and dmin) of the A operand's row
     static_assert((RING - 1) * RG::W_N + 256 + 16 < 65536, "weight slots within the LDS immediate");
-    static_assert(RG::ACT_N + 8 * KM_TOK * 64 < 65536, "two activation slots within the LDS immediate");
-    // activation chunk reads of slot S at inner offset O
-    auto act_rd = [&](auto SC, auto OC) -> u32x4 {
-        constexpr int S = decltype(SC)::value, O = decltype(OC)::value;
-        if constexpr (S < 2) return ds_r128<S * RG::ACT_N + O>(a_act);
-        else return ds_r128<(S - 2) * RG::ACT_N + O>(a_act2);
+    static_assert(RG::ACT_N + KM_TOK * 512 < 65536, "two activation slots within the LDS immediate");
+    // the activation operand of lane l, column tile c in slot S: at the address act_at<l>(S) of its l
+    auto act_at = [&](auto SC, auto LC) -> uint32_t {
+        constexpr int S = decltype(SC)::value, l = decltype(LC)::value;
+        return ring0 + (p_act ^ (64 * (l & 3))) + (S == 2 ? 2 * RG::ACT_N : 0);
+    };
+    auto act_rd = [&](auto SC, auto LC, auto CC, uint32_t at) -> u32x4 {
+        constexpr int S = decltype(SC)::value, l = decltype(LC)::value, c = decltype(CC)::value;
+        return ds_r128<(S < 2 ? S : 0) * RG::ACT_N + 256 * (l >> 2) + 8192 * c>(at);
     };
 
     // super-block b in slot S
@@ -1099,16 +1107,17 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
         constexpr int OY = S * RG::YD_N, OB = S * RG::BSM_N;
         if (!FOLD) YD[0] = ds_r32<OY>(a_yd);
         if (Q4K && !FOLD) BS[0] = ds_r64<OB>(a_bs);
-        B[0][0] = act_rd(SC, ic<0>{});
+        const uint32_t at0 = act_at(SC, ic<0>{});
+        B[0][0] = act_rd(SC, ic<0>{}, ic<0>{}, at0);
         if (NJ > 1) {
             if (!FOLD) YD[1 % NJ] = ds_r32<OY + 64>(a_yd);
             if (Q4K && !FOLD) BS[1 % NJ] = ds_r64<OB + 128>(a_bs);
-            B[0][1 % NJ] = act_rd(SC, ic<256>{});
+            B[0][1 % NJ] = act_rd(SC, ic<0>{}, ic<1>{}, at0);
         }
         if (NJ > 2) {
             if (!FOLD) YD[2 % NJ] = ds_r32<OY + 128>(a_yd);
             if (Q4K && !FOLD) BS[2 % NJ] = ds_r64<OB + 256>(a_bs);
-            B[0][2 % NJ] = act_rd(SC, ic<512>{});
+            B[0][2 % NJ] = act_rd(SC, ic<0>{}, ic<2>{}, at0);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         tie(D0);
@@ -1231,9 +1240,11 @@ __device__ __forceinline__ void kmma_tile(const MmaArgs& g, const Tile& tl, int 
         auto step = [&](auto LC) {
             constexpr int l = decltype(LC)::value, cur = l & 1;
             if (l + 1 < 8) {
-                B[cur ^ 1][0] = act_rd(SC, ic<(l + 1) * KM_TOK * 64>{});
-                if (NJ > 1) B[cur ^ 1][1 % NJ] = act_rd(SC, ic<(l + 1) * KM_TOK * 64 + 256>{});
-                if (NJ > 2) B[cur ^ 1][2 % NJ] = act_rd(SC, ic<(l + 1) * KM_TOK * 64 + 512>{});
+                constexpr int n = (l + 1) % 8;
+                const uint32_t at = act_at(SC, ic<n>{});
+                B[cur ^ 1][0] = act_rd(SC, ic<n>{}, ic<0>{}, at);
+                if (NJ > 1) B[cur ^ 1][1 % NJ] = act_rd(SC, ic<n>{}, ic<1>{}, at);
+                if (NJ > 2) B[cur ^ 1][2 % NJ] = act_rd(SC, ic<n>{}, ic<2>{}, at);
             }
             mh8 A, A2;
             a_op(l, A, A2);
