@@ -122,7 +122,126 @@ __device__ __forceinline__ uint32_t act_off(int t, int q)
     return (uint32_t)((t >> 4) * 1024 + (tl * 4 + (q ^ (tl >> 2))) * 16);
 }
 
-// One workgroup's tile: NJ active 32-token column tiles (1..4).  ring: the workgroup's LDS ring.
+// The end of a tile: the GELU-gated requant of a paired launch, then the fp32 results.  S: the wave's 32 rows (half
+// of row group gI) by NJ 32-token columns.
+template <int NJ>
+__device__ __forceinline__ void mma_finish(const MmaArgs& g, const Tile& tl, int cnt, unsigned char* ring, const mf16 (&S)[NJ],
+                                           int gI, int half, bool live)
+{
+    const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (g.qout.qh) {  // uniform: the requant epilogue (src/GemmaCpu.cs:415, src/CpuRef.cs:49-62)
+        // the gate wave of each pair (half 0) forms gelu(g) (src/CpuRefGemma.cs:85-92: the table lookups
+        // of all its values issued together) and hands it to the up wave through the ring
+        __syncthreads();  // every wave is done with the ring
+        float* xg = (float*)ring + (wave >> 1) * (MMA_NT * 16 * 64);
+        if (half == 0) {
+            float tv[NJ][16];
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int q = 0; q < 16; q++) tv[j][q] = g.gelu_tab[f2h_bits(S[j][q])];
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int q = 0; q < 16; q++) {
+                    const float v = S[j][q];
+                    xg[(j * 16 + q) * 64 + lane] = v <= -10.0f ? 0.0f : (v >= 10.0f ? v : tv[j][q]);
+                }
+        }
+        __syncthreads();
+        if (half == 1 && live) {
+            const Act& o = g.qout;
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                // lane (r32, h): token column r32 of tile j, block columns 8 (q / 4) + 4 h + q % 4
+                float e[16], am = 0.0f;
+#pragma unroll
+                for (int q = 0; q < 16; q++) {
+                    const int col = gI * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
+                    e[q] = col < g.split ? xg[(j * 16 + q) * 64 + lane] * S[j][q] : 0.0f;
+                    am = fmaxf(am, fabsf(e[q]));
+                }
+                am = fmaxf(am, __shfl_xor(am, 32, 64));  // the other 16 columns: lane r32 + 32 (1 - 2 h)
+                const float dd = am / 127.0f;
+                const float id = dd != 0.0f ? 1.0f / dd : 0.0f;
+                // the integers as exact fp16 (signed bytes through the 1152 bias), four per column group
+                uint32_t w[4][2];
+#pragma unroll
+                for (int g4 = 0; g4 < 4; g4++) {
+                    const int q0 = (int)roundf(e[4 * g4] * id), q1 = (int)roundf(e[4 * g4 + 1] * id),
+                              q2 = (int)roundf(e[4 * g4 + 2] * id), q3 = (int)roundf(e[4 * g4 + 3] * id);
+                    const uint32_t u = (uint32_t)((q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) |
+                                                  ((unsigned)q3 << 24)) ^ 0x80808080u;
+                    w[g4][0] = bias_pair(u, 0, 1152.0f);
+                    w[g4][1] = bias_pair(u, 1, 1152.0f);
+                }
+                // this lane writes columns 16 h .. 16 h + 15: groups 2 h and 2 h + 1 of both halves (the
+                // partner lane's half from it)
+                const uint32_t s0 = h ? w[0][0] : w[2][0], s1 = h ? w[0][1] : w[2][1];
+                const uint32_t s2 = h ? w[1][0] : w[3][0], s3 = h ? w[1][1] : w[3][1];
+                const uint32_t p0 = (uint32_t)__shfl_xor((int)s0, 32, 64), p1 = (uint32_t)__shfl_xor((int)s1, 32, 64);
+                const uint32_t p2 = (uint32_t)__shfl_xor((int)s2, 32, 64), p3 = (uint32_t)__shfl_xor((int)s3, 32, 64);
+                const uint4 lo = h ? make_uint4(p0, p1, w[2][0], w[2][1]) : make_uint4(w[0][0], w[0][1], p0, p1);
+                const uint4 hi = h ? make_uint4(p2, p3, w[3][0], w[3][1]) : make_uint4(w[1][0], w[1][1], p2, p3);
+                const int sidx = 32 * j + r32;
+                if (sidx < cnt) {
+                    const int64_t pos = (int64_t)gI * g.qnpos + tl.start + sidx;
+                    uint16_t* hq = o.qh + pos * 32 + 16 * h;
+                    *(uint4*)hq = lo;
+                    *(uint4*)(hq + 8) = hi;
+                    if (h == 0) o.d[pos] = h2f(f2h_bits(dd));
+                }
+            }
+        }
+    }
+
+    // results: lane holds rows i_q = 8 (q / 4) + 4 h + (q % 4) of the wave's 32, token column r32 (a
+    // paired launch without g and u outputs ends with its requant)
+    if (!live || (g.paired && !g.out0)) return;
+    // the lane's assignment indices, every load before the first store (a store's wait would otherwise
+    // hold the next index's load back)
+    int pa[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) pa[j] = mma_perm(g, tl.start + min(32 * j + r32, cnt - 1));
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int sidx = 32 * j + r32;
+        if (sidx >= cnt) continue;
+        const int64_t a = pa[j];
+        // four consecutive rows (columns of the output row a) per q4: one 16-byte store where the four
+        // lie inside the output and the row stride keeps them aligned, else element by element
+        const bool vec = (g.out_stride & 3) == 0;
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) {
+            const int lg0 = half * 32 + 8 * q4 + 4 * h;  // lane within the row group of the first of four
+            const float4 v = make_float4(S[j][4 * q4], S[j][4 * q4 + 1], S[j][4 * q4 + 2], S[j][4 * q4 + 3]);
+            if (g.paired) {
+                const int col = gI * 32 + (lg0 & 31);
+                float* dst = (half ? g.out1 : g.out0) + a * g.out_stride + col;
+                if (vec && col + 3 < g.split) *(float4*)dst = v;
+                else
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (col + i < g.split) dst[i] = S[j][4 * q4 + i];
+            } else {
+                const int row = gI * 64 + lg0;
+                if (vec && row + 3 < min(g.rows, g.split)) *(float4*)(g.out0 + a * g.out_stride + row) = v;
+                else
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int r = row + i;
+                        if (r < g.rows) {
+                            if (r < g.split) g.out0[a * g.out_stride + r] = S[j][4 * q4 + i];
+                            else g.out1[a * g.out_stride + r - g.split] = S[j][4 * q4 + i];
+                        }
+                    }
+            }
+        }
+    }
+}
+
+// One workgroup's tile: NJ active 32-token column tiles (2..4).  ring: the workgroup's LDS ring.
 template <int TYPE, int NJ>
 __device__ __forceinline__ void mma_tile(const MmaArgs& g, const Tile& tl, int cnt, unsigned char* ring, int bx)
 {
@@ -310,115 +429,180 @@ __device__ __forceinline__ void mma_tile(const MmaArgs& g, const Tile& tl, int c
     // the loads issued past the last block land in this workgroup's LDS: let them finish before it ends
     __builtin_amdgcn_s_waitcnt(0);
 
-    if (g.qout.qh) {  // uniform: the requant epilogue (src/GemmaCpu.cs:415, src/CpuRef.cs:49-62)
-        // the gate wave of each pair (half 0) forms gelu(g) (src/CpuRefGemma.cs:85-92: the table lookups
-        // of all its values issued together) and hands it to the up wave through the ring
-        __syncthreads();  // every wave is done with the ring
-        float* xg = (float*)ring + (wave >> 1) * (MMA_NT * 16 * 64);
-        if (half == 0) {
-            float tv[NJ][16];
-#pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int q = 0; q < 16; q++) tv[j][q] = g.gelu_tab[f2h_bits(S[j][q])];
-#pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int q = 0; q < 16; q++) {
-                    const float v = S[j][q];
-                    xg[(j * 16 + q) * 64 + lane] = v <= -10.0f ? 0.0f : (v >= 10.0f ? v : tv[j][q]);
-                }
-        }
-        __syncthreads();
-        if (half == 1 && live) {
-            const Act& o = g.qout;
-#pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                // lane (r32, h): token column r32 of tile j, block columns 8 (q / 4) + 4 h + q % 4
-                float e[16], am = 0.0f;
-#pragma unroll
-                for (int q = 0; q < 16; q++) {
-                    const int col = gI * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-                    e[q] = col < g.split ? xg[(j * 16 + q) * 64 + lane] * S[j][q] : 0.0f;
-                    am = fmaxf(am, fabsf(e[q]));
-                }
-                am = fmaxf(am, __shfl_xor(am, 32, 64));  // the other 16 columns: lane r32 + 32 (1 - 2 h)
-                const float dd = am / 127.0f;
-                const float id = dd != 0.0f ? 1.0f / dd : 0.0f;
-                // the integers as exact fp16 (signed bytes through the 1152 bias), four per column group
-                uint32_t w[4][2];
-#pragma unroll
-                for (int g4 = 0; g4 < 4; g4++) {
-                    const int q0 = (int)roundf(e[4 * g4] * id), q1 = (int)roundf(e[4 * g4 + 1] * id),
-                              q2 = (int)roundf(e[4 * g4 + 2] * id), q3 = (int)roundf(e[4 * g4 + 3] * id);
-                    const uint32_t u = (uint32_t)((q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) |
-                                                  ((unsigned)q3 << 24)) ^ 0x80808080u;
-                    w[g4][0] = bias_pair(u, 0, 1152.0f);
-                    w[g4][1] = bias_pair(u, 1, 1152.0f);
-                }
-                // this lane writes columns 16 h .. 16 h + 15: groups 2 h and 2 h + 1 of both halves (the
-                // partner lane's half from it)
-                const uint32_t s0 = h ? w[0][0] : w[2][0], s1 = h ? w[0][1] : w[2][1];
-                const uint32_t s2 = h ? w[1][0] : w[3][0], s3 = h ? w[1][1] : w[3][1];
-                const uint32_t p0 = (uint32_t)__shfl_xor((int)s0, 32, 64), p1 = (uint32_t)__shfl_xor((int)s1, 32, 64);
-                const uint32_t p2 = (uint32_t)__shfl_xor((int)s2, 32, 64), p3 = (uint32_t)__shfl_xor((int)s3, 32, 64);
-                const uint4 lo = h ? make_uint4(p0, p1, w[2][0], w[2][1]) : make_uint4(w[0][0], w[0][1], p0, p1);
-                const uint4 hi = h ? make_uint4(p2, p3, w[3][0], w[3][1]) : make_uint4(w[1][0], w[1][1], p2, p3);
-                const int sidx = 32 * j + r32;
-                if (sidx < cnt) {
-                    const int64_t pos = (int64_t)gI * g.qnpos + tl.start + sidx;
-                    uint16_t* hq = o.qh + pos * 32 + 16 * h;
-                    *(uint4*)hq = lo;
-                    *(uint4*)(hq + 8) = hi;
-                    if (h == 0) o.d[pos] = h2f(f2h_bits(dd));
-                }
-            }
-        }
-    }
+    mma_finish<NJ>(g, tl, cnt, ring, S, gI, half, live);
+}
 
-    // results: lane holds rows i_q = 8 (q / 4) + 4 h + (q % 4) of the wave's 32, token column r32 (a
-    // paired launch without g and u outputs ends with its requant)
-    if (!live || (g.paired && !g.out0)) return;
-    // the lane's assignment indices, every load before the first store (a store's wait would otherwise
-    // hold the next index's load back)
-    int pa[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) pa[j] = mma_perm(g, tl.start + min(32 * j + r32, cnt - 1));
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int sidx = 32 * j + r32;
-        if (sidx >= cnt) continue;
-        const int64_t a = pa[j];
-        // four consecutive rows (columns of the output row a) per q4: one 16-byte store where the four
-        // lie inside the output and the row stride keeps them aligned, else element by element
-        const bool vec = (g.out_stride & 3) == 0;
-#pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-            const int lg0 = half * 32 + 8 * q4 + 4 * h;  // lane within the row group of the first of four
-            const float4 v = make_float4(S[j][4 * q4], S[j][4 * q4 + 1], S[j][4 * q4 + 2], S[j][4 * q4 + 3]);
-            if (g.paired) {
-                const int col = gI * 32 + (lg0 & 31);
-                float* dst = (half ? g.out1 : g.out0) + a * g.out_stride + col;
-                if (vec && col + 3 < g.split) *(float4*)dst = v;
-                else
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        if (col + i < g.split) dst[i] = S[j][4 * q4 + i];
-            } else {
-                const int row = gI * 64 + lg0;
-                if (vec && row + 3 < min(g.rows, g.split)) *(float4*)(g.out0 + a * g.out_stride + row) = v;
-                else
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int r = row + i;
-                        if (r < g.rows) {
-                            if (r < g.split) g.out0[a * g.out_stride + r] = S[j][4 * q4 + i];
-                            else g.out1[a * g.out_stride + r - g.split] = S[j][4 * q4 + i];
-                        }
-                    }
-            }
+// A tile of one 32-token column (few assignments per expert, or few rows): the weights' stream bounds it, so its
+// ring holds only 32 tokens and steps of two blocks: three direct loads per wave and step (five for
+// Q8_0) where mma_tile issues eight (ten), and the LDS of three workgroups per CU keeps eight (Q8_0: six)
+// blocks ahead in flight instead of three.  77 tokens, 8 of 128 experts, 704 x 2816 Q4_0: gate|up 131 -> 112 us
+// beside the shared FFN, down 57 -> 51, the layer 225 -> 205 us (2048 tokens, whose tiles' remainders come here:
+// 563 -> 553 us).
+//   activations [32 tokens][8 parts of 16 B]: parts 0-3 the step's first block, 4-7 its second, part p at
+//   position p ^ small_swz(token) (an operand read's 16 lanes hit 16 distinct bank groups); token scales
+//   [2 blocks][32]; payload per wave [2 blocks][32 rows][PAY]; weight scales in the scale ring of mma_tile (Q4_0),
+//   or the step's two per row, 4 bytes, in the slot (Q8_0, whose scale ring would take the third workgroup).
+// A row of an odd number of blocks ends with the step (nb - 2, nb - 1), of which only the second block is new; a
+// row of one block takes it as both.
+template <int TYPE>
+struct MmaSmall {
+    static constexpr int PAY = TYPE == PHX_Q4_0_DEV ? 16 : 32;
+    static constexpr bool SG = PAY == 16;
+    static constexpr int DMA = SG ? 3 : 5;                 // direct loads per wave per step (scale groups aside)
+    static constexpr int RING = PAY == 16 ? 5 : 4;         // steps; the scale ring allows at most eight blocks ahead
+    static constexpr int ACT = 0, ADX = ACT + 4096, WQ = ADX + 256;
+    static constexpr int WD = WQ + 4 * 64 * PAY;           // (Q8_0) per wave [32 rows][2 fp16]
+    static constexpr int BYTES = WD + (SG ? 0 : 4 * 128);
+    static constexpr int SR = RING * BYTES;                // (Q4_0) scale ring: [2 groups][4 waves][32 rows][8 fp16]
+    static constexpr int LDS = SR + (SG ? 2 * 4 * 512 : 0);
+    static_assert(2 * (RING - 1) <= 8 && LDS <= 42 * 1280, "three workgroups per CU (LDS comes in 1280-byte units); a scale group's slot is refilled only after its last block");
+    static_assert(RING * BYTES < 65536, "ring offsets fit the LDS immediate");
+};
+__device__ __forceinline__ int small_swz(int t) { return (t ^ (t >> 3)) & 7; }
+
+template <int TYPE>
+__device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int cnt, unsigned char* ring, int bx)
+{
+    using SL = MmaSmall<TYPE>;
+    constexpr int PAY = SL::PAY, RING = SL::RING;
+    const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gI = bx * 2 + (wave >> 1), half = wave & 1;
+    const bool live = gI < g.rg;  // a wave past the last row group computes a clamped one, stores nothing
+    const int nb = g.nb;
+    const uint32_t ring0 = (uint32_t)(uintptr_t)(lds_void_t)ring;
+    const bool lst = g.npos > 0;
+    const uint32_t xstep = lst ? (uint32_t)g.npos * 64u : 64u, dstep = lst ? (uint32_t)g.npos * 4u : 4u;  // bytes per block
+    const uint32_t two = nb > 1 ? 1u : 0u;  // the second block's offset (a row of one block: the same again)
+    auto arow = [&](int t) -> int64_t {     // past cnt: a valid row, never stored
+        const int p = tl.start + min(t, cnt - 1);
+        return lst ? (int64_t)p : (int64_t)(mma_perm(g, p) / g.act_div);
+    };
+    // (1) activations of tokens 8 w + lane / 8
+    const int ta = 8 * wave + (lane >> 3), pa_ = (lane & 7) ^ small_swz(ta);
+    const uint32_t vx = (uint32_t)(2 * arow(ta) * (lst ? 32 : g.act.qhstride)) + 16u * (pa_ & 3) + (pa_ >> 2) * two * xstep;
+    // (2) token scales: lanes 16 w .. 16 w + 15 of [2 blocks][32 tokens]
+    const uint32_t vd = (uint32_t)(4 * arow(r32) * (lst ? 1 : g.act.dstride)) + h * two * dstep;
+    // (3) payload: Q4_0 rows 32 half + r32 of both blocks, Q8_0 row 32 half + lane / 2, half lane % 2, of one block
+    // per load
+    const int gIc = min(gI, g.rg - 1);
+    const __amdgpu_buffer_rsrc_t r_act = buf_rsrc(g.act.qh), r_ds = buf_rsrc(g.act.d);
+    const __amdgpu_buffer_rsrc_t r_w = buf_rsrc(g.payload + tl.e * g.mat_pay + gIc * g.rg_pay);
+    const uint32_t vw = PAY == 16 ? (32 * half + r32) * 16 + h * two * 1024
+                                  : (32 * half + (lane >> 1)) * 32 + 16 * (lane & 1);
+    const uint32_t vsg = (uint32_t)g.sc_off + (32 * half + r32) * 16;
+
+    auto issue = [&](auto SC, int b) {  // the step from block b (even) into slot S
+        constexpr int S = decltype(SC)::value;
+        const uint32_t bc = (uint32_t)min(b, max(nb - 2, 0));
+        unsigned char* slot = ring + S * SL::BYTES;
+        if (SL::SG && (b & 7) == 0 && h == 0)  // the group's weight scales, ahead of the step's own loads
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_w, (lds_void_t)(ring + SL::SR + ((b >> 3) & 1) * 2048 + 512 * wave), 16,
+                                                     vsg, (uint32_t)min(b >> 3, (nb - 1) >> 3) * 1024, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r_act, (lds_void_t)(slot + SL::ACT + 1024 * wave), 16, vx, bc * xstep, 0, 0);
+        if ((lane >> 4) == wave)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_ds, (lds_void_t)(slot + SL::ADX), 4, vd, bc * dstep, 0, 0);
+        if constexpr (PAY == 16) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_w, (lds_void_t)(slot + SL::WQ + 1024 * wave), 16, vw, bc * 1024, 0, 0);
+        } else {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_w, (lds_void_t)(slot + SL::WQ + 2048 * wave), 16, vw, bc * 2048, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_w, (lds_void_t)(slot + SL::WQ + 2048 * wave + 1024), 16, vw,
+                                                     (bc + two) * 2048, 0, 0);
+            const uint32_t be = (uint32_t)min(b, (nb - 1) & ~1);  // an even block: its pair lies in one scale group
+            if (h == 0)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r_w, (lds_void_t)(slot + SL::WD + 128 * wave), 4, vsg,
+                                                         (be >> 3) * 1024 + (be & 7) * 2, 0, 0);
         }
-    }
+    };
+    // the step in slot S has landed once at most the RING - 2 later steps' loads are outstanding; the barrier then
+    // publishes it and ends every wave's reads of the slot that the next issue refills
+    auto land = [&](auto SC, int b) {
+        constexpr int S = decltype(SC)::value;
+        __builtin_amdgcn_s_waitcnt(vm_wait(SL::DMA * (RING - 2)));
+        __builtin_amdgcn_s_barrier();
+        issue(ic<(S + RING - 1) % RING>{}, b + 2 * (RING - 1));
+    };
+
+    mf16 S[1];
+#pragma unroll
+    for (int q = 0; q < 16; q++) S[0][q] = 0.0f;
+    const mf16 zero = {};
+    const uint32_t hmask = h == 0 ? 0xFFFFu : 0u;  // the scale MFMA's single k sits in lanes 0-31, element 0
+    // the lane's read addresses in slot 0: [block of the step][operand half]
+    const uint32_t p0 = r32 * 128 + (h ^ small_swz(r32)) * 16;
+    const uint32_t A_B[2][2] = {{ring0 + SL::ACT + p0, ring0 + SL::ACT + (p0 ^ 32)},
+                                {ring0 + SL::ACT + (p0 ^ 64), ring0 + SL::ACT + (p0 ^ 96)}};
+    const uint32_t A_DX = ring0 + SL::ADX + 4 * r32;
+    const uint32_t A_WQ = ring0 + SL::WQ + 64 * PAY * wave + PAY * r32 + 8 * h;
+    const uint32_t A_SG = ring0 + SL::SR + 512 * wave + 16 * r32, A_WD = ring0 + SL::WD + 128 * wave + 4 * r32;
+    u32x2 wq0, wq1;
+    uint32_t wdv, dx;
+    u32x4 B0, B1;
+    // block b: the second (sec, uniform) or first block of the step in slot S.  (Addresses, not branches, choose: a
+    // read's result must reach its wait without a join in between.)
+    auto start_reads = [&](auto SC, bool sec, int b) {
+        constexpr int O = decltype(SC)::value * SL::BYTES;
+        const uint32_t aw = A_WQ + (sec ? 32 * PAY : 0), ax = A_DX + (sec ? 128 : 0);
+        const uint32_t a0 = sec ? A_B[1][0] : A_B[0][0], a1 = sec ? A_B[1][1] : A_B[0][1];
+        wq0 = ds_r64<O>(aw);
+        if (PAY == 32) wq1 = ds_r64<O + 16>(aw);
+        if constexpr (SL::SG) wdv = ds_ru16<0>(A_SG + (uint32_t)(((b >> 3) & 1) * 2048 + (b & 7) * 2));
+        else wdv = ds_ru16<O>(A_WD + 2 * (b & 1));
+        B0 = ds_r128<O>(a0);
+        B1 = ds_r128<O>(a1);
+        dx = ds_r32<O>(ax);
+    };
+    auto start_wait = [&]() {
+        if (PAY == 32) lds_wait(B0, B1, dx, wq0, wq1, wdv);
+        else lds_wait(B0, B1, dx, wq0, wdv);
+    };
+    u32x4 bd = {0u, 0u, 0u, 0u}, ad = {0u, 0u, 0u, 0u};  // scale operands: one nonzero element
+    // block H of the step in slot S, its operands already read; then the next block's reads (of this step, or of
+    // the next one once it has landed), and the chain behind them
+    auto block = [&](auto SC, auto HC, int b) {
+        constexpr int SV = decltype(SC)::value, H = decltype(HC)::value;
+        mh8 A0, A1;
+        if (TYPE == PHX_Q4_0_DEV) {
+            A0 = bias8(wq0.x & 0x0F0F0F0Fu, wq0.y & 0x0F0F0F0Fu, 1032.0f);
+            A1 = bias8((wq0.x >> 4) & 0x0F0F0F0Fu, (wq0.y >> 4) & 0x0F0F0F0Fu, 1032.0f);
+        } else {
+            A0 = bias8(wq0.x ^ 0x80808080u, wq0.y ^ 0x80808080u, 1152.0f);
+            A1 = bias8(wq1.x ^ 0x80808080u, wq1.y ^ 0x80808080u, 1152.0f);
+        }
+        ad.x = wdv & hmask;
+        bd.x = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__uint_as_float(dx)) & hmask;  // (exact)
+        mf16 C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0, __builtin_bit_cast(mh8, B0), zero, 0, 0, 0);
+        C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, __builtin_bit_cast(mh8, B1), C, 0, 0, 0);
+        const mf16 D = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mh8, ad), __builtin_bit_cast(mh8, bd), zero, 0, 0, 0);
+        if constexpr (H == 0) {
+            start_reads(SC, true, b + 1);
+        } else {
+            constexpr int S1 = (SV + 1) % RING;
+            land(ic<S1>{}, b + 1);
+            start_reads(ic<S1>{}, b + 2 == nb, b + 1);  // a row's last odd block is the second of its step
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 16; q++) S[0][q] = S[0][q] + C[q] * D[q];
+        asm volatile("" : "+v"(S[0]));  // the chain stays here
+        __builtin_amdgcn_sched_barrier(0);
+        start_wait();
+    };
+    auto step = [&](auto SC, int b) {  // blocks b, b + 1, or the last one alone
+        if (b + 1 < nb) block(SC, ic<0>{}, b);
+        block(SC, ic<1>{}, min(b + 1, nb - 1));
+    };
+    static_for<RING - 1>([&](auto I) { issue(I, 2 * decltype(I)::value); });
+    land(ic<0>{}, 0);
+    start_reads(ic<0>{}, nb == 1, 0);
+    start_wait();
+    for (int b = 0; b < nb; b += 2 * RING)
+        static_for<RING>([&](auto I) {
+            const int bi = b + 2 * decltype(I)::value;
+            if (bi < nb) step(I, bi);
+        });
+    __builtin_amdgcn_s_waitcnt(0);  // the loads issued past the last block land before the workgroup ends
+    mma_finish<1>(g, tl, cnt, ring, S, gI, half, live);
 }
 
 // XCD-aware order of the grouped products' grid (gridDim.x row-group pairs by tile slots, the slots
@@ -438,7 +622,7 @@ inline int xcd_tile_slots(int max_tiles) { return (max_tiles + 7) / 8 * 8; }
 template <int TYPE>
 __global__ __launch_bounds__(256, 3) void k_grouped_mfma(MmaArgs g)
 {
-    __shared__ __align__(16) unsigned char ring[MmaSlot<TYPE>::LDS];
+    __shared__ __align__(16) unsigned char ring[std::max(MmaSlot<TYPE>::LDS, MmaSmall<TYPE>::LDS)];
     int bx;
     const int tile = xcd_tile(&bx);
     Tile tl;
@@ -451,7 +635,7 @@ __global__ __launch_bounds__(256, 3) void k_grouped_mfma(MmaArgs g)
     if (threadIdx.x == 0 && wgf < 8192) phx_tl[tbase + 2 * wgf] = wall_clock64();
 #endif
     switch ((cnt + 31) / 32) {  // active 32-token column tiles
-    case 1: mma_tile<TYPE, 1>(g, tl, cnt, ring, bx); break;
+    case 1: mma_small<TYPE>(g, tl, cnt, ring, bx); break;
     case 2: mma_tile<TYPE, 2>(g, tl, cnt, ring, bx); break;
     case 3: mma_tile<TYPE, 3>(g, tl, cnt, ring, bx); break;
     default: mma_tile<TYPE, 4>(g, tl, cnt, ring, bx); break;

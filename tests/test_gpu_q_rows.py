@@ -5,7 +5,8 @@ phx_matmul runs up to 16 rows, and more while that gives few workgroups, through
 caller's planar rows: eight blocks per wave, up to 16 waves a round, four input rows per tile.  The cases sit at
 those edges: one block, one wave, one block more, a full round and one block past it, ragged tiles and row
 groups, and rows whose address is 4 but not 16 bytes aligned.  Larger calls run on the matrix cores in tiles
-chosen by the size of the launch (32 rows for the Q4_0 cases here; 16, 32 and 48 for the K-quant ones).  A
+chosen by the size of the launch (32 rows for the Q4_0 cases here, of one
+block and of three too; 16, 32 and 48 for the K-quant ones).  A
 layer of few experts takes the whole-row kernel with its fused requantization.  Every sum is the reference's
 chain, so results are equal bit for bit."""
 import numpy as np
@@ -28,7 +29,8 @@ def check_rows(y, ref, T, rng):
 
 @pytest.mark.parametrize("wtype", [2, 8])
 @pytest.mark.parametrize("T,rows,cols", [(1, 1, 32), (3, 130, 256), (5, 63, 288), (1, 65, 4096), (2, 64, 4128),
-                                         (4, 64, 8224), (17, 2112, 704), (19, 9300, 96), (300, 4224, 256)])
+                                         (4, 64, 8224), (17, 2112, 704), (19, 9300, 32), (19, 9300, 96),
+                                         (300, 4224, 256)])
 def test_dense_rows_match_oracle(ctx, pkg, orc, wtype, T, rows, cols):
     say(f"q rows: type={wtype} T={T} rows={rows} cols={cols}")
     rng = np.random.default_rng(rows + cols + wtype + T)
