@@ -868,11 +868,17 @@ static bool kmma_path(const phx_moe_layer_desc& D, int T, int ncu)
     return n >= 8 * D.n_expert || (n >= D.n_expert && (int64_t)n * ((D.n_ff + 31) / 32) > 4 * ncu);
 }
 
+// prefill-sized: from eight assignments per expert the tolerance flag applies to the experts' products and the gate
+// and up products are stored only on request; the smaller calls on the matrix cores do neither (exact products,
+// intermediates kept, like the VALU rows' calls below them)
+static bool prefill_sized(const phx_moe_layer_desc& D, int T) { return T * D.n_used >= 8 * D.n_expert; }
+
 // whether a call stores the gate and up products for phx_moe_get_intermediates: the matrix-core Q4_0 /
-// Q8_0 products requantize gelu(g) * u in registers and store g and u only when asked to
+// Q8_0 products requantize gelu(g) * u in registers and store g and u only when asked to or not prefill-sized
 bool keeps_gu(phx_moe_ctx* c, const Layer& L, int T, unsigned flags)
 {
-    return (flags & PHX_FLAG_KEEP_INTERMEDIATES) || use_decode(c, L, T, flags) || !mma_path(L.desc, T);
+    return (flags & PHX_FLAG_KEEP_INTERMEDIATES) || use_decode(c, L, T, flags) || !mma_path(L.desc, T) ||
+           !prefill_sized(L.desc, T);
 }
 
 // Tiles of a single matrix's matrix-core product over T rows in order (row-group pairs x tiles workgroups).
@@ -894,7 +900,7 @@ int ident_tile_k(int T, int pairs, int ncu)
 }
 
 int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, const float* shared, float* out, float* xres,
-                      bool exact, bool fast, bool keep)
+                      bool exact, bool fast, bool keep)  // keep: keeps_gu
 {
     const phx_moe_layer_desc& D = L.desc;
     hipStream_t st = c->stream;
@@ -903,6 +909,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
     const bool shared_ffn = shared == nullptr && D.n_ff_shared > 0;
     const bool mma = mma_path(D, T);
     const bool kmma = kmma_path(D, T, c->ncu);
+    const bool efast = fast && (mma || kmma) && prefill_sized(D, T);  // (the shared FFN's own rule: smma)
     const bool smma = shared_ffn && mfma_type(D.shared_type) && T >= 32;
     Act agu = make_act(c, act_fmt(D.gate_up_type), d, W_AGU_Q, W_AGU_D, W_AGU_S);
     if (mma || kmma) {
@@ -911,7 +918,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
     }
     // the tolerance mode (the matrix-core products): every fp16 activation copy carries its block scale
     // folded in, which selects the tolerance-mode products
-    agu.fold = fast && (mma || kmma);
+    agu.fold = efast;
     if (kmma && D.gate_up_type == PHX_Q4_K) {
         agu.bh = wp<uint16_t>(c, W_AGU_BH);
         agu.bhstride = d / 16;
@@ -1048,8 +1055,8 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             }
         }
     }
-    // tile sizes: the MFMA kernels' 128 (Q4_0 / Q8_0) and 32 (K-quants), the VALU kernels' 4 (their row
-    // walk is VALU-bound: larger tiles cost occupancy and measured slower)
+    // tile sizes: the MFMA kernels' 128 (Q4_0 / Q8_0) and 48 (K-quants), the VALU kernels' 4 (their rows
+    // are VALU-bound: larger tiles cost occupancy and measured slower)
     const int tileA = mma ? kMmaTile : kmma ? kKmmaTile : kTileA;
     const int max_tiles = std::min(n, (n + tileA - 1) / tileA + E);
     if (!(cert && T == 1)) {
@@ -1063,7 +1070,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
         adn.qh = wp<uint16_t>(c, W_ADN_H);
         adn.qhstride = D.down_cols;
     }
-    adn.fold = fast && (mma || kmma);
+    adn.fold = efast;
     if (kmma && D.down_type == PHX_Q4_K) {
         adn.bh = wp<uint16_t>(c, W_ADN_BH);
         adn.bhstride = D.down_cols / 16;
@@ -1119,7 +1126,7 @@ int run_layer(phx_moe_ctx* c, const Layer& L, int T, const float* x, const float
 {
     if (use_decode(c, L, T, flags)) return run_layer_decode(c, L, T, x, shared, out, xres);
     return run_layer_general(c, L, T, x, shared, out, xres, (flags & PHX_FLAG_EXACT_ROUTER) != 0,
-                             (flags & PHX_FLAG_FAST_MATH) != 0, (flags & PHX_FLAG_KEEP_INTERMEDIATES) != 0);
+                             (flags & PHX_FLAG_FAST_MATH) != 0, keeps_gu(c, L, T, flags));
 }
 
 int upload_f32(phx_moe_ctx* c, const float* src, size_t n, float** dst)
@@ -2107,8 +2114,7 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
         return set_err(c, PHX_ERR_ARG, "matmul_k: xq, xd and y need 4-byte alignment");
     ENTER(c);
     const int cols = w->cols;
-    // the general path's rule with one matrix (at least 8 rows per matrix): the matrix cores, else the
-    // VALU row walk
+    // from 8 rows the matrix cores, else the VALU rows
     const bool kmma = T >= 8 && kmma_type(w->type);
     const int A = kmma ? ident_tile_k(T, (w->q.rg + 1) / 2, c->ncu) : kTileA;
     const int max_tiles = (T + A - 1) / A;

@@ -37,6 +37,24 @@ def test_mid_sized_layers_match_oracle(ctx, pkg, orc, case, exact):
     check_layer(ctx, orc, L, pkg.synth.make_input(cfg, T=T), tag=f"mid {case}", exact=exact)
 
 
+@pytest.mark.parametrize("case", ["q4_0_at", "q8_0_at_shared_mfma", "q4k_q6k_matrix_cores"])
+def test_mid_sized_calls_are_not_prefill_sized(ctx, pkg, case):
+    """Under eight assignments per expert a call keeps its gate and up products unasked, and the tolerance flag
+    leaves the experts' products exact (the shared FFN follows its own rule, so it is given here)."""
+    cfg, T = CASES[case]
+    say(f"mid layer flags {case}")
+    L = pkg.synth.make_layer(cfg, norms="random")
+    ctx.upload(0, L)
+    x = pkg.synth.make_input(cfg, T=T)
+    sh = x[::-1].copy()
+    want = ctx.ffn(0, x, sh, keep_intermediates=True)
+    inter = ctx.intermediates()
+    for kw in ({}, dict(fast_math=True)):
+        np.testing.assert_array_equal(ctx.ffn(0, x, sh, **kw), want)
+        for a, b in zip(ctx.intermediates(), inter):
+            np.testing.assert_array_equal(a, b)
+
+
 def test_shared_branch_stream_order(pkg):
     say("shared FFN beside the experts: queued calls and a captured stack")
     cfg = dict(idx=97, T=40, d=512, E=16, k=2, nf=256, gu=2, dn=2, nff=512, sh=2)
