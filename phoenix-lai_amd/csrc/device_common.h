@@ -618,6 +618,10 @@ __device__ __forceinline__ void lds_wait(u32x4& a, u32x4& b, uint32_t& c)
 {
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c)::"memory");
 }
+__device__ __forceinline__ void lds_wait(u32x4& a, uint32_t& c, u32x2& d, u32x2& e, uint32_t& f)
+{
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(c), "+v"(d), "+v"(e), "+v"(f)::"memory");
+}
 __device__ __forceinline__ void lds_wait(u32x4& a, u32x4& b, uint32_t& c, u32x2& d, uint32_t& f)
 {
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(f)::"memory");

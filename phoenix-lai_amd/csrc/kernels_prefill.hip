@@ -34,6 +34,7 @@
 namespace phx {
 
 typedef _Float16 mh8 __attribute__((ext_vector_type(8)));
+typedef float mf4 __attribute__((ext_vector_type(4)));
 typedef float mf16 __attribute__((ext_vector_type(16)));
 
 struct MmaArgs {
@@ -432,25 +433,28 @@ __device__ __forceinline__ void mma_tile(const MmaArgs& g, const Tile& tl, int c
     mma_finish<NJ>(g, tl, cnt, ring, S, gI, half, live);
 }
 
-// A tile of one 32-token column (few assignments per expert, or few rows): the weights' stream bounds it, so its
-// ring holds only 32 tokens and steps of two blocks: three direct loads per wave and step (five for
+// A tile of one token column of NT = 32 or 16 (few assignments per expert, or few rows): the weights' stream
+// bounds it, so its ring holds only NT tokens and steps of two blocks: three direct loads per wave and step (five for
 // Q8_0) where mma_tile issues eight (ten), and the LDS of three workgroups per CU keeps eight (Q8_0: six)
 // blocks ahead in flight instead of three.  77 tokens, 8 of 128 experts, 704 x 2816 Q4_0: gate|up 131 -> 112 us
 // beside the shared FFN, down 57 -> 51, the layer 225 -> 205 us (2048 tokens, whose tiles' remainders come here:
 // 563 -> 553 us).
-//   activations [32 tokens][8 parts of 16 B]: parts 0-3 the step's first block, 4-7 its second, part p at
+// Up to 16 tokens the wave's 32 rows are two 16 x 16 tiles of v_mfma_f32_16x16x32_f16, a block each: half the
+// matrix-core passes, chain steps and activation bytes of the 32-token column (77 tokens, 4.8 per expert: gate|up
+// 112 -> 105 us, down 51 -> 48, the layer 203 -> 197).
+//   activations [NT tokens][8 parts of 16 B]: parts 0-3 the step's first block, 4-7 its second, part p at
 //   position p ^ small_swz(token) (an operand read's 16 lanes hit 16 distinct bank groups); token scales
-//   [2 blocks][32]; payload per wave [2 blocks][32 rows][PAY]; weight scales in the scale ring of mma_tile (Q4_0),
+//   [2 blocks][NT]; payload per wave [2 blocks][32 rows][PAY]; weight scales in the scale ring of mma_tile (Q4_0),
 //   or the step's two per row, 4 bytes, in the slot (Q8_0, whose scale ring would take the third workgroup).
 // A row of an odd number of blocks ends with the step (nb - 2, nb - 1), of which only the second block is new; a
 // row of one block takes it as both.
-template <int TYPE>
+template <int TYPE, int NT>
 struct MmaSmall {
     static constexpr int PAY = TYPE == PHX_Q4_0_DEV ? 16 : 32;
     static constexpr bool SG = PAY == 16;
     static constexpr int DMA = SG ? 3 : 5;                 // direct loads per wave per step (scale groups aside)
     static constexpr int RING = PAY == 16 ? 5 : 4;         // steps; the scale ring allows at most eight blocks ahead
-    static constexpr int ACT = 0, ADX = ACT + 4096, WQ = ADX + 256;
+    static constexpr int ACT = 0, ADX = ACT + 128 * NT, WQ = ADX + 8 * NT;
     static constexpr int WD = WQ + 4 * 64 * PAY;           // (Q8_0) per wave [32 rows][2 fp16]
     static constexpr int BYTES = WD + (SG ? 0 : 4 * 128);
     static constexpr int SR = RING * BYTES;                // (Q4_0) scale ring: [2 groups][4 waves][32 rows][8 fp16]
@@ -460,12 +464,12 @@ struct MmaSmall {
 };
 __device__ __forceinline__ int small_swz(int t) { return (t ^ (t >> 3)) & 7; }
 
-template <int TYPE>
+template <int TYPE, int NT>
 __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int cnt, unsigned char* ring, int bx)
 {
-    using SL = MmaSmall<TYPE>;
+    using SL = MmaSmall<TYPE, NT>;
     constexpr int PAY = SL::PAY, RING = SL::RING;
-    const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, h = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, h = lane >> 5, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int gI = bx * 2 + (wave >> 1), half = wave & 1;
     const bool live = gI < g.rg;  // a wave past the last row group computes a clamped one, stores nothing
@@ -478,11 +482,11 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
         const int p = tl.start + min(t, cnt - 1);
         return lst ? (int64_t)p : (int64_t)(mma_perm(g, p) / g.act_div);
     };
-    // (1) activations of tokens 8 w + lane / 8
-    const int ta = 8 * wave + (lane >> 3), pa_ = (lane & 7) ^ small_swz(ta);
+    // (1) activations of tokens NT / 4 * w + lane / 8 (NT = 16: lanes 0-31)
+    const int ta = NT / 4 * wave + (lane >> 3) % (NT / 4), pa_ = (lane & 7) ^ small_swz(ta);
     const uint32_t vx = (uint32_t)(2 * arow(ta) * (lst ? 32 : g.act.qhstride)) + 16u * (pa_ & 3) + (pa_ >> 2) * two * xstep;
-    // (2) token scales: lanes 16 w .. 16 w + 15 of [2 blocks][32 tokens]
-    const uint32_t vd = (uint32_t)(4 * arow(r32) * (lst ? 1 : g.act.dstride)) + h * two * dstep;
+    // (2) token scales: a quarter of [2 blocks][NT tokens] per wave
+    const uint32_t vd = (uint32_t)(4 * arow(lane % NT) * (lst ? 1 : g.act.dstride)) + lane / NT % 2 * two * dstep;
     // (3) payload: Q4_0 rows 32 half + r32 of both blocks, Q8_0 row 32 half + lane / 2, half lane % 2, of one block
     // per load
     const int gIc = min(gI, g.rg - 1);
@@ -499,8 +503,10 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
         if (SL::SG && (b & 7) == 0 && h == 0)  // the group's weight scales, ahead of the step's own loads
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r_w, (lds_void_t)(ring + SL::SR + ((b >> 3) & 1) * 2048 + 512 * wave), 16,
                                                      vsg, (uint32_t)min(b >> 3, (nb - 1) >> 3) * 1024, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r_act, (lds_void_t)(slot + SL::ACT + 1024 * wave), 16, vx, bc * xstep, 0, 0);
-        if ((lane >> 4) == wave)
+        if (NT == 32 || h == 0)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_act, (lds_void_t)(slot + SL::ACT + 32 * NT * wave), 16, vx, bc * xstep,
+                                                     0, 0);
+        if (lane / (NT / 2) == wave)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r_ds, (lds_void_t)(slot + SL::ADX), 4, vd, bc * dstep, 0, 0);
         if constexpr (PAY == 16) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r_w, (lds_void_t)(slot + SL::WQ + 1024 * wave), 16, vw, bc * 1024, 0, 0);
@@ -524,16 +530,22 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
     };
 
     mf16 S[1];
+    mf4 S4[2];  // NT = 16: rows 16 i + 4 (lane / 16) .. + 3 of token lane % 16
 #pragma unroll
     for (int q = 0; q < 16; q++) S[0][q] = 0.0f;
+    S4[0] = S4[1] = mf4{0.0f, 0.0f, 0.0f, 0.0f};
     const mf16 zero = {};
-    const uint32_t hmask = h == 0 ? 0xFFFFu : 0u;  // the scale MFMA's single k sits in lanes 0-31, element 0
-    // the lane's read addresses in slot 0: [block of the step][operand half]
-    const uint32_t p0 = r32 * 128 + (h ^ small_swz(r32)) * 16;
+    const mf4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    // the scale MFMA's single k: element 0 of lanes 0-31; NT = 16: of lanes 0-15 for rows 0-15 and of lanes 16-31
+    // for rows 16-31, whose scales those lanes read
+    const uint32_t hmask = (NT == 32 ? h == 0 : kq == 0) ? 0xFFFFu : 0u, hmask1 = kq == 1 ? 0xFFFFu : 0u;
+    // the lane's read addresses in slot 0: [block of the step][operand half] (NT = 16: the lane's part is all of it)
+    const int rt = lane % NT;
+    const uint32_t p0 = rt * 128 + ((NT == 32 ? h : kq) ^ small_swz(rt)) * 16;
     const uint32_t A_B[2][2] = {{ring0 + SL::ACT + p0, ring0 + SL::ACT + (p0 ^ 32)},
                                 {ring0 + SL::ACT + (p0 ^ 64), ring0 + SL::ACT + (p0 ^ 96)}};
-    const uint32_t A_DX = ring0 + SL::ADX + 4 * r32;
-    const uint32_t A_WQ = ring0 + SL::WQ + 64 * PAY * wave + PAY * r32 + 8 * h;
+    const uint32_t A_DX = ring0 + SL::ADX + 4 * rt;
+    const uint32_t A_WQ = ring0 + SL::WQ + 64 * PAY * wave + PAY * rt + 8 * (NT == 32 ? h : PAY == 16 ? kq & 1 : kq);
     const uint32_t A_SG = ring0 + SL::SR + 512 * wave + 16 * r32, A_WD = ring0 + SL::WD + 128 * wave + 4 * r32;
     u32x2 wq0, wq1;
     uint32_t wdv, dx;
@@ -542,18 +554,20 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
     // read's result must reach its wait without a join in between.)
     auto start_reads = [&](auto SC, bool sec, int b) {
         constexpr int O = decltype(SC)::value * SL::BYTES;
-        const uint32_t aw = A_WQ + (sec ? 32 * PAY : 0), ax = A_DX + (sec ? 128 : 0);
+        const uint32_t aw = A_WQ + (sec ? 32 * PAY : 0), ax = A_DX + (sec ? 4 * NT : 0);
         const uint32_t a0 = sec ? A_B[1][0] : A_B[0][0], a1 = sec ? A_B[1][1] : A_B[0][1];
         wq0 = ds_r64<O>(aw);
-        if (PAY == 32) wq1 = ds_r64<O + 16>(aw);
+        if (NT == 16) wq1 = ds_r64<O + 16 * PAY>(aw);  // row 16 + rt
+        else if (PAY == 32) wq1 = ds_r64<O + 16>(aw);
         if constexpr (SL::SG) wdv = ds_ru16<0>(A_SG + (uint32_t)(((b >> 3) & 1) * 2048 + (b & 7) * 2));
         else wdv = ds_ru16<O>(A_WD + 2 * (b & 1));
         B0 = ds_r128<O>(a0);
-        B1 = ds_r128<O>(a1);
+        if (NT == 32) B1 = ds_r128<O>(a1);
         dx = ds_r32<O>(ax);
     };
     auto start_wait = [&]() {
-        if (PAY == 32) lds_wait(B0, B1, dx, wq0, wq1, wdv);
+        if (NT == 16) lds_wait(B0, dx, wq0, wq1, wdv);
+        else if (PAY == 32) lds_wait(B0, B1, dx, wq0, wq1, wdv);
         else lds_wait(B0, B1, dx, wq0, wdv);
     };
     u32x4 bd = {0u, 0u, 0u, 0u}, ad = {0u, 0u, 0u, 0u};  // scale operands: one nonzero element
@@ -562,7 +576,11 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
     auto block = [&](auto SC, auto HC, int b) {
         constexpr int SV = decltype(SC)::value, H = decltype(HC)::value;
         mh8 A0, A1;
-        if (TYPE == PHX_Q4_0_DEV) {
+        if (NT == 16 && TYPE == PHX_Q4_0_DEV) {  // k 0-15 the low nibbles, 16-31 the high ones
+            const int sh = 2 * (kq & 2);
+            A0 = bias8((wq0.x >> sh) & 0x0F0F0F0Fu, (wq0.y >> sh) & 0x0F0F0F0Fu, 1032.0f);
+            A1 = bias8((wq1.x >> sh) & 0x0F0F0F0Fu, (wq1.y >> sh) & 0x0F0F0F0Fu, 1032.0f);
+        } else if (TYPE == PHX_Q4_0_DEV) {
             A0 = bias8(wq0.x & 0x0F0F0F0Fu, wq0.y & 0x0F0F0F0Fu, 1032.0f);
             A1 = bias8((wq0.x >> 4) & 0x0F0F0F0Fu, (wq0.y >> 4) & 0x0F0F0F0Fu, 1032.0f);
         } else {
@@ -570,10 +588,21 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
             A1 = bias8(wq1.x ^ 0x80808080u, wq1.y ^ 0x80808080u, 1152.0f);
         }
         ad.x = wdv & hmask;
-        bd.x = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__uint_as_float(dx)) & hmask;  // (exact)
-        mf16 C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0, __builtin_bit_cast(mh8, B0), zero, 0, 0, 0);
-        C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, __builtin_bit_cast(mh8, B1), C, 0, 0, 0);
-        const mf16 D = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mh8, ad), __builtin_bit_cast(mh8, bd), zero, 0, 0, 0);
+        const uint32_t dxh = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__uint_as_float(dx));  // (exact)
+        bd.x = dxh & hmask;
+        mf16 C, D;
+        mf4 C4[2], D4[2];
+        if constexpr (NT == 16) {
+            const u32x4 ad1 = {wdv & hmask1, 0u, 0u, 0u}, bd1 = {dxh & hmask1, 0u, 0u, 0u};
+            C4[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, __builtin_bit_cast(mh8, B0), zero4, 0, 0, 0);
+            C4[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1, __builtin_bit_cast(mh8, B0), zero4, 0, 0, 0);
+            D4[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mh8, ad), __builtin_bit_cast(mh8, bd), zero4, 0, 0, 0);
+            D4[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mh8, ad1), __builtin_bit_cast(mh8, bd1), zero4, 0, 0, 0);
+        } else {
+            C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0, __builtin_bit_cast(mh8, B0), zero, 0, 0, 0);
+            C = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, __builtin_bit_cast(mh8, B1), C, 0, 0, 0);
+            D = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mh8, ad), __builtin_bit_cast(mh8, bd), zero, 0, 0, 0);
+        }
         if constexpr (H == 0) {
             start_reads(SC, true, b + 1);
         } else {
@@ -582,9 +611,15 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
             start_reads(ic<S1>{}, b + 2 == nb, b + 1);  // a row's last odd block is the second of its step
         }
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NT == 16) {
 #pragma unroll
-        for (int q = 0; q < 16; q++) S[0][q] = S[0][q] + C[q] * D[q];
-        asm volatile("" : "+v"(S[0]));  // the chain stays here
+            for (int q = 0; q < 8; q++) S4[q >> 2][q & 3] = S4[q >> 2][q & 3] + C4[q >> 2][q & 3] * D4[q >> 2][q & 3];
+            asm volatile("" : "+v"(S4[0]), "+v"(S4[1]));  // the chain stays here
+        } else {
+#pragma unroll
+            for (int q = 0; q < 16; q++) S[0][q] = S[0][q] + C[q] * D[q];
+            asm volatile("" : "+v"(S[0]));
+        }
         __builtin_amdgcn_sched_barrier(0);
         start_wait();
     };
@@ -602,6 +637,10 @@ __device__ __forceinline__ void mma_small(const MmaArgs& g, const Tile& tl, int 
             if (bi < nb) step(I, bi);
         });
     __builtin_amdgcn_s_waitcnt(0);  // the loads issued past the last block land before the workgroup ends
+    if constexpr (NT == 16) {  // mma_finish's layout: rows 8 (q / 4) + 4 h + q % 4 (its tokens past 15: copies, not stored)
+#pragma unroll
+        for (int q = 0; q < 16; q++) S[0][q] = __shfl(S4[q >> 3][q & 3], (lane & 15) + 16 * h + 32 * ((q >> 2) & 1), 64);
+    }
     mma_finish<1>(g, tl, cnt, ring, S, gI, half, live);
 }
 
@@ -622,7 +661,7 @@ inline int xcd_tile_slots(int max_tiles) { return (max_tiles + 7) / 8 * 8; }
 template <int TYPE>
 __global__ __launch_bounds__(256, 3) void k_grouped_mfma(MmaArgs g)
 {
-    __shared__ __align__(16) unsigned char ring[std::max(MmaSlot<TYPE>::LDS, MmaSmall<TYPE>::LDS)];
+    __shared__ __align__(16) unsigned char ring[std::max(MmaSlot<TYPE>::LDS, MmaSmall<TYPE, 32>::LDS)];
     int bx;
     const int tile = xcd_tile(&bx);
     Tile tl;
@@ -635,7 +674,10 @@ __global__ __launch_bounds__(256, 3) void k_grouped_mfma(MmaArgs g)
     if (threadIdx.x == 0 && wgf < 8192) phx_tl[tbase + 2 * wgf] = wall_clock64();
 #endif
     switch ((cnt + 31) / 32) {  // active 32-token column tiles
-    case 1: mma_small<TYPE>(g, tl, cnt, ring, bx); break;
+    case 1:
+        if (cnt <= 16) mma_small<TYPE, 16>(g, tl, cnt, ring, bx);
+        else mma_small<TYPE, 32>(g, tl, cnt, ring, bx);
+        break;
     case 2: mma_tile<TYPE, 2>(g, tl, cnt, ring, bx); break;
     case 3: mma_tile<TYPE, 3>(g, tl, cnt, ring, bx); break;
     default: mma_tile<TYPE, 4>(g, tl, cnt, ring, bx); break;
@@ -1128,7 +1170,6 @@ struct KmRing {
 };
 
 typedef _Float16 mh4 __attribute__((ext_vector_type(4)));
-typedef float mf4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t pk_fma(uint32_t a, mh2 b, mh2 c)
 {

@@ -30,6 +30,7 @@ def check_rows(y, ref, T, rng):
 @pytest.mark.parametrize("wtype", [2, 8])
 @pytest.mark.parametrize("T,rows,cols", [(1, 1, 32), (3, 130, 256), (5, 63, 288), (1, 65, 4096), (2, 64, 4128),
                                          (4, 64, 8224), (17, 2112, 704), (19, 9300, 32), (19, 9300, 96),
+                                         (33, 9300, 32), (48, 4224, 96),
                                          (300, 4224, 256)])
 def test_dense_rows_match_oracle(ctx, pkg, orc, wtype, T, rows, cols):
     say(f"q rows: type={wtype} T={T} rows={rows} cols={cols}")
