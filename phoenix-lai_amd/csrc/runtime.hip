@@ -792,6 +792,9 @@ DecLayerH dec_layer(phx_moe_ctx* c, const Layer& L, int T, const float* x, const
     return h;
 }
 
+// The decode path's four launches up to 16 tokens.  Against the general path (same results; 8 of 128 experts,
+// d = 2816): Q4_0 with a shared FFN T = 4 58 us against 82, T = 8 86 against 124, T = 16 151 against 155; Q8_0
+// T = 8 91 against 122, T = 16 137 against 136; 4 of 32 experts, d = 1024: T = 8 32 against 61, T = 16 42 against 63.
 bool use_decode(phx_moe_ctx* c, const Layer& L, int T, unsigned flags)
 {
     const phx_moe_layer_desc& D = L.desc;
