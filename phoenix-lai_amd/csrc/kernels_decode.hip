@@ -99,9 +99,11 @@ struct DecArgs {
     const float* xin;     // with xres: the residual's source rows when not xres itself (or null)
     const float* gelu_tab;
     int* flags;           // [0] norm fallbacks, [1] router fallbacks
-    Tile* gtiles;         // one token: the general path's tile list and count, written by the selection (or null)
-    int* ngtiles;
 };
+// The workgroup size, which the runtime puts 12 bytes past a kernel's own arguments, shares the arguments' last
+// cache line; with 16 bytes more it is one line further (8 of 128 experts, d = 2816, Q4_0 with a shared FFN, a
+// layer call with those 16 bytes and without: T = 2 39.55 and 39.3 us, T = 8 81.2 and 80.9).
+static_assert(sizeof(DecArgs) / 64 == (sizeof(DecArgs) + 17) / 64, "the workgroup size lies on the arguments' last line");
 
 // ------------------------------------------------------------------------------ helpers
 
@@ -1609,9 +1611,16 @@ __global__ __launch_bounds__(CF_NT) void k_cert_fallback(DecArgs a)
     }
 }
 
+// One token: where the general path's tile list and count go (or null).  An argument of the selection alone, not
+// of DecArgs (see the assertion there).
+struct OneLists {
+    Tile* tiles;
+    int* n;
+};
+
 // Few tokens (at most two workgroups per compute unit): one workgroup of CF_NT threads per token, the
 // fast path in wave 0 and, for a token the bounds leave open, the exact selection in the same launch.
-__global__ __launch_bounds__(CF_NT) void k_cert_select_one(DecArgs a)
+__global__ __launch_bounds__(CF_NT) void k_cert_select_one(DecArgs a, OneLists lists)
 {
     extern __shared__ __align__(16) unsigned char csm[];  // sel_lds(1, E, d, CF_NT, CF_P)
     __shared__ int s_ids[PHX_MAX_USED_DEV];
@@ -1631,7 +1640,7 @@ __global__ __launch_bounds__(CF_NT) void k_cert_select_one(DecArgs a)
     if (exact) select_exact<true>(b, csm, s_ids, &s_bad, red, true);
     if (wave == 0) token_routing_out(a, t, exact ? (const double*)csm : b.Lb, s_ids);
     // one token: its lists here, as k_dispatch would write them (an assignment per expert, in expert order)
-    if (!a.gtiles) return;  // uniform
+    if (!lists.tiles) return;  // uniform
     __syncthreads();        // the exact selection's ids
     if (wave == 1) {
         const int id = clamp_id(s_ids[min(lane, a.k - 1)], a.E);
@@ -1642,9 +1651,9 @@ __global__ __launch_bounds__(CF_NT) void k_cert_select_one(DecArgs a)
         }
         if (lane < a.k) {
             a.perm[pos] = lane;
-            a.gtiles[pos] = Tile{id, pos, 1};
+            lists.tiles[pos] = Tile{id, pos, 1};
         }
-        if (lane == 0) *a.ngtiles = a.k;
+        if (lane == 0) *lists.n = a.k;
         for (int e = lane; e <= a.E; e += 64) {
             int c = 0;
             for (int j = 0; j < a.k; j++) c += __builtin_amdgcn_readlane(id, j) < e;
@@ -2244,8 +2253,6 @@ static DecArgs dec_args(const DecLayerH& h)
     a.xin = h.xin;
     a.gelu_tab = h.gelu_tab;
     a.flags = h.flags;
-    a.gtiles = h.gtiles;
-    a.ngtiles = h.ngtiles;
     return a;
 }
 
@@ -2355,7 +2362,7 @@ void launch_cert_select(hipStream_t st, const DecLayerH& h)
     if (cert_select_one_launch(h)) {  // a workgroup per token in at most two rounds: one launch
         const size_t lds1 = sel_lds(1, h.E, h.d, CF_NT, CF_P).total;
         raise_lds(k_cert_select_one, lds1);
-        launch(k_cert_select_one, dim3(h.T), dim3(CF_NT), (uint32_t)lds1, st, a);
+        launch(k_cert_select_one, dim3(h.T), dim3(CF_NT), (uint32_t)lds1, st, a, OneLists{h.gtiles, h.ngtiles});
         return;
     }
     launch(k_cert_select, dim3((h.T + CS_TPW - 1) / CS_TPW), dim3(64 * CS_TPW), 0, st, a);
