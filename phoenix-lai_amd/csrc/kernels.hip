@@ -804,8 +804,9 @@ struct GroupArgs {
     int snf = 0;
     const uint16_t* d16 = nullptr;  // k_grouped_q_wide: the scales as planar fp16 bits (act.d unused)
     int nident = 0;    // > 0 (tiles null): one matrix, tile i the rows 4 i .. 4 i + 3 of nident, in order
-    int amax = 4;      // k_grouped_k, k_grouped_q_wide: assignments a tile can hold in this call (its LDS), and the most tiles
-    int mt = 1;        // (workgroup b: tile b % mt, row group b / mt)
+    int amax = 4;      // k_grouped_k, k_grouped_q_wide: assignments a tile can hold in this call (its LDS)
+    int mt = 1;        // k_grouped_q_wide: the most tiles (workgroup b: tile b % mt, row group b / mt)
+    bool rgx = false;  // k_grouped_k: the grid's x the row groups and y the tiles, else x the tiles
     const void* grid;  // IQ types: the expanded codebook (64-bit words for IQ2_XXS / IQ2_S, 32-bit for IQ3_S)
     Act req;                       // req.q set: the paired gate|up kernel also writes gelu(g) * u as Q8_0 rows
     const float* gelu_tab = nullptr;
@@ -1225,12 +1226,11 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
     constexpr bool Q4K = TYPE == PHX_Q4_K_DEV, Q5K = TYPE == PHX_Q5_K_DEV;
     constexpr bool AFF = Q4K || Q5K;  // scales and mins per 32 (the min term); else 16 signed scales per 16
     constexpr int PAY = Q4K ? 144 : Q5K ? 176 : 208, NT = gk_terms<TYPE>();
-    const int tile = blockIdx.x % g.mt;
     Tile tl;
-    if (!group_tile(g, tile, &tl)) return;
+    if (!group_tile(g, g.rgx ? blockIdx.y : blockIdx.x, &tl)) return;
     const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, nw = nt >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int rgi = blockIdx.x / g.mt, nb = g.nb, cnt = min(tl.cnt, g.amax);
+    const int rgi = g.rgx ? blockIdx.x : blockIdx.y, nb = g.nb, cnt = min(tl.cnt, g.amax);
     const int sg = min(nb, GK_W / nw * nw);  // super-blocks staged at a time: whole rounds of the waves
     extern __shared__ __align__(16) unsigned char gk_smem[];
     float* term = (float*)gk_smem;                                // [buffer][wave][NT][64]
@@ -1410,17 +1410,23 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
 // waves, several workgroups to a compute unit: their loads and chains run under each other's products, which
 // then bound it (about 700 VALU instructions per super-block and wave; 16 waves each 10-20% slower from 32
 // tokens on).
+// The grid has two dimensions (tiles times row groups times threads may pass the 2^32 threads a dimension can
+// hold).  Lists of several tokens have slots past their last tile, whose workgroups end at once: with the tiles in
+// x, these recur at the same places of every row group's run and leave some of the engines that the dispatcher
+// serves in turn with less work than others, so the row groups are in x and the empty slots at the grid's end (64
+// experts of 4096 columns, T = 8: the layer 204 -> 122 us; 128 of 2816: 107 -> 88).  Rows in order have no empty
+// slots, and neighbours in x share a row group's weights.
 template <int TYPE>
 static void launch_grouped_k(hipStream_t st, GroupArgs g, int max_tiles, int ncu)
 {
-    g.mt = max_tiles;
     const bool wide = (int64_t)max_tiles * g.rg <= ncu;
     const int rounds = wide ? (g.nb + GK_W - 1) / GK_W : (g.nb + 3) / 4, nw = (g.nb + rounds - 1) / rounds;
     const int lds = gk_lds<TYPE>(nw, g.amax, std::min(g.nb, GK_W / nw * nw), g.gsrc != nullptr);
     static_assert(gk_lds<TYPE>(GK_W, 4, GK_W, true) <= 160 * 1024, "the widest launch fits a compute unit's LDS");
     (void)hipFuncSetAttribute((const void*)k_grouped_k<TYPE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               gk_lds<TYPE>(GK_W, 4, GK_W, true));
-    launch(k_grouped_k<TYPE>, dim3((unsigned)max_tiles * (unsigned)g.rg), dim3(64 * nw), (uint32_t)lds, st, g);
+    g.rgx = g.nident ? g.rg > 65535 : !wide && g.amax > 1;
+    launch(k_grouped_k<TYPE>, g.rgx ? dim3(g.rg, max_tiles) : dim3(max_tiles, g.rg), dim3(64 * nw), (uint32_t)lds, st, g);
 }
 
 // Signs applied to four codebook bytes: bit j of nib set negates byte j.  The bit spread gives 0x01 in

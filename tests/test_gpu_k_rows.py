@@ -1,4 +1,4 @@
-"""K-quant products of a few rows (k_grouped_k): its rounds, tiles and alignments against the oracle.
+"""K-quant products on the vector units (k_grouped_k): rounds, tiles, alignments and grid against the oracle.
 
 A workgroup takes a 64-row group and a tile of up to four input rows, a wave per super-block in rounds of up
 to 16 (a launch that fills less than the chip) or about four.  The cases sit at those edges: one super-block,
@@ -37,6 +37,33 @@ def test_few_rows_match_oracle(ctx, orc, wtype, T, rows, cols):
             y = bufs[2].download((T, rows))
             for t in range(T):
                 np.testing.assert_array_equal(y[t], orc.matvec(wtype, w, rows, cols, x[t]), err_msg=f"token {t}")
+    finally:
+        for b in bufs:
+            b.free()
+        ctx.weight_free(h)
+
+
+def test_grid_past_one_dimension(ctx, orc):
+    """The largest T of a Q5_K product (no matrix-core kernel takes it) over 1024 row groups: 16384 tiles x 1024 row
+    groups x 256 threads are 2^32, one more than a grid's dimension holds."""
+    wtype, T, rows, cols = 13, 65535, 65473, 1024
+    say(f"k rows: grid past one dimension T={T} rows={rows}")
+    rng = np.random.default_rng(5)
+    w = gguf_k_rows(rng, wtype, rows, cols)
+    x = rng.standard_normal((7, cols)).astype(np.float32)
+    qs, d, _ = ctx.Q8K(0, x)
+    h = ctx.weight_upload(wtype, w, rows, cols)
+    at = np.arange(T) % len(x)
+    bufs = [ctx.alloc(T * cols), ctx.alloc(T * cols // 256 * 4), ctx.alloc(T * rows * 4)]
+    try:
+        bufs[0].upload(qs.reshape(-1, cols)[at])
+        bufs[1].upload(d.reshape(len(x), -1)[at])
+        ctx.matmul_k_device(h, T, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr)
+        ctx.sync()
+        for t in (0, 3, T // 2, T - 2, T - 1):
+            y = np.empty(rows, np.float32)
+            ctx._check(ctx.lib.phx_moe_memcpy_d2h(ctx.h, y.ctypes.data, bufs[2].ptr + t * rows * 4, y.nbytes))
+            np.testing.assert_array_equal(y, orc.matvec(wtype, w, rows, cols, x[t % len(x)]), err_msg=f"token {t}")
     finally:
         for b in bufs:
             b.free()
