@@ -806,7 +806,7 @@ struct GroupArgs {
     int nident = 0;    // > 0 (tiles null): one matrix, tile i the rows 4 i .. 4 i + 3 of nident, in order
     int amax = 4;      // k_grouped_k, k_grouped_q_wide: assignments a tile can hold in this call (its LDS)
     int mt = 1;        // k_grouped_q_wide: the most tiles (workgroup b: tile b % mt, row group b / mt)
-    bool rgx = false;  // k_grouped_k: the grid's x the row groups and y the tiles, else x the tiles
+    bool rgx = false;  // K-quants: the grid's x the row groups (or fours of them) and y the tiles, else x the tiles
     const void* grid;  // IQ types: the expanded codebook (64-bit words for IQ2_XXS / IQ2_S, 32-bit for IQ3_S)
     Act req;                       // req.q set: the paired gate|up kernel also writes gelu(g) * u as Q8_0 rows
     const float* gelu_tab = nullptr;
@@ -1199,6 +1199,116 @@ __global__ __launch_bounds__(64 * GQ_W) void k_grouped_q_wide(GroupArgs g)
     }
 }
 
+// A lane's row of one K-quant super-block: the values as byte dwords (dword 8 s + l: elements 32 s + l + 8 m, m =
+// 0..3; Q6_K: value - 32, signed), the sub-block scales (and mins), the super-block's scales.
+template <int TYPE>
+struct GkRow {
+    static constexpr bool Q4K = TYPE == PHX_Q4_K_DEV, Q5K = TYPE == PHX_Q5_K_DEV;
+    static constexpr bool AFF = Q4K || Q5K;  // scales and mins per 32 (the min term); else 16 signed scales per 16
+    static constexpr int PAY = Q4K ? 144 : Q5K ? 176 : 208, SBY = AFF ? 4 : 2;
+    static constexpr int BLK = 64 * (PAY + SBY);  // 64 rows' super-block: the rows' scales follow the chunks
+    uint32_t wv[PAY / 4], dmw;  // as loaded
+    uint32_t v[64];
+    int sc[16], mn[8];
+    float d, dmin;
+    // bp: the super-block's first chunk of lane `lane`
+    __device__ __forceinline__ void load(const uint8_t* bp, int lane)
+    {
+        const uint4* src = (const uint4*)bp;
+#pragma unroll
+        for (int c = 0; c < PAY / 16; c++) {
+            const uint4 t4 = src[c * 64];
+            wv[4 * c] = t4.x; wv[4 * c + 1] = t4.y; wv[4 * c + 2] = t4.z; wv[4 * c + 3] = t4.w;
+        }
+        const uint8_t* sp = bp + 64 * PAY - lane * (16 - SBY);
+        dmw = AFF ? *(const uint32_t*)sp : *(const uint16_t*)sp;
+    }
+    __device__ __forceinline__ void unpack()
+    {
+        d = h2f(dmw & 0xFFFF);
+        dmin = AFF ? h2f(dmw >> 16) : 0.0f;
+#pragma unroll
+        for (int w = 0; w < 32; w++) {
+            v[2 * w] = wv[w] & 0x0F0F0F0Fu;
+            v[2 * w + 1] = (wv[w] >> 4) & 0x0F0F0F0Fu;
+        }
+        if (AFF) {
+            if (Q5K)  // the fifth bits: bit l of byte mm of dword s belongs to value dword 8 s + l, byte mm
+#pragma unroll
+                for (int x = 0; x < 64; x++) v[x] |= ((wv[PAY / 4 - 8 + x / 8] >> (x % 8)) & 0x01010101u) << 4;
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                sc[s] = (wv[32 + s / 4] >> (8 * (s % 4))) & 0xFF;
+                mn[s] = (wv[34 + s / 4] >> (8 * (s % 4))) & 0xFF;
+            }
+        } else {
+#pragma unroll
+            for (int x = 0; x < 64; x++) {  // minus 32 per byte: 0x60 .. 0x9F after the add, no carry between bytes
+                v[x] |= ((wv[32 + x / 4] >> (2 * (x % 4))) & 0x03030303u) << 4;
+                v[x] = (v[x] + 0x60606060u) ^ 0x80808080u;
+            }
+#pragma unroll
+            for (int s = 0; s < 16; s++) sc[s] = (int)(int8_t)((wv[PAY / 4 - 4 + s / 4] >> (8 * (s % 4))) & 0xFF);
+        }
+    }
+    // the eight integer lanes against an input row's staged super-block x4
+    __device__ __forceinline__ void dot(const uint4* x4, int (&aux)[8]) const
+    {
+#pragma unroll
+        for (int l = 0; l < 8; l++) aux[l] = 0;
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const uint4 xa = x4[2 * s], xc = x4[2 * s + 1];
+            const uint32_t x[8] = {xa.x, xa.y, xa.z, xa.w, xc.x, xc.y, xc.z, xc.w};
+#pragma unroll
+            for (int l = 0; l < 8; l++) {
+                const int p = __builtin_amdgcn_sdot4((int)v[8 * s + l], (int)x[l], 0, false);
+                if (AFF) {
+                    aux[l] += __mul24(sc[s], p);
+                } else {  // elements l, l + 8 carry scale 2 s, l + 16, l + 24 scale 2 s + 1
+                    const int pa = __builtin_amdgcn_sdot4((int)v[8 * s + l], (int)(x[l] & 0xFFFFu), 0, false);
+                    aux[l] += __mul24(sc[2 * s], pa);
+                    aux[l] += __mul24(sc[2 * s + 1], p - pa);
+                }
+            }
+        }
+    }
+    // the min term's integer against the input's eight sums of 32
+    __device__ __forceinline__ int mins(const int* bs) const
+    {
+        int sumi = 0;
+#pragma unroll
+        for (int s = 0; s < 8; s++) sumi += __mul24(bs[s], mn[s]);
+        return sumi;
+    }
+};
+
+// An input sub-block of 32 (dwords 0..3 in n0, 4..7 in n1, elements 4 j .. 4 j + 3 in dword j) in the weights' order,
+// dst[l] = elements l + 8 m: 4 x 4 byte transposes, bytes l of dwords j, j + 2, j + 4, j + 6 (l = 4 j .. 4 j + 3)
+__device__ __forceinline__ void gk_spread(const u32x4_a4& n0, const u32x4_a4& n1, uint32_t* dst)
+{
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const uint32_t a0 = n0[j], a1 = n0[j + 2], a2 = n1[j], a3 = n1[j + 2];
+        const uint32_t p0 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), p1 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
+        const uint32_t p2 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), p3 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
+        *(uint4*)(dst + 4 * j) = make_uint4(__builtin_amdgcn_perm(p2, p0, 0x05040100u),
+                                            __builtin_amdgcn_perm(p2, p0, 0x07060302u),
+                                            __builtin_amdgcn_perm(p3, p1, 0x05040100u),
+                                            __builtin_amdgcn_perm(p3, p1, 0x07060302u));
+    }
+}
+__device__ __forceinline__ int gk_sum(const u32x4_a4& n0, const u32x4_a4& n1)
+{
+    int sm = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        sm = __builtin_amdgcn_sdot4((int)n0[j], 0x01010101, sm, false);
+        sm = __builtin_amdgcn_sdot4((int)n1[j], 0x01010101, sm, false);
+    }
+    return sm;
+}
+
 // K-quant rows of a few assignments: DotK (src/CpuRefKQuants.cs:177-212) per (row, assignment): per
 // super-block the eight integer lanes aux32[l] (element e contributes to lane e % 8), float lanes
 // sums[l] += (d * yd) * aux32[l], the Q4_K / Q5_K min term sumf -= (dmin * yd) * sumi, finally sumf += sums[l].
@@ -1223,9 +1333,8 @@ __host__ __device__ constexpr int gk_lds(int nw, int amax, int sg, bool form)
 template <int TYPE>
 __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
 {
-    constexpr bool Q4K = TYPE == PHX_Q4_K_DEV, Q5K = TYPE == PHX_Q5_K_DEV;
-    constexpr bool AFF = Q4K || Q5K;  // scales and mins per 32 (the min term); else 16 signed scales per 16
-    constexpr int PAY = Q4K ? 144 : Q5K ? 176 : 208, NT = gk_terms<TYPE>();
+    constexpr bool AFF = GkRow<TYPE>::AFF;
+    constexpr int NT = gk_terms<TYPE>();
     Tile tl;
     if (!group_tile(g, g.rgx ? blockIdx.y : blockIdx.x, &tl)) return;
     const int tid = threadIdx.x, lane = tid & 63, nt = blockDim.x, nw = nt >> 6;
@@ -1240,22 +1349,10 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
     float* xd = (float*)(xb + g.amax * sg * 8);                   // [assignment][super-block]
     uint32_t* xn = (uint32_t*)(xd + g.amax * sg);                 // [assignment][super-block][64], rows formed here
     const uint8_t* wp = g.payload + tl.e * g.mat_pay + rgi * g.rg_pay + lane * 16;
-    constexpr int SBY = AFF ? 4 : 2, BLK = 64 * (PAY + SBY);  // the rows' scales follow the block's chunks
     auto arow = [&](int i) -> int64_t {
         return group_perm(g, tl.start + i) / g.act_div;
     };
-    uint32_t wv[PAY / 4], dmw;
-    auto load = [&](int r0) {  // this wave's super-block of the round (past the end: the last one again)
-        const int b = min(r0 + wave, nb - 1);
-        const uint4* src = (const uint4*)(wp + (int64_t)b * BLK);
-#pragma unroll
-        for (int c = 0; c < PAY / 16; c++) {
-            const uint4 t4 = src[c * 64];
-            wv[4 * c] = t4.x; wv[4 * c + 1] = t4.y; wv[4 * c + 2] = t4.z; wv[4 * c + 3] = t4.w;
-        }
-        const uint8_t* sp = wp + (int64_t)b * BLK + 64 * PAY - lane * (16 - SBY);
-        dmw = AFF ? *(const uint32_t*)sp : *(const uint16_t*)sp;
-    };
+    GkRow<TYPE> w;
     // integers of super-blocks s0 .. s0 + n - 1: a thread per 32-element sub-block and round loads eight dwords
     // (elements 4 j .. 4 j + 3)
     auto stage = [&](int s0, int n) {
@@ -1288,97 +1385,31 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
                 n1 = src[1];
             }
             if (!g.gsrc && (xr & 7) == 0) xd[xi * sg + (xr >> 3)] = g.act.d[arow(xi) * g.act.dstride + s0 + (xr >> 3)];
-            // 4 x 4 byte transposes: bytes l of dwords j, j + 2, j + 4, j + 6 (l = 4 j .. 4 j + 3)
-            uint32_t* dst = xs + (xi * sg + (xr >> 3)) * 64 + (xr & 7) * 8;
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const uint32_t a0 = n0[j], a1 = n0[j + 2], a2 = n1[j], a3 = n1[j + 2];
-                const uint32_t p0 = __builtin_amdgcn_perm(a1, a0, 0x05010400u), p1 = __builtin_amdgcn_perm(a1, a0, 0x07030602u);
-                const uint32_t p2 = __builtin_amdgcn_perm(a3, a2, 0x05010400u), p3 = __builtin_amdgcn_perm(a3, a2, 0x07030602u);
-                *(uint4*)(dst + 4 * j) = make_uint4(__builtin_amdgcn_perm(p2, p0, 0x05040100u),
-                                                    __builtin_amdgcn_perm(p2, p0, 0x07060302u),
-                                                    __builtin_amdgcn_perm(p3, p1, 0x05040100u),
-                                                    __builtin_amdgcn_perm(p3, p1, 0x07060302u));
-            }
-            if (AFF) {
-                int sm = 0;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    sm = __builtin_amdgcn_sdot4((int)n0[j], 0x01010101, sm, false);
-                    sm = __builtin_amdgcn_sdot4((int)n1[j], 0x01010101, sm, false);
-                }
-                xb[(xi * sg + (xr >> 3)) * 8 + (xr & 7)] = sm;
-            }
+            gk_spread(n0, n1, xs + (xi * sg + (xr >> 3)) * 64 + (xr & 7) * 8);
+            if (AFF) xb[(xi * sg + (xr >> 3)) * 8 + (xr & 7)] = gk_sum(n0, n1);
         }
     };
     int buf = 0;
     for (int r0 = 0; r0 < nb; r0 += nw) {
         const int nbr = min(nw, nb - r0);
-        load(r0);
+        // this wave's super-block of the round (past the end: the last one again)
+        w.load(wp + (int64_t)min(r0 + wave, nb - 1) * GkRow<TYPE>::BLK, lane);
         if (r0 % sg == 0) {  // uniform; every read of the staged rows and terms before it is over
             stage(r0, min(sg, nb - r0));
             __syncthreads();
         }
         const int sl = r0 % sg + min(wave, nbr - 1);  // this wave's staged super-block
-        const float d = h2f(dmw & 0xFFFF), dmin = AFF ? h2f(dmw >> 16) : 0.0f;
-        // the row's values as byte dwords (Q6_K: value - 32, signed) and its scales
-        uint32_t v[64];
-        int sc[16], mn[8];
-#pragma unroll
-        for (int w = 0; w < 32; w++) {
-            v[2 * w] = wv[w] & 0x0F0F0F0Fu;
-            v[2 * w + 1] = (wv[w] >> 4) & 0x0F0F0F0Fu;
-        }
-        if (AFF) {
-            if (Q5K)  // the fifth bits: bit l of byte mm of dword s belongs to value dword 8 s + l, byte mm
-#pragma unroll
-                for (int x = 0; x < 64; x++) v[x] |= ((wv[PAY / 4 - 8 + x / 8] >> (x % 8)) & 0x01010101u) << 4;
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                sc[s] = (wv[32 + s / 4] >> (8 * (s % 4))) & 0xFF;
-                mn[s] = (wv[34 + s / 4] >> (8 * (s % 4))) & 0xFF;
-            }
-        } else {
-#pragma unroll
-            for (int x = 0; x < 64; x++) {  // minus 32 per byte: 0x60 .. 0x9F after the add, no carry between bytes
-                v[x] |= ((wv[32 + x / 4] >> (2 * (x % 4))) & 0x03030303u) << 4;
-                v[x] = (v[x] + 0x60606060u) ^ 0x80808080u;
-            }
-#pragma unroll
-            for (int s = 0; s < 16; s++) sc[s] = (int)(int8_t)((wv[PAY / 4 - 4 + s / 4] >> (8 * (s % 4))) & 0xFF);
-        }
+        w.unpack();
         for (int i = 0; i < cnt; i++) {  // uniform
-            const uint4* x4 = (const uint4*)(xs + (i * sg + sl) * 64);
             int aux[8];
-#pragma unroll
-            for (int l = 0; l < 8; l++) aux[l] = 0;
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const uint4 xa = x4[2 * s], xc = x4[2 * s + 1];
-                const uint32_t x[8] = {xa.x, xa.y, xa.z, xa.w, xc.x, xc.y, xc.z, xc.w};
-#pragma unroll
-                for (int l = 0; l < 8; l++) {
-                    const int p = __builtin_amdgcn_sdot4((int)v[8 * s + l], (int)x[l], 0, false);
-                    if (AFF) {
-                        aux[l] += __mul24(sc[s], p);
-                    } else {  // elements l, l + 8 carry scale 2 s, l + 16, l + 24 scale 2 s + 1
-                        const int pa = __builtin_amdgcn_sdot4((int)v[8 * s + l], (int)(x[l] & 0xFFFFu), 0, false);
-                        aux[l] += __mul24(sc[2 * s], pa);
-                        aux[l] += __mul24(sc[2 * s + 1], p - pa);
-                    }
-                }
-            }
-            const float yd = xd[i * sg + sl], dd = d * yd;
+            w.dot((const uint4*)(xs + (i * sg + sl) * 64), aux);
+            const float yd = xd[i * sg + sl], dd = w.d * yd;
             float* t = term + (buf * nw + wave) * NT * 64 + lane;
 #pragma unroll
             for (int l = 0; l < 8; l++) t[l * 64] = dd * (float)aux[l];
             if (AFF) {
-                const int* bs = xb + (i * sg + sl) * 8;
-                int sumi = 0;
-#pragma unroll
-                for (int s = 0; s < 8; s++) sumi += __mul24(bs[s], mn[s]);
-                const float dm = dmin * yd;
-                t[8 * 64] = dm * (float)sumi;
+                const float dm = w.dmin * yd;
+                t[8 * 64] = dm * (float)w.mins(xb + (i * sg + sl) * 8);
             }
             __syncthreads();  // the terms are there; the other buffer's chains are done
             for (int c = wave; c < NT; c += nw) {
@@ -1404,6 +1435,79 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
     }
 }
 
+// The same products of a launch of many assignments: a wave takes a row group's whole row of super-blocks with its
+// chains in registers (no terms through LDS, no barrier per assignment), and the workgroup's four row groups share
+// the tile's staged integers, KW_S super-blocks at a time.  It is bound by its VALU instructions: 1200 for a wave's
+// Q5_K super-block and four assignments, 97% of the SIMDs' cycles (4224 x 4096, T = 1024: 555 us; three waves to a
+// SIMD by its 146 to 160 VGPRs).
+constexpr int KW_S = 8;
+template <int TYPE>
+__global__ __launch_bounds__(256) void k_grouped_k_walk(GroupArgs g)
+{
+    constexpr bool AFF = GkRow<TYPE>::AFF;
+    constexpr int A = 4;
+    Tile tl;
+    if (!group_tile(g, g.rgx ? blockIdx.y : blockIdx.x, &tl)) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rgi = (g.rgx ? blockIdx.x : blockIdx.y) * 4 + wave, nb = g.nb, cnt = min(tl.cnt, A);
+    const bool live = rgi < g.rg;  // a wave past the last row group walks a clamped one, stores nothing
+    __shared__ __align__(16) uint32_t xs[A * KW_S * 64];  // [assignment][super-block][64]
+    __shared__ int xb[A * KW_S * 8];                      // [assignment][super-block][8]
+    __shared__ float xd[A * KW_S];                        // [assignment][super-block]
+    const uint8_t* wp = g.payload + tl.e * g.mat_pay + min(rgi, g.rg - 1) * g.rg_pay + lane * 16;
+    GkRow<TYPE> w;
+    float sums[A][8], sumf[A];
+#pragma unroll
+    for (int i = 0; i < A; i++) {
+        sumf[i] = 0.0f;
+#pragma unroll
+        for (int l = 0; l < 8; l++) sums[i][l] = 0.0f;
+    }
+    for (int s0 = 0; s0 < nb; s0 += KW_S) {
+        const int n = min(KW_S, nb - s0);
+        if (s0) __syncthreads();  // the staged rows before these are read
+        for (int x = tid; x < cnt * n * 8; x += 256) {
+            const int xi = x / (n * 8), xr = x - xi * n * 8, o = xi * KW_S + (xr >> 3);
+            const int64_t r = group_perm(g, tl.start + xi) / g.act_div;
+            const u32x4_a4* src = (const u32x4_a4*)(g.act.q + r * g.act.qstride + (int64_t)s0 * 256 + xr * 32);
+            const u32x4_a4 n0 = src[0], n1 = src[1];
+            if ((xr & 7) == 0) xd[o] = g.act.d[r * g.act.dstride + s0 + (xr >> 3)];
+            gk_spread(n0, n1, xs + o * 64 + (xr & 7) * 8);
+            if (AFF) xb[o * 8 + (xr & 7)] = gk_sum(n0, n1);
+        }
+        __syncthreads();
+        for (int b = 0; b < n; b++) {
+            w.load(wp + (int64_t)(s0 + b) * GkRow<TYPE>::BLK, lane);
+            w.unpack();
+#pragma unroll
+            for (int i = 0; i < A; i++) {
+                if (i < cnt) {  // uniform
+                    const int o = i * KW_S + b;
+                    int aux[8];
+                    w.dot((const uint4*)(xs + o * 64), aux);
+                    const float yd = xd[o], dd = w.d * yd;
+#pragma unroll
+                    for (int l = 0; l < 8; l++) sums[i][l] += dd * (float)aux[l];
+                    if (AFF) {
+                        const float dm = w.dmin * yd;
+                        sumf[i] -= dm * (float)w.mins(xb + o * 8);
+                    }
+                }
+            }
+        }
+    }
+    if (!live) return;  // wave-uniform
+#pragma unroll
+    for (int i = 0; i < A; i++)
+        if (i < cnt) {
+            float s = sumf[i];
+#pragma unroll
+            for (int l = 0; l < 8; l++) s += sums[i][l];
+            store_row(g, rgi, lane, group_perm(g, tl.start + i), s);
+        }
+}
+
 // A launch whose workgroups all find a compute unit of their own takes a wave per super-block (everything in
 // flight at once: a 4096-column Q4_K row group of four experts, 176 workgroups, 10.4 us against 37 for one
 // wave walking all 16 super-blocks; the Q6_K down 9.6 against 28).  A larger one takes rounds of about four
@@ -1416,9 +1520,20 @@ __global__ __launch_bounds__(64 * GK_W) void k_grouped_k(GroupArgs g)
 // serves in turn with less work than others, so the row groups are in x and the empty slots at the grid's end (64
 // experts of 4096 columns, T = 8: the layer 204 -> 122 us; 128 of 2816: 107 -> 88).  Rows in order have no empty
 // slots, and neighbours in x share a row group's weights.
+// Past 24 assignments times row groups per compute unit (nassign: the launch's assignments) the waves walk whole
+// rows instead: Q5_K rows in order, 4224 x 4096 T = 80 (21 per unit) 80 us for k_grouped_k and 87 for the walk, T =
+// 96 100 and 87, T = 1024 782 and 555; 2816 x 2304 T = 1024 318 and 211; layers of 128 experts, d = 2816, Q4_K /
+// Q6_K, T = 32 189 and 181, T = 64 270 and 249; 16 experts of 4096 with 64 assignments (32 and 16 per unit) 254 and
+// 220 with the walk for the gate and up product alone, 245 for both.
 template <int TYPE>
-static void launch_grouped_k(hipStream_t st, GroupArgs g, int max_tiles, int ncu)
+static void launch_grouped_k(hipStream_t st, GroupArgs g, int max_tiles, int nassign, int ncu)
 {
+    if ((int64_t)nassign * g.rg > 24 * ncu && !g.gsrc) {
+        const int rg4 = (g.rg + 3) / 4;
+        g.rgx = g.nident ? rg4 > 65535 : g.amax > 1;
+        launch(k_grouped_k_walk<TYPE>, g.rgx ? dim3(rg4, max_tiles) : dim3(max_tiles, rg4), dim3(256), 0, st, g);
+        return;
+    }
     const bool wide = (int64_t)max_tiles * g.rg <= ncu;
     const int rounds = wide ? (g.nb + GK_W - 1) / GK_W : (g.nb + 3) / 4, nw = (g.nb + rounds - 1) / rounds;
     const int lds = gk_lds<TYPE>(nw, g.amax, std::min(g.nb, GK_W / nw * nw), g.gsrc != nullptr);
@@ -1566,9 +1681,10 @@ static void launch_grouped_q_wide(hipStream_t st, GroupArgs g, int max_tiles)
            (uint32_t)(g.amax * ch * (256 + 40)), st, g);
 }
 
-void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles, int A,
-                    const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
-                    const Act* req, const float* gelu_tab, int req_rows, int nident, int amax, const uint16_t* d16, const GeluRows* form)
+void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
+                    int nassign, int ncu, const int* perm, int act_div, float* out0, float* out1, int split,
+                    int out_stride, const Act* req, const float* gelu_tab, int nident, int amax, const uint16_t* d16,
+                    const GeluRows* form)
 {
     GroupArgs g;
     g.payload = w.payload;
@@ -1612,7 +1728,6 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
         g.gelu_tab = gelu_tab;
     }
     dim3 grid(max_tiles, (w.rg + 3) / 4);
-    (void)A;  // the tile size the dispatch used: 4, the one instantiation
     switch (w.type) {
     case PHX_Q4_0_DEV:
         if (wide) launch_grouped_q_wide<PHX_Q4_0_DEV>(st, g, max_tiles);
@@ -1624,14 +1739,14 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
         else if (w.nb > QG_SHORT) launch((k_grouped_q_ring<PHX_Q8_0_DEV, 4>), grid, dim3(256), grouped_q_lds(w.type, w.nb), st, g);
         else launch((k_grouped_q<PHX_Q8_0_DEV, 4>), grid, dim3(256), 0, st, g);
         break;
-    case PHX_Q4_K_DEV: launch_grouped_k<PHX_Q4_K_DEV>(st, g, max_tiles, 256); break;
-    case PHX_Q5_K_DEV: launch_grouped_k<PHX_Q5_K_DEV>(st, g, max_tiles, 256); break;
-    case PHX_Q6_K_DEV: launch_grouped_k<PHX_Q6_K_DEV>(st, g, max_tiles, 256); break;
+    case PHX_Q4_K_DEV: launch_grouped_k<PHX_Q4_K_DEV>(st, g, max_tiles, nassign, ncu); break;
+    case PHX_Q5_K_DEV: launch_grouped_k<PHX_Q5_K_DEV>(st, g, max_tiles, nassign, ncu); break;
+    case PHX_Q6_K_DEV: launch_grouped_k<PHX_Q6_K_DEV>(st, g, max_tiles, nassign, ncu); break;
     case PHX_IQ2_XXS_DEV: launch((k_grouped_iq<PHX_IQ2_XXS_DEV, 4>), grid, dim3(256), 0, st, g); break;
     case PHX_IQ2_S_DEV: launch((k_grouped_iq<PHX_IQ2_S_DEV, 4>), grid, dim3(256), 0, st, g); break;
     case PHX_IQ3_S_DEV: launch((k_grouped_iq<PHX_IQ3_S_DEV, 4>), grid, dim3(256), 0, st, g); break;
     }
-    if (req && !fuse) launch_requant(st, req_rows, split, out0, out1, gelu_tab, *req);
+    if (req && !fuse) launch_requant(st, nassign, split, out0, out1, gelu_tab, *req);
 }
 
 // ------------------------------------------------------------------------------ GELU-gated requant

@@ -165,13 +165,14 @@ void launch_dispatch(hipStream_t st, int n_assign, int E, int A, const int* ids,
 // form (K-quant types, with gelu_tab): the input rows are the Q8_K of gelu(g) * u, rows of nf values and zeros past
 // them, formed by the product itself; act is unused
 struct GeluRows { const float *g, *u; int nf; };
-// req: the paired gate|up product's down input (gelu(g) * u as Q8_0 rows, req_rows of them), formed in
+// nassign: the assignments of the launch (the rows, with nident); ncu: the device's compute units.
+// req: the paired gate|up product's down input (gelu(g) * u as Q8_0 rows, nassign of them), formed in
 // the product's epilogue where it can be, else by k_requant after it.  nident > 0 (tiles and perm
 // unused): one matrix over nident rows in order.  amax: no tile of the call holds more assignments;
 // d16 (Q4_0 / Q8_0): the scales as planar fp16 bits [row][cols / 32] in place of act.d
 void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, const int* ntiles, int max_tiles,
-                    int A, const int* perm, int act_div, float* out0, float* out1, int split, int out_stride,
-                    const Act* req = nullptr, const float* gelu_tab = nullptr, int req_rows = 0, int nident = 0,
+                    int nassign, int ncu, const int* perm, int act_div, float* out0, float* out1, int split,
+                    int out_stride, const Act* req = nullptr, const float* gelu_tab = nullptr, int nident = 0,
                     int amax = 4, const uint16_t* d16 = nullptr, const GeluRows* form = nullptr);
 void launch_requant(hipStream_t st, int rows, int nf, const float* g, const float* u, const float* gelu_tab, Act act);
 // standalone Q8_0 (fmt_k 0) / Q8_K (fmt_k 1) quantizer of rows x n inputs; mode as PHX_QUANT_*; -1 on a bad mode

@@ -955,14 +955,14 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             launch_grouped_mfma(st, L.sgu, ash, nullptr, nullptr, smax, nullptr, 1, nullptr, nullptr, nff, nff, 0, &asd, T,
                                 c->gelu_tab, T, sA);  // (no reader of g, u)
         else
-            launch_grouped(st, L.sgu, ash, nullptr, nullptr, smax, kTileA, nullptr, 1, wp<float>(c, W_SHG),
-                           wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T, T, T);
+            launch_grouped(st, L.sgu, ash, nullptr, nullptr, smax, T, c->ncu, nullptr, 1, wp<float>(c, W_SHG),
+                           wp<float>(c, W_SHU), nff, nff, &asd, c->gelu_tab, T, T);
         if (smma)
             launch_grouped_mfma(st, L.sdn, asd, nullptr, nullptr, smaxb, nullptr, 1, wp<float>(c, W_SHOUT),
                                 wp<float>(c, W_SHOUT), d, d, T, nullptr, 0, nullptr, T, sB);
         else
-            launch_grouped(st, L.sdn, asd, nullptr, nullptr, smaxb, kTileA, nullptr, 1, wp<float>(c, W_SHOUT),
-                           wp<float>(c, W_SHOUT), d, d, nullptr, nullptr, 0, T, T);
+            launch_grouped(st, L.sdn, asd, nullptr, nullptr, smaxb, T, c->ncu, nullptr, 1, wp<float>(c, W_SHOUT),
+                           wp<float>(c, W_SHOUT), d, d, nullptr, nullptr, T, T);
     };
     auto start_shared = [&](bool on_side) -> int {  // on_side: its input was written on the side stream
         if (!shared_ffn) return PHX_OK;
@@ -1091,8 +1091,9 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             launch_grouped_kmma(st, L.gu, agu, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, wp<int>(c, W_PERM), k,
                                 wp<float>(c, W_G), wp<float>(c, W_U), nf, nf);
         else  // the down input from the product's epilogue (or k_requant right after it)
-            launch_grouped(st, L.gu, agu, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, tileA, wp<int>(c, W_PERM),
-                           k, wp<float>(c, W_G), wp<float>(c, W_U), nf, nf, form ? nullptr : &adn, c->gelu_tab, n, 0, T);
+            launch_grouped(st, L.gu, agu, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, n, c->ncu,
+                           wp<int>(c, W_PERM), k, wp<float>(c, W_G), wp<float>(c, W_U), nf, nf, form ? nullptr : &adn,
+                           c->gelu_tab, 0, T);
     }
     if (kmma) {
         ProfScope p(c, PHX_K_REQUANT);
@@ -1108,9 +1109,9 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
                                 wp<float>(c, W_YD), wp<float>(c, W_YD), d, d);
         else {
             const GeluRows rows{wp<float>(c, W_G), wp<float>(c, W_U), nf};
-            launch_grouped(st, L.dn, adn, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, tileA, wp<int>(c, W_PERM),
-                           1, wp<float>(c, W_YD), wp<float>(c, W_YD), d, d, nullptr, c->gelu_tab, 0, 0, T, nullptr,
-                           form ? &rows : nullptr);
+            launch_grouped(st, L.dn, adn, wp<Tile>(c, W_TILES), wp<int>(c, W_NTILES), max_tiles, n, c->ncu,
+                           wp<int>(c, W_PERM), 1, wp<float>(c, W_YD), wp<float>(c, W_YD), d, d, nullptr, c->gelu_tab, 0, T,
+                           nullptr, form ? &rows : nullptr);
         }
     }
     if (shared_ffn) HIPCHK(c, hipStreamWaitEvent(st, c->ev_shared, 0));  // the shared branch, before the combine
@@ -2100,8 +2101,8 @@ int phx_matmul(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, con
         launch_grouped_mfma(st, w->q, a, nullptr, nullptr, max_tiles, nullptr, 1, y, y, w->rows, w->rows, 0, nullptr, 0,
                             nullptr, T, A);
     else
-        launch_grouped(st, w->q, a, nullptr, nullptr, max_tiles, A, nullptr, 1, y, y, w->rows, w->rows, nullptr, nullptr, 0,
-                       T, T, xd);
+        launch_grouped(st, w->q, a, nullptr, nullptr, max_tiles, T, c->ncu, nullptr, 1, y, y, w->rows, w->rows, nullptr,
+                       nullptr, T, T, xd);
     HIPCHK(c, launch_status(c));
     return PHX_OK;
 }
@@ -2132,8 +2133,8 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
         a.qstride = cols;
         a.d = (float*)xd;
         a.dstride = cols / 256;
-        launch_grouped(st, w->q, a, nullptr, nullptr, max_tiles, A, nullptr, 1, y, y, w->rows, w->rows, nullptr, nullptr, 0,
-                       T, T);
+        launch_grouped(st, w->q, a, nullptr, nullptr, max_tiles, T, c->ncu, nullptr, 1, y, y, w->rows, w->rows, nullptr,
+                       nullptr, T, T);
         HIPCHK(c, launch_status(c));
         return PHX_OK;
     }

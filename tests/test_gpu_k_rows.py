@@ -8,6 +8,7 @@ bytes aligned.  Every sum is the reference's chain, so results are equal bit for
 import numpy as np
 import pytest
 
+from test_gpu_parity import check_layer
 from test_gpu_quant import gguf_k_rows
 
 pytestmark = pytest.mark.gpu
@@ -41,6 +42,43 @@ def test_few_rows_match_oracle(ctx, orc, wtype, T, rows, cols):
         for b in bufs:
             b.free()
         ctx.weight_free(h)
+
+
+# Past 6144 assignments times row groups (24 per compute unit) a wave walks whole rows (k_grouped_k_walk), eight
+# super-blocks staged at a time, four row groups to a workgroup: the last size below that, a super-block, a whole
+# stage and one past it, a row group alone and one past a multiple of four, ragged tiles.
+@pytest.mark.parametrize("T,rows,cols", [(94, 4100, 512), (95, 4100, 256), (97, 4100, 2304), (6145, 63, 2048)])
+def test_walk_matches_oracle(ctx, orc, T, rows, cols):
+    say(f"k walk: T={T} rows={rows} cols={cols}")
+    rng = np.random.default_rng(T + cols)
+    w = gguf_k_rows(rng, 13, rows, cols)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    qs, d, _ = ctx.Q8K(0, x)
+    h = ctx.weight_upload(13, w, rows, cols)
+    try:
+        y = ctx.MatMulK(h, rows, cols, qs, d)
+    finally:
+        ctx.weight_free(h)
+    for t in sorted({0, 1, T - 2, T - 1, *rng.choice(T, 12).tolist()}):
+        np.testing.assert_array_equal(y[t], orc.matvec(13, w, rows, cols, x[t]), err_msg=f"token {t}")
+
+
+WALK_LAYERS = {  # 192 assignments, 33 or more row groups; gate|up and down of different kinds stay on the vector units
+    "q4k_gate_nb9": dict(idx=101, d=2304, E=8, k=2, nf=1056, gu=12, dn=8),
+    "q6k_gate_nb1": dict(idx=102, d=256, E=8, k=2, nf=1056, gu=14, dn=2),
+    "q5k_both": dict(idx=103, d=2304, E=8, k=2, nf=1056, gu=13, dn=13),
+    "q6k_down": dict(idx=104, d=2112, E=8, k=2, nf=288, gu=8, dn=14),
+    "q4k_down": dict(idx=105, d=2112, E=8, k=2, nf=288, gu=2, dn=12),
+}
+
+
+@pytest.mark.parametrize("case", list(WALK_LAYERS))
+def test_walk_layer_matches_oracle(ctx, pkg, orc, case):
+    cfg = dict(WALK_LAYERS[case], T=96)
+    say(f"k walk layer {case}")
+    L = pkg.synth.make_layer(cfg, norms="random")
+    ctx.upload(0, L)
+    check_layer(ctx, orc, L, pkg.synth.make_input(cfg, T=96), tag=f"k walk {case}")
 
 
 def test_grid_past_one_dimension(ctx, orc):
