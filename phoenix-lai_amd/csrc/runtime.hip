@@ -861,14 +861,21 @@ static bool mma_path(const phx_moe_layer_desc& D, int T)
     return mfma_type(D.gate_up_type) && mfma_type(D.down_type) && T * D.n_used >= 3 * D.n_expert;
 }
 
-// K-quants: from one per expert, unless the VALU rows' workgroups (a row group and a tile each) stay few
-// (64 experts of d = 4096: T = 4 82 us on the VALU rows against 101, T = 8 157 against 153, T = 16 257 against
-// 200, T = 64 442 against 325, T = 127 680 against 360)
+// K-quants: a matrix-core workgroup has a compute unit to itself and takes about 10 us whatever its tile holds, so a
+// layer's W of them (both products, an expert's assignments in one tile) cost rounds over the chip, the VALU rows
+// their assignments.  Past six rounds, from 3.5 assignments per expert (Q4_K / Q6_K; VALU rows and matrix cores: d =
+// 2816, 128 experts, 3 each 219 us and 258, 4 each 249 and 266, 6 each 300 and 262; d = 4096, 64 experts, 2 each 229
+// and 272, 3 each 270 and 316; d = 2048, 256 experts, 3.5 each 213 and 269); at fewer rounds either may be faster by
+// a tenth (16 experts of d = 4096: 2 each 173 and 190, 3 each 210 and 195; 32 of 2816: 1.5 each 74 and 64, 2 each 77
+// and 85; 8 of 4096, W = 512: 3 each 91 and 63): from one, unless the VALU rows' workgroups (a row group and a tile
+// each) stay few.
 static bool kmma_path(const phx_moe_layer_desc& D, int T, int ncu)
 {
     if (!kmma_type(D.gate_up_type) || !kmma_type(D.down_type)) return false;
-    const int n = T * D.n_used;
-    return n >= 8 * D.n_expert || (n >= D.n_expert && (int64_t)n * ((D.n_ff + 31) / 32) > 4 * ncu);
+    const int n = T * D.n_used, rgu = (D.n_ff + 31) / 32, rdn = (D.d + kRowGroup - 1) / kRowGroup;
+    if (n >= 8 * D.n_expert) return true;
+    const int64_t W = (int64_t)D.n_expert * ((rgu + 1) / 2 + (rdn + 1) / 2);
+    return W > 6 * ncu ? 2 * n >= 7 * D.n_expert : n >= D.n_expert && (int64_t)n * rgu > 4 * ncu;
 }
 
 // prefill-sized: from eight assignments per expert the tolerance flag applies to the experts' products and the gate

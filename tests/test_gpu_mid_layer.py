@@ -1,10 +1,11 @@
 """Layers of a few assignments per expert, on both sides of the matrix cores' thresholds, and the shared FFN
 beside the experts (it runs on the context's second stream, joined before the combine).
 
-Q4_0 / Q8_0 products move to the matrix cores at three assignments per expert, K-quant ones at one where the
-row walk would take more than a few workgroups per compute unit; both are the reference's chains, so every
-stage equals the oracle bit for bit.  The stream test queues calls without waits, over two layers, several
-token counts and both routers, and replays a captured stack: every result equals the same call made alone."""
+Q4_0 / Q8_0 products move to the matrix cores at three assignments per expert, K-quant ones at three and a half
+where the matrix-core workgroups would be many, else at one where the VALU rows' workgroups are; all are the
+reference's chains, so every stage equals the oracle bit for bit.  The stream test queues calls without
+waits, over two layers, several token counts and both routers, and replays a captured stack: every result
+equals the same call made alone."""
 import numpy as np
 import pytest
 
@@ -23,6 +24,8 @@ CASES = {
     "q8_0_at_shared_mfma": (dict(idx=93, T=36, d=512, E=24, k=2, nf=256, gu=8, dn=8, nff=256, sh=8), 36),
     "q4k_q6k_few_workgroups": (dict(idx=94, T=8, d=512, E=8, k=2, nf=512, gu=12, dn=14), 8),
     "q4k_q6k_matrix_cores": (dict(idx=95, T=20, d=512, E=8, k=2, nf=1024, gu=12, dn=14), 20),
+    "q4k_q6k_many_below": (dict(idx=98, T=55, d=768, E=64, k=4, nf=1280, gu=12, dn=14), 55),
+    "q4k_q6k_many_at": (dict(idx=99, T=56, d=768, E=64, k=4, nf=1280, gu=12, dn=14), 56),
     "q6k_q4k_shared_q5k": (dict(idx=96, T=24, d=512, E=8, k=2, nf=1024, gu=14, dn=12, nff=512, sh=13), 24),
 }
 
