@@ -846,7 +846,12 @@ bool cert_route(const Layer& L, int T, bool shared_ffn)
     if ((int64_t)T * D.n_expert > CERT_MAX_TE || D.d > 4096 || D.d % 256 != 0 || D.n_expert > 256) return false;
     if (D.d / 32 > 32 * D.n_expert) return false;
     if (dec_type(D.gate_up_type) && (!shared_ffn || dec_type(D.shared_type))) return true;
-    DecLayerH h{};  // Q8_K inputs (K-quant and IQ weights): whole super-blocks by the router's waves
+    // Q8_K inputs (K-quant and IQ weights): whole super-blocks by the router's waves, while the per-pair workgroups and
+    // the selection take less than the exact chains (up to 64 experts those select in the router's own launch: layers
+    // of 64 experts, d = 4096, T = 64 322 us against 325, T = 80 330 against 327, T = 128 354 against 331; 128 of 2816,
+    // T = 48 257 against 261, T = 56 262 against 262, T = 64 265 against 262)
+    if (T * D.n_expert > (D.n_expert <= 64 ? 5120 : 7168)) return false;
+    DecLayerH h{};
     h.T = T;
     h.d = D.d;
     h.E = D.n_expert;
