@@ -5,10 +5,10 @@ phx_matmul runs up to 16 rows, and more while that gives few workgroups, through
 caller's planar rows: eight blocks per wave, up to 16 waves a round, four input rows per tile.  The cases sit at
 those edges: one block, one wave, one block more, a full round and one block past it, ragged tiles and row
 groups, and rows whose address is 4 but not 16 bytes aligned.  Larger calls run on the matrix cores in tiles
-chosen by the size of the launch (32 rows for the Q4_0 cases here, of one
-block and of three too; 16, 32 and 48 for the K-quant ones).  A
-layer of few experts takes the whole-row kernel with its fused requantization.  Every sum is the reference's
-chain, so results are equal bit for bit."""
+chosen by the size of the launch (of Q4_0 / Q8_0 32 rows, of one block and of three too, and 128; of K-quants 16,
+32 and 48).  A layer of few experts and few assignments takes the whole-row kernel with its fused
+requantization; a shared FFN of many row groups and long rows the ring kernel (k_grouped_q_ring) with its
+activations in several chunks.  Every sum is the reference's chain, so results are equal bit for bit."""
 import numpy as np
 import pytest
 
@@ -31,7 +31,7 @@ def check_rows(y, ref, T, rng):
 @pytest.mark.parametrize("T,rows,cols", [(1, 1, 32), (3, 130, 256), (5, 63, 288), (1, 65, 4096), (2, 64, 4128),
                                          (4, 64, 8224), (17, 2112, 704), (19, 9300, 32), (19, 9300, 96),
                                          (33, 9300, 32), (48, 4224, 96),
-                                         (300, 4224, 256)])
+                                         (300, 4224, 256), (2047, 4224, 256)])
 def test_dense_rows_match_oracle(ctx, pkg, orc, wtype, T, rows, cols):
     say(f"q rows: type={wtype} T={T} rows={rows} cols={cols}")
     rng = np.random.default_rng(rows + cols + wtype + T)
@@ -72,10 +72,23 @@ def test_k_tiles_match_oracle(ctx, orc, wtype, T):
 
 
 @pytest.mark.parametrize("wtype", [2, 8])
-@pytest.mark.parametrize("d,nf,nff,T", [(1024, 512, 1024, 20), (512, 96, 288, 18)])
+@pytest.mark.parametrize("d,nf,nff,T", [(1024, 512, 1024, 11), (512, 96, 288, 9)])
 def test_few_expert_layer_matches_oracle(ctx, pkg, orc, wtype, d, nf, nff, T):
+    """Under three assignments per expert (22 and 18 over 8), exact router: no decode path, no matrix cores."""
     say(f"q rows layer: type={wtype} d={d} nf={nf} T={T}")
     cfg = dict(idx=90, T=T, d=d, E=8, k=2, nf=nf, gu=wtype, dn=wtype, nff=nff, sh=wtype)
     L = pkg.synth.make_layer(cfg, norms="random")
     ctx.upload(0, L)
     check_layer(ctx, orc, L, pkg.synth.make_input(cfg, T=T), tag=f"q rows layer {wtype}", exact=True)
+
+
+@pytest.mark.parametrize("wtype", [2, 8])
+def test_ring_chunks_match_oracle(ctx, pkg, orc, wtype):
+    """k_grouped_q_ring over rows of 136 blocks (a chunk of 128 and one of 8) and its fused requantization: 29
+    tokens' shared gate and up rows, eight tiles (the last of one row) of 257 row groups, past the 2048 workgroups
+    that the whole-row kernel takes."""
+    say(f"q rows ring chunks: type={wtype}")
+    cfg = dict(idx=94, T=29, d=4352, E=8, k=2, nf=64, gu=wtype, dn=wtype, nff=8224, sh=wtype)
+    L = pkg.synth.make_layer(cfg, norms="random")
+    ctx.upload(0, L)
+    check_layer(ctx, orc, L, pkg.synth.make_input(cfg, T=29), tag=f"q rows ring chunks {wtype}", exact=True)
