@@ -167,9 +167,9 @@ def test_matvec_matches_oracle(ctx, orc, wtype, T, rows, cols):
                                          (200, 2112, 2816), (2048, 2816, 2112)])
 def test_matmul_matches_oracle(ctx, orc, wtype, T, rows, cols):
     """phx_weight_upload + phx_matmul (KernelsPrefill.MatMulQ4Q8Tile as GemmaGpu.Mm records it) equal
-    CpuRef.MatVec per token, bit for bit: the VALU row walk below 32 tokens, the matrix cores from 32 (one
-    partial 128-token tile, several, and C3's 2048 prompt rows through the shared FFN's down shape); row
-    counts not a multiple of the 64-row group."""
+    CpuRef.MatVec per token, bit for bit: the VALU rows up to 16 tokens and while they give few workgroups
+    (here up to 32 tokens), else the matrix cores (32- and 64-row tiles, and C3's 2048 prompt rows through the
+    shared FFN's down shape); row counts not a multiple of the 64-row group."""
     say(f"matmul: type={wtype} T={T} rows={rows} cols={cols}")
     rng = np.random.default_rng(rows + cols + wtype + T)
     w = gguf_rows(rng, wtype, rows, cols)
@@ -207,7 +207,7 @@ def gguf_k_rows(rng, wtype, rows, cols):
                                          (48, 4096, 1536), (200, 2112, 4096), (512, 4096, 1536)])
 def test_matmul_k_matches_oracle(ctx, orc, wtype, T, rows, cols):
     """phx_quant_q8_k, phx_weight_upload and phx_matmul_k (KernelsK.MatVec as GemmaGpu.MatVec records it for
-    Q4_K / Q6_K weights) equal CpuRefKQuants.MatVecK per token, bit for bit: the VALU row walk below 8
+    Q4_K / Q6_K weights) equal CpuRefKQuants.MatVecK per token, bit for bit: the VALU rows below 8
     tokens, the matrix cores from 8 (one partial tile, whole tiles, and C4's 512 rows through its down
     shape); row counts not a multiple of the 64-row group."""
     say(f"matmul_k: type={wtype} T={T} rows={rows} cols={cols}")
