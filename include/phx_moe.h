@@ -75,8 +75,10 @@ extern "C" {
                                   into fp16 operands and whole rows accumulated on the matrix cores.  Routing,
                                   ids and lists are unchanged (bit-exact); the products differ from the CPU
                                   reference's chains by the operands' fp16 rounding, and the GELU-gated requant
-                                  amplifies that where a value sits near a rounding boundary.  Decode-sized
-                                  calls ignore it. */
+                                  amplifies that where a value sits near a rounding boundary.  Expert
+                                  products of fewer than eight assignments per expert (T * k < 8 E) ignore it;
+                                  a layer's own Q4_0 / Q8_0 shared FFN has a line of its own, T >= 32, except
+                                  in decode-sized calls. */
 #define PHX_FLAG_KEEP_INTERMEDIATES 32u /* also store the gate and up products for phx_moe_get_intermediates
                                            (debug; no counterpart in the reference).  The prefill-sized Q4_0 /
                                            Q8_0 expert products feed their GELU-gated requant straight into the
@@ -296,8 +298,9 @@ int phx_matvec(phx_moe_ctx* ctx, int type, const void* w, int rows, int cols, in
  * src/GemmaGpu.cs:344-352, 402-436); phx_weight_free releases them.  phx_matmul: xq / xd are
  * T Q8_0 rows in the layout of phx_quant_q8_0 (device pointers, xq 4-byte aligned) and
  * y[t][r] = CpuRef.MatVec's value for token t (src/CpuRef.cs:91-119, src/CpuRefGemma.cs:12-40: the block
- * terms (float)isum * (d_w * d_x) added in block order), on the matrix cores for T >= 32;
- * asynchronous on the context's stream.  cols a multiple of 32, at most 16384. */
+ * terms (float)isum * (d_w * d_x) added in block order), on the matrix cores past 16 rows where the launch
+ * is large, else on the vector units straight from xq and xd (same values); asynchronous on the context's
+ * stream.  cols a multiple of 32, at most 16384. */
 typedef struct phx_weight phx_weight;
 int phx_weight_upload(phx_moe_ctx* ctx, int type, int rows, int cols, const void* gguf_rows, phx_weight** out);
 void phx_weight_free(phx_moe_ctx* ctx, phx_weight* w);
@@ -311,8 +314,8 @@ int phx_matmul(phx_moe_ctx* ctx, const phx_weight* w, int T, const int8_t* xq, c
  * PHX_ERR_UNSUPPORTED).  xq / xd: T Q8_K input rows in the layout of phx_quant_q8_k (qs int8 [T][cols],
  * d float [T][cols/256]; device pointers, 4-byte aligned); the block sums are formed from xq.
  * y[t][r] = CpuRefKQuants.MatVecK's value for token t (src/CpuRefKQuants.cs:176-232: DotK's integer lane
- * sums, the eight float lanes and their fold); on the matrix cores from 8 rows, the VALU row walk below;
- * asynchronous on the context's stream. */
+ * sums, the eight float lanes and their fold); on the matrix cores from 8 rows (Q5_K never), else on the
+ * vector units straight from xq and xd (same values); asynchronous on the context's stream. */
 int phx_matmul_k(phx_moe_ctx* ctx, const phx_weight* w, int T, const int8_t* xq, const float* xd, float* y);
 
 #ifdef __cplusplus

@@ -58,6 +58,27 @@ def test_mid_sized_calls_are_not_prefill_sized(ctx, pkg, case):
             np.testing.assert_array_equal(a, b)
 
 
+def test_mid_sized_fast_call_folds_only_the_shared_ffn(ctx, pkg):
+    """The tolerance flag at 36 tokens, 72 assignments of 24 experts, with the layer's own shared FFN: from 32 tokens
+    the shared FFN follows the flag (its own rule), the experts' products under eight assignments per expert do not.
+    Bound: the folded operands' fp16 rounding (2^-11 each) flips a few percent of the shared down input's integers
+    by one quantum of their block, 1/127 of its largest value: under 1/127 = 8e-3 of the outputs' size in the mean
+    square and less than 0.25 of it anywhere (the limits of test_gpu_fast_math.py are 2e-2 and 0.25)."""
+    cfg, T = CASES["q8_0_at_shared_mfma"]
+    say("mid layer: fast shared FFN")
+    L = pkg.synth.make_layer(cfg, norms="random")
+    ctx.upload(0, L)
+    x = pkg.synth.make_input(cfg, T=T)
+    want = ctx.ffn(0, x, keep_intermediates=True)
+    inter = ctx.intermediates()
+    got = ctx.ffn(0, x, fast_math=True)
+    for a, b in zip(ctx.intermediates(), inter):
+        np.testing.assert_array_equal(a, b)
+    assert not np.array_equal(got, want)
+    err, rms = (got - want).astype(np.float64), np.sqrt(np.mean(want.astype(np.float64) ** 2))
+    assert np.sqrt(np.mean(err ** 2)) <= rms / 127 and np.abs(err).max() <= 0.25 * rms
+
+
 def test_shared_branch_stream_order(pkg):
     say("shared FFN beside the experts: queued calls and a captured stack")
     cfg = dict(idx=97, T=40, d=512, E=16, k=2, nf=256, gu=2, dn=2, nff=512, sh=2)
