@@ -2069,6 +2069,23 @@ void phx_weight_free(phx_moe_ctx* c, phx_weight* w)
     delete w;
 }
 
+// The VALU products read the caller's rows (qb bytes of integers, db of scales) while they write y: where y shares
+// bytes with them, they read a copy instead, enqueued first.
+static int rows_apart(phx_moe_ctx* c, const int8_t*& xq, int64_t qb, const void*& xd, int64_t db, const float* y, int64_t yb)
+{
+    auto meets = [&](const void* p, int64_t n) {
+        return (uintptr_t)p < (uintptr_t)y + yb && (uintptr_t)y < (uintptr_t)p + n;
+    };
+    if (!meets(xq, qb) && !meets(xd, db)) return PHX_OK;
+    if (int rc = ensure(c, W_MM_H, (size_t)(qb + db))) return rc;  // qb: a multiple of 32
+    uint8_t* h = wp<uint8_t>(c, W_MM_H);
+    HIPCHK(c, hipMemcpyAsync(h, xq, qb, hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(h + qb, xd, db, hipMemcpyDeviceToDevice, c->stream));
+    xq = (const int8_t*)h;
+    xd = h + qb;
+    return PHX_OK;
+}
+
 int phx_matmul(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, const uint16_t* xd, float* y)
 {
     if (!c) return PHX_ERR_ARG;
@@ -2093,6 +2110,10 @@ int phx_matmul(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, con
     if (mma) {
         ENS(W_MM_D, (size_t)T * nb * 4);
         ENS(W_MM_H, (size_t)T * w->cols * 2);
+    } else {
+        const void* d = xd;
+        if ((rc = rows_apart(c, xq, (int64_t)T * w->cols, d, (int64_t)T * nb * 2, y, (int64_t)T * w->rows * 4))) return rc;
+        xd = (const uint16_t*)d;
     }
 #undef ENS
     hipStream_t st = c->stream;
@@ -2138,6 +2159,10 @@ int phx_matmul_k(phx_moe_ctx* c, const phx_weight* w, int T, const int8_t* xq, c
     int rc;
     if (!kmma) {
         // the VALU rows read the caller's planar rows and take them in order: one launch, no workspace
+        const void* d = xd;
+        if ((rc = rows_apart(c, xq, (int64_t)T * cols, d, (int64_t)T * (cols / 256) * 4, y, (int64_t)T * w->rows * 4)))
+            return rc;
+        xd = (const float*)d;
         Act a;
         a.fmt = ACT_Q8K;
         a.cols = cols;

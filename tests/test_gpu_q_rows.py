@@ -92,3 +92,41 @@ def test_ring_chunks_match_oracle(ctx, pkg, orc, wtype):
     L = pkg.synth.make_layer(cfg, norms="random")
     ctx.upload(0, L)
     check_layer(ctx, orc, L, pkg.synth.make_input(cfg, T=29), tag=f"q rows ring chunks {wtype}", exact=True)
+
+
+@pytest.mark.parametrize("wtype,T,rows,cols", [(2, 3, 130, 256), (8, 40, 130, 512), (2, 300, 4224, 256),
+                                               (12, 5, 300, 512), (13, 20, 130, 512), (14, 20, 130, 512)])
+@pytest.mark.parametrize("over", ["integers", "scales"])
+def test_output_over_the_input_rows(ctx, pkg, orc, wtype, T, rows, cols, over):
+    """y written over the integers or the scales of the call's own input rows: the result is that of rows apart."""
+    say(f"q rows: type={wtype} T={T} y over the {over}")
+    rng = np.random.default_rng(T + wtype)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    if wtype in (2, 8):
+        w = pkg.synth.quantize(wtype, rng.standard_normal((rows, cols)).astype(np.float32))
+        qs, d = ctx.Q80(0, x)
+        mm = ctx.matmul_device
+    else:
+        w = gguf_k_rows(rng, wtype, rows, cols)
+        qs, d, _ = ctx.Q8K(0, x)
+        mm = ctx.matmul_k_device
+    h = ctx.weight_upload(wtype, w, rows, cols)
+    ny = T * rows * 4
+    pool, other = ctx.alloc(max(ny, qs.nbytes) + 64), ctx.alloc(max(qs.nbytes, d.nbytes))
+    try:
+        inside = qs if over == "integers" else d
+        at = max(0, ny - inside.nbytes) // 2 // 16 * 16  # in the middle of y
+        buf = np.zeros(pool.nbytes, np.uint8)
+        buf[at:at + inside.nbytes] = inside.reshape(-1).view(np.uint8)
+        for _ in range(3):
+            pool.upload(buf)
+            other.upload(d if over == "integers" else qs)
+            q, s = (pool.ptr + at, other.ptr) if over == "integers" else (other.ptr, pool.ptr + at)
+            mm(h, T, q, s, pool.ptr)
+            ctx.sync()
+            y = pool.download((T, rows))
+            check_rows(y, lambda t: orc.matvec(wtype, w, rows, cols, x[t]), T, rng)
+    finally:
+        pool.free()
+        other.free()
+        ctx.weight_free(h)
