@@ -1715,12 +1715,13 @@ void launch_grouped(hipStream_t st, const QMat& w, Act act, const Tile* tiles, c
         g.snf = form->nf;
         g.gelu_tab = gelu_tab;
     }
-    // Q4_0 / Q8_0: the whole-row kernel while a launch has few workgroups (a layer of 32 experts, d = 1024, T = 24:
-    // 60 us against 168 for the walks below; of 128 experts, d = 2816, about 3000 workgroups: 133 either way,
+    // Q4_0 / Q8_0: the whole-row kernel while a launch has few workgroups (a layer of 32 experts, d = 1024, T = 23:
+    // 60 us against 174 for the walks below; of 128 experts, d = 2816, about 3000 workgroups: 133 either way,
     // and from 4000 the walks' several workgroups per compute unit are faster, 136 against 160)
     const bool wide = w.has_sc8() && (d16 || (int64_t)max_tiles * w.rg <= 2048);
-    // the down input in the ring kernel's epilogue where it covers every block of the row (paired Q4_0 /
-    // Q8_0 rows past QG_SHORT blocks into Q8_0 rows with no padding blocks); else k_requant after it
+    // the down input in the whole-row or the ring kernel's epilogue where it covers every block of the row (paired
+    // Q4_0 / Q8_0 rows, for the walks past QG_SHORT blocks, into Q8_0 rows with no padding blocks); else k_requant
+    // after it
     const bool fuse = req && w.paired && (wide || w.nb > QG_SHORT) && (w.type == PHX_Q4_0_DEV || w.type == PHX_Q8_0_DEV) &&
                       req->fmt == ACT_Q8_0 && req->cols == 32 * w.rg && split == 32 * w.rg && !req->qh;
     if (fuse) {
@@ -2250,20 +2251,6 @@ void launch_copy_done(hipStream_t st, void* d0, const void* s0, void* d1, const 
 {
     launch(k_copy_done, dim3(1), dim3(1024), 0, st, (uint4*)d0, (const uint4*)s0, (uint4*)d1, (const uint4*)s1,
            bytes / 16, ctr, done);
-}
-
-// Fill n 32-bit words with v: clears workspace that must start at zero with a kernel rather than a
-// memset node, so the enqueued work stays a plain kernel when a caller captures it into a graph.
-__global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ p, int64_t n, uint32_t v)
-{
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
-}
-
-void launch_fill_u32(hipStream_t st, uint32_t* p, int64_t n, uint32_t v)
-{
-    const int64_t blocks = std::min<int64_t>((n + 255) / 256, 1024);
-    launch(k_fill_u32, dim3((unsigned)std::max<int64_t>(blocks, 1)), dim3(256), 0, st, p, n, v);
 }
 
 // ------------------------------------------------------------------------------ arithmetic self-test

@@ -2380,14 +2380,14 @@ bool router_mm_supported(int T, int d, int E)
            (int64_t)E * d * 4 < ((int64_t)1 << 31);
 }
 
-void launch_router_mm(hipStream_t st, int T, int d, int E, float eps, const float* x, const float* Ws, const float* Wn,
-                      float* xscale, double* Lb, double* Bb, uint32_t* kb, int* cbad, int* flags)
+void launch_router_mm(hipStream_t st, int T, int d, int E, int ncu, float eps, const float* x, const float* Ws,
+                      const float* Wn, float* xscale, double* Lb, double* Bb, uint32_t* kb, int* cbad, int* flags)
 {
     const RmArgs a{T, d, E, eps, x, Ws, Wn, xscale, Lb, Bb, (uint4*)kb, cbad, flags};
     // 16 x 16 tiles while they run in two rounds over the compute units (a workgroup each), 32 x 32 above: one
     // round of those takes what two rounds of the small ones do (128 experts, d = 2816: T = 1500, 188 large tiles
     // or three rounds of small ones)
-    if ((int64_t)((T + 15) / 16) * ((E + 15) / 16) > 512) {
+    if ((int64_t)((T + 15) / 16) * ((E + 15) / 16) > 2 * ncu) {
         using RG = RmLds<2, 2>;
         raise_lds(KRm<2, 2>::fn, RG::BYTES);
         launch(KRm<2, 2>::fn, dim3((T + 31) / 32, (E + 31) / 32), dim3(RM_NW * 64), (uint32_t)RG::BYTES, st, a);

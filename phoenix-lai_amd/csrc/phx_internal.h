@@ -255,8 +255,8 @@ __host__ __device__ inline void router_range(int d, int r, int* c0, int* cnt)
     *cnt = base + (r < extra);
 }
 bool router_mm_supported(int T, int d, int E);
-void launch_router_mm(hipStream_t st, int T, int d, int E, float eps, const float* x, const float* Ws, const float* Wn,
-                      float* xscale, double* Lb, double* Bb, uint32_t* kb, int* cbad, int* flags);
+void launch_router_mm(hipStream_t st, int T, int d, int E, int ncu, float eps, const float* x, const float* Ws,
+                      const float* Wn, float* xscale, double* Lb, double* Bb, uint32_t* kb, int* cbad, int* flags);
 // a stack layer's router with the previous layer's combine folded in (prev: that layer, its xin the
 // rows it reads, its xres where the new x goes; h.x must be prev.xres)
 void launch_dec_route_fused(hipStream_t st, const DecLayerH& prev, const DecLayerH& h);
@@ -265,7 +265,6 @@ void launch_dec_down(hipStream_t st, const DecLayerH& h);
 void launch_dec_combine(hipStream_t st, const DecLayerH& h);
 void launch_stream_read(hipStream_t st, const void* src, int64_t bytes, uint32_t* sink);
 void launch_stream_copy(hipStream_t st, void* dst, const void* src, int64_t bytes);
-void launch_fill_u32(hipStream_t st, uint32_t* p, int64_t n, uint32_t v);
 // a small copy (bytes a multiple of 16, either side may be pinned host memory) as one kernel
 void launch_copy_small(hipStream_t st, void* dst, const void* src, int64_t bytes);
 // the last copies of a host-buffer call (d1 / s1 may be null), then *done = ++*ctr (ctr device memory,

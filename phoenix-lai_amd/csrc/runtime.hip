@@ -859,8 +859,11 @@ bool cert_route(const Layer& L, int T, bool shared_ffn)
 }
 
 // prefill-sized expert work (several assignments per expert on average) runs on the matrix cores, whose
-// kernels read the activations' fp16 copies: from three per expert (128 experts of d = 2816, Q4_0: T = 32 145 us
-// on the VALU rows against 177, T = 48 192 against 188, T = 77 238 against 205, T = 127 317 against 207)
+// kernels read the activations' fp16 copies: from three per expert.  The VALU rows and the matrix cores (us): 8 of 128
+// experts, d = 2816, Q4_0, T = 32 (two per expert) 145 and 177, T = 48 (three) 206 and 177, T = 64 229 and 184; with a
+// shared FFN T = 48 217 and 191; Q8_0 T = 48 249 and 217; 8 of 256 experts, d = 2048, T = 96 (three) 186 and 184, T =
+// 128 201 and 185; 4 of 32, d = 1024, Q8_0, with a shared FFN, T = 24 62 and 65, T = 63 72 and 65; 2 of 8, d = 4096,
+// n_ff = 2048, T = 17 88 and 74, T = 31 128 and 75
 static bool mma_path(const phx_moe_layer_desc& D, int T)
 {
     return mfma_type(D.gate_up_type) && mfma_type(D.down_type) && T * D.n_used >= 3 * D.n_expert;
@@ -1044,7 +1047,7 @@ int run_layer_general(phx_moe_ctx* c, const Layer& L, int T, const float* x, con
             if (!late) HIPCHK(c, hipEventRecord(c->ev_fork, st));
             {
                 ProfScope p(c, PHX_K_ROUTER);
-                launch_router_mm(st, T, d, E, D.eps, x, L.wsc, L.wnr, wp<float>(c, W_RSCALE), h.Lb, h.Bb, h.kb, h.bad,
+                launch_router_mm(st, T, d, E, c->ncu, D.eps, x, L.wsc, L.wnr, wp<float>(c, W_RSCALE), h.Lb, h.Bb, h.kb, h.bad,
                                  c->flags);
             }
             if (late) HIPCHK(c, hipEventRecord(c->ev_fork, st));
