@@ -1515,11 +1515,11 @@ __global__ __launch_bounds__(256) void k_grouped_k_walk(GroupArgs g)
 // then bound it (about 700 VALU instructions per super-block and wave; 16 waves each 10-20% slower from 32
 // tokens on).
 // The grid has two dimensions (tiles times row groups times threads may pass the 2^32 threads a dimension can
-// hold).  Lists of several tokens have slots past their last tile, whose workgroups end at once: with the tiles in
-// x, these recur at the same places of every row group's run and leave some of the engines that the dispatcher
-// serves in turn with less work than others, so the row groups are in x and the empty slots at the grid's end (64
-// experts of 4096 columns, T = 8: the layer 204 -> 122 us; 128 of 2816: 107 -> 88).  Rows in order have no empty
-// slots, and neighbours in x share a row group's weights.
+// hold).  Lists of several tokens have slots past their last tile, whose workgroups end at once.  With the tiles in x
+// these recur in every row group's run, and where the run's length divides the number of engines that the dispatcher
+// serves in turn, at the same engines (a gate and up launch of 42 tiles in 64 slots took 114 us, in 68 slots 87): so
+// the row groups are in x and the empty slots at the grid's end (64 experts of 4096 columns, T = 8: the layer 204 ->
+// 122 us; 128 of 2816: 107 -> 88).  Rows in order have no empty slots, and neighbours in x share a row group's weights.
 // Past 24 assignments times row groups per compute unit (nassign: the launch's assignments) the waves walk whole
 // rows instead: Q5_K rows in order, 4224 x 4096 T = 80 (21 per unit) 80 us for k_grouped_k and 87 for the walk, T =
 // 96 100 and 87, T = 1024 782 and 555; 2816 x 2304 T = 1024 318 and 211; layers of 128 experts, d = 2816, Q4_K /
