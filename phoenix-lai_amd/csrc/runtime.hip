@@ -2082,8 +2082,8 @@ static int rows_apart(phx_moe_ctx* c, const int8_t*& xq, int64_t qb, const void*
     if (!meets(xq, qb) && !meets(xd, db)) return PHX_OK;
     if (int rc = ensure(c, W_MM_H, (size_t)(qb + db))) return rc;  // qb: a multiple of 32
     uint8_t* h = wp<uint8_t>(c, W_MM_H);
-    HIPCHK(c, hipMemcpyAsync(h, xq, qb, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(h + qb, xd, db, hipMemcpyDeviceToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(h, xq, qb, hipMemcpyDefault, c->stream));
+    HIPCHK(c, hipMemcpyAsync(h + qb, xd, db, hipMemcpyDefault, c->stream));
     xq = (const int8_t*)h;
     xd = h + qb;
     return PHX_OK;
